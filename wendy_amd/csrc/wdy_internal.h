@@ -290,6 +290,8 @@ u32 small_max_n(int device);
 // at 2^11.
 constexpr u64 SMALL_MAX_EQUAL = 6144;
 constexpr u64 SMALL_MAX_UNEQUAL = 1536;
+// Sheets one wave holds in registers for a whole interval: 8 per lane.
+constexpr u64 SMALL_WAVE_MAX = 512;
 int launch_small_advance(wdy_sim *s, double h, int nleap, double *acc_out,
                          double *cum_out);
 int launch_energy(wdy_sim *s, double twopiG, double omega2, double *e_out);
