@@ -38,11 +38,13 @@ extern "C" {
 
 /* wdy_create flags */
 #define WDY_EQUAL_MASS 1  /* every m[i] is the same value: force from rank */
-/* Path selection.  By default n up to the per-workgroup LDS capacity
- * (12 B per sheet) runs as one persistent workgroup per output interval
- * ("small" path), larger n as a multi-kernel step over the whole GPU
- * ("large" path).  These flags force one path, e.g. so that tests reach the
- * large path's code at small n. */
+/* Path selection.  By default up to 512 sheets run as one wave per output
+ * interval, up to 2^22 as windows of sheets that take several leapfrog steps
+ * per launch, where those are faster than a launch per step over the whole
+ * GPU ("large" path), which takes the rest.  WDY_FORCE_LARGE keeps a
+ * simulation on the large path, WDY_FORCE_SMALL (n up to the LDS capacity, 12 B
+ * per sheet) on one persistent workgroup per interval, e.g. so that tests reach
+ * that code at any n. */
 #define WDY_FORCE_LARGE 2
 #define WDY_FORCE_SMALL 4
 /* The large path re-sorts each leapfrog step with one warm-start kernel
@@ -223,14 +225,15 @@ int wdy_set_ext_force_host(wdy_sim *sim,
 /* The simulation clock t0 (advanced only while an external force is set). */
 int wdy_time(wdy_sim *sim, double *t_out);
 
-/* Leapfrog steps taken so far by the warm-start kernel and by the radix
- * path, and the number of output intervals redone on the radix path after a
- * warm-start failure.  No reference counterpart. */
+/* Leapfrog steps taken so far by the warm-start kernel or the windows (those
+ * only above the one-workgroup sizes) and by the radix path, and the number of
+ * output intervals redone after a failure of either.  No reference
+ * counterpart. */
 int wdy_path_stats(wdy_sim *sim, int64_t *warm_steps, int64_t *cold_steps,
                    int64_t *redos);
 
-/* Warm intervals redone so far, by cause: a bucket outgrew its capacity,
- * far movers overflowed their list, or a bounded wait of the look-back gave
+/* Intervals redone so far, by cause: a bucket outgrew its capacity, far
+ * movers overflowed their list or a window's halo, or a bounded wait of the look-back gave
  * up (the last disables the warm path for the sim).  No reference
  * counterpart. */
 int wdy_warm_failures(wdy_sim *sim, int64_t *capacity, int64_t *overflow,

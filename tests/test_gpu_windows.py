@@ -1,9 +1,11 @@
-"""The one-wave kernel (n <= 512) against the oracle, at the sizes where a
-lane's block ends.
+"""Several leapfrog steps per launch: the one-wave kernel (n <= 512) and the
+windows of sorted sheets with halos (the default path above), against the
+oracle, at the sizes where a tile, a lane's block or a window ends.
 
 Equal masses are a power of two here, so that rank * m is the reference's
 running sum exactly: those cases are bitwise, and so is the one-wave kernel's
-sequential prefix of any masses.
+sequential prefix of any masses.  The windows' unequal masses use the exact
+fixed-point prefix: 1e-10, the bar of the approximate path.
 """
 import numpy
 import pytest
@@ -56,3 +58,82 @@ def test_one_wave(gpu_lib, n, mass):
     x, v, m = disk(n, mass)
     for dt, nleap in ((0.05, 20), (2., 7)):
         check(x, v, m, dt, nleap, 2, omega=0.3)
+
+
+@pytest.mark.parametrize('mass', ['equal', 'lognormal'])
+@pytest.mark.parametrize('n', [513, 1024, 1025, 2047, 4096, 4097, 6144, 6145,
+                               16385, 50001])
+def test_windows(gpu_lib, n, mass):
+    """Step sizes from less than a rank to hundreds of ranks per step, one to
+    many steps per launch, an uneven number of steps."""
+    x, v, m = disk(n, mass)
+    for dt, nleap in ((0.0005, 1), (0.0023, 23), (0.02, 13)):
+        st, _ = check(x, v, m, dt, nleap, 2, omega=0.1, exact=mass == 'equal')
+        if n > 6144 and nleap > 1:
+            assert st == (2 * nleap, 0, 0)  # no radix interval, nothing redone
+
+
+@pytest.mark.parametrize('force', [forces.Harmonic(0.3), forces.Pulse(0.4, 0.01, 0.02)])
+@pytest.mark.parametrize('n', [200, 3000, 20000])
+def test_external_force(gpu_lib, n, force):
+    x, v, m = disk(n, 'equal')
+    # the device's exp differs from the host's in the last place
+    check(x, v, m, 0.02, 10, 2, force=force, exact=isinstance(force, forces.Harmonic))
+
+
+@pytest.mark.parametrize('n', [500, 3000, 20000])
+def test_tied_groups(gpu_lib, n):
+    """Groups of 40 sheets that start and stay at one position."""
+    x, v, m = disk(n, 'equal')
+    x = x[(numpy.arange(n) // 40) * 40]
+    v = numpy.zeros(n)
+    m = numpy.zeros(n)
+    m[0] = 1.
+    check(x, v, m, 0.1, 8, 2)
+
+
+def test_halo_too_narrow_is_redone(gpu_lib):
+    """The inner sheets move together during the first interval, to half the
+    distances the halos were sized for: the windows there report it and the
+    interval is redone with wider ones."""
+    n = 20000
+    x, v, m = disk(n, 'equal')
+    v = numpy.where(numpy.abs(x) < 0.05, -10. * x, 0.)
+    st, fail = check(x, v, m, 0.05, 10, 3)
+    assert st[0] > 0 and st[2] >= 1 and fail[1] >= 1
+
+
+@pytest.mark.parametrize('kind', ['outliers', 'tails', 'clump'])
+@pytest.mark.parametrize('n', [600, 1000, 4000, 6144, 20000])
+def test_uneven_density(gpu_lib, n, kind):
+    """Bins of one width would hold most of the sheets here: the windows cut
+    theirs by rank."""
+    x, v, m = disk(n, 'equal')
+    if kind == 'outliers':
+        x[0], x[1] = 300., -1e4
+    elif kind == 'tails':
+        x = numpy.clip(numpy.random.default_rng(n).standard_cauchy(n), -1e5, 1e5)
+    else:
+        x[:n // 3] *= 1e-5
+    for dt, nleap in ((0.006, 20), (0.2, 20)):
+        check(x, v, m, dt, nleap, 2, omega=0.1)
+
+
+@pytest.mark.parametrize('n', [200, 3000, 20000])
+def test_overflow_as_on_the_other_paths(gpu_lib, n):
+    """A sheet that overflows to infinity, then NaN: the others' ranks are as
+    the keys' order has them."""
+    x, v, m = disk(n, 'equal')
+    x[7] = 1.7e308
+    out = []
+    for kw in ({}, {'path': 'large', 'warm': False}):
+        sim = wendy_amd.Sim(x, v, m, numpy.sum(m), 900., **kw)
+        gx, gv = numpy.empty(n), numpy.empty(n)
+        for _ in range(3):
+            sim.advance(0.001, 4)
+        sim.read(gx, gv)
+        sim.close()
+        out.append((gx, gv))
+    assert numpy.isnan(out[0][0]).any()
+    for a, b in zip(*out):
+        assert numpy.array_equal(a, b, equal_nan=True)

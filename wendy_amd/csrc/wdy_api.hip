@@ -125,6 +125,7 @@ static void free_sim(wdy_sim *s) {
   for (int b = 0; b < 2; ++b)
     if (s->perm[b]) (void)hipFree(s->perm[b]);
   warm_free(s);
+  span_free(s);
   if (s->skey) (void)hipFree(s->skey);
   if (s->cum) (void)hipFree(s->cum);
   if (s->tile_sums) (void)hipFree(s->tile_sums);
@@ -215,8 +216,15 @@ static int create_impl(int64_t n, const double *x_slot, const i32 *id_slot,
                   (long long)n, smax);
     const u64 lim = eq ? SMALL_MAX_EQUAL : SMALL_MAX_UNEQUAL;
     const u64 slim = smax < lim ? smax : lim;
-    s->small = (flags & WDY_FORCE_SMALL) ||
-               (!(flags & WDY_FORCE_LARGE) && (u64)n <= slim);
+    bool nonneg = true;  // the fixed-point mass prefixes need it
+    for (int64_t i = 0; nonneg && i < n; ++i) nonneg = m_id[i] >= 0.0;
+    // several steps per launch, for a simulation whose path is not asked for
+    const bool span = nonneg && (u64)n > SMALL_WAVE_MAX && (u64)n <= SPAN_MAX &&
+                      !(flags & (WDY_FORCE_SMALL | WDY_FORCE_LARGE | WDY_NO_WARM |
+                                 WDY_SHARED_GPU));
+    s->small_class = (flags & WDY_FORCE_SMALL) ||
+                     (!(flags & WDY_FORCE_LARGE) && (u64)n <= slim);
+    s->small = s->small_class && !span;
     WDY_HIP(hipStreamCreate(&s->stream));
     WDY_HIP(hipStreamCreate(&s->copy_stream));
     WDY_HIP(hipEventCreate(&s->ev0));
@@ -272,15 +280,18 @@ static int create_impl(int64_t n, const double *x_slot, const i32 *id_slot,
     r = launch_build_state(s, s->out_x, s->idx[1], s->out_v, s->cum);
     if (r) return r;
     // warm-start step for the large path, unless disabled; it needs
-    // non-negative masses (fixed-point prefix)
-    bool warm = !s->small && !(flags & WDY_NO_WARM);
-    for (int64_t i = 0; warm && i < n; ++i) warm = m_id[i] >= 0.0;
-    if (warm) {
-      const int shape0 = (flags & WDY_SHARED_GPU) ? WARM_SHAPE_DEFAULT
-                                                  : warm_initial_shape(n, eq);
-      r = warm_configure(s, shape0, 0u, (u32)WARM_WINDOW_DEFAULT);
-      if (r) return r;
-      s->disp_rate = displacement_rate(n, x_slot, v_id, id_slot);
+    // non-negative masses (fixed-point prefix).  With windows it is set up
+    // when it is first needed.
+    s->warm_ok = !s->small_class && !(flags & WDY_NO_WARM) && nonneg;
+    s->warm_shape0 = (flags & WDY_SHARED_GPU) ? WARM_SHAPE_DEFAULT
+                                              : warm_initial_shape(n, eq);
+    if (s->warm_ok) s->disp_rate = displacement_rate(n, x_slot, v_id, id_slot);
+    if (span) {
+      double vmax = 0.0;
+      for (int64_t i = 0; i < n; ++i) vmax = std::max(vmax, std::fabs(v_id[i]));
+      if ((r = span_create(s, vmax))) return r;
+    } else if ((r = warm_ensure(s))) {
+      return r;
     }
     WDY_HIP(hipMemcpyAsync(s->h_rerr, radix_err_word(&s->radix), 4,
                            hipMemcpyDeviceToHost, s->stream));
@@ -288,6 +299,7 @@ static int create_impl(int64_t n, const double *x_slot, const i32 *id_slot,
     if (*s->h_rerr)
       return fail(WDY_ERUNTIME, "wdy_create: a look-back wait of the initial "
                   "sort gave up");
+    if (s->span) span_created(s);
     return WDY_OK;
   }();
   if (rc) {
@@ -326,6 +338,7 @@ static int advance_host_force(wdy_sim *s, double h, int nleap,
   f.tab = s->ext_tab;
   const ExtForce saved = s->ext;
   s->ext = f;
+  s->span_sorted = false;
   int rc = [&]() -> int {
     if (int r = launch_drift(s, h / 2.)) return r;
     double t = s->t0;
@@ -381,9 +394,11 @@ static int cold_interval(wdy_sim *s, double h, int nleap, double *acc_last,
                          double *cum_last) {
   // size the warm-start layout for this h before the splitters of the
   // next partition are written (a resize reallocates their buffers)
+  if (int rc = warm_ensure(s)) return rc;
   if (s->warm) {
     if (int rc = warm_fit(s, h)) return rc;
   }
+  s->span_sorted = false;
   int rc = launch_drift(s, h / 2.);
   if (rc) return rc;
   u32 T = 0, nb = 0;
@@ -437,6 +452,26 @@ static int settle(wdy_sim *s) {
       if (int rc = radix_check_enqueue(s)) return rc;
     }
   }
+  if (s->span) {
+    bool failed = false;
+    double h = 0.0;
+    int nleap = 0;
+    if (int rc = span_settle(s, &failed, &h, &nleap)) return rc;
+    while (failed) {  // again with wider halos, or on the other paths
+      s->redos += 1;
+      SpanPlan p;
+      if (span_plan(s, h, nleap, &p)) {
+        if (int rc = span_interval(s, h, nleap, p)) return rc;
+        WDY_HIP(hipEventRecord(s->ev1, s->stream));
+        if (int rc = span_settle(s, &failed, &h, &nleap)) return rc;
+      } else {
+        failed = false;
+        if (int rc = cold_interval(s, h, nleap, nullptr, nullptr)) return rc;
+        WDY_HIP(hipEventRecord(s->ev1, s->stream));
+        if (int rc = radix_check_enqueue(s)) return rc;
+      }
+    }
+  }
   if (s->rerr_pending) {
     WDY_HIP(hipEventSynchronize(s->ev_rerr));
     s->rerr_pending = false;
@@ -455,6 +490,7 @@ static int advance_impl(wdy_sim *s, double h, int nleap, double *acc_last,
   if (int rc = settle(s)) return rc;
   warm_gang_release(s);  // ev0/ev1 bracket this interval
   WDY_HIP(hipEventRecord(s->ev0, s->stream));
+  SpanPlan plan;
   if (s->host_force) {
     if (int rc = advance_host_force(s, h, nleap, acc_last, cum_last)) return rc;
     if (int rc = radix_check_enqueue(s)) return rc;
@@ -463,10 +499,16 @@ static int advance_impl(wdy_sim *s, double h, int nleap, double *acc_last,
     if (rc) return rc;
     if (s->ext.kind)  // the kernel's clock, replayed (wendy/wendy.c:401-408)
       for (int ii = 0; ii < nleap; ++ii) s->t0 = s->t0 + h;
+  } else if (!acc_last && !cum_last && span_plan(s, h, nleap, &plan)) {
+    const bool resorts = !s->span_sorted;
+    if (int rc = span_interval(s, h, nleap, plan)) return rc;
+    if (resorts)
+      if (int rc = radix_check_enqueue(s)) return rc;
   } else if (!acc_last && !cum_last && warm_ready_for(s, h)) {
     // warm interval when the state is partitioned for this h and nothing
     // asks for the last force: enqueued and checked by the next settle,
     // which redoes it on the radix path after a device-side failure
+    s->span_sorted = false;
     if (int rc = warm_interval(s, h, nleap)) return rc;
   } else {
     if (int rc = cold_interval(s, h, nleap, acc_last, cum_last)) return rc;
@@ -724,7 +766,8 @@ int wdy_gang_advance(wdy_gang *gang, wdy_sim *const *sims, int count,
 
 int wdy_tune(wdy_sim *sim, int shape, int bucket_target, int window) {
   if (int rc = check_settled(sim, "wdy_tune")) return rc;
-  if (sim->small || !sim->warm)
+  if (int rc = warm_ensure(sim)) return rc;
+  if (sim->small_class || !sim->warm)
     return fail(WDY_EUNSUPPORTED, "wdy_tune: the sim has no warm-start path");
   if (shape < -1 || shape >= WARM_NSHAPES)
     return fail(WDY_EINVAL, "wdy_tune: shape %d out of range", shape);
@@ -737,6 +780,7 @@ int wdy_tune(wdy_sim *sim, int shape, int bucket_target, int window) {
   WDY_HIP(hipSetDevice(sim->device));
   WDY_HIP(hipStreamSynchronize(sim->stream));
   warm_mark_tuned(sim);
+  span_off(sim);  // the tuned kernel runs from now on
   return warm_configure(sim, shape, (u32)bucket_target, (u32)window);
 }
 
@@ -774,7 +818,7 @@ int wdy_set_ext_force_host(wdy_sim *sim,
   if (int rc = check_settled(sim, "wdy_set_ext_force_host")) return rc;
   if (!std::isfinite(t0))
     return fail(WDY_EINVAL, "wdy_set_ext_force_host: t0 not finite");
-  if (force && sim->small)
+  if (force && sim->small_class)
     return fail(WDY_EUNSUPPORTED,
                 "wdy_set_ext_force_host: the simulation runs on the small path; "
                 "create it with WDY_FORCE_LARGE");
@@ -813,6 +857,7 @@ int wdy_warm_failures(wdy_sim *sim, int64_t *capacity, int64_t *overflow,
 
 int wdy_warm_config(wdy_sim *sim, int *shape, int *bucket_target, int *window) {
   if (int rc = check_settled(sim, "wdy_warm_config")) return rc;
+  if (int rc = warm_ensure(sim)) return rc;
   int sh = -1;
   u32 T = 0, W = 0;
   if (!warm_config(sim, &sh, &T, &W)) sh = -1;

@@ -179,6 +179,7 @@ int radix_sort_pairs(RadixWork *w, hipStream_t s, Timer *tm, u64 *k0, u64 *k1,
 // Simulation state
 // --------------------------------------------------------------------------
 struct WarmCtx;  // warm-start step metadata (wdy_warm.hip)
+struct SpanCtx;  // multi-step windows (wdy_span.hip)
 }  // namespace wdy
 
 struct wdy_sim {
@@ -213,7 +214,16 @@ struct wdy_sim {
   double *out_x = nullptr;       // de-sorted output staging
   double *out_v = nullptr;
   wdy::RadixWork radix;
-  wdy::WarmCtx *warm = nullptr;  // null: the large path uses radix steps only
+  wdy::WarmCtx *warm = nullptr;  // null: no warm path, or not set up yet
+  bool warm_ok = false;          // the warm path may be set up
+  int warm_shape0 = 0;           // the tile shape it starts from
+  // several steps per launch over windows of sheets (null: not for this
+  // sim); span_sorted: the current set is in sorted order for it
+  wdy::SpanCtx *span = nullptr;
+  bool span_sorted = false;
+  // of a size that takes the one-workgroup path when windows do not apply:
+  // its limits at the API (no tuning, no host-function force) are kept
+  bool small_class = false;
 
   // external force and its clock: t0 advances by h after every force
   // evaluation while an external force is set (wendy/wendy.c:401-402,407-408)
@@ -281,17 +291,24 @@ int energy_enqueue(hipStream_t st, u32 n, const double *x, const double *v,
                    u32 *epoch, const u32 **err_word);
 // small mode (wdy_small.hip)
 u32 small_max_n(int device);
-// Largest n the one-workgroup path takes by default (further capped by its
-// LDS capacity).  It runs a whole interval in one workgroup, so its time
-// grows with n while the large path's stays near its floor of ~0.33 ms per
-// 20-step interval up to ~2^16 sheets: measured, equal masses 0.21 vs 0.32
-// ms at 2^12 and 0.43 vs 0.32 at 2^13; unequal masses (whose mass prefix
-// the small path runs sequentially) 0.23 vs 0.40 at 2^10 and 0.43 vs 0.33
-// at 2^11.
+// Largest n that counts as a small simulation (further capped by the LDS): it
+// has no warm-start layout and takes no host-function force, and its windows
+// can always be a single one.  Negative masses, which the windows do not take,
+// run it in one workgroup: its time grows with n while the large path's stays
+// near its floor of ~0.33 ms per 20-step interval up to ~2^16 sheets: measured,
+// equal masses 0.21 vs 0.32 ms at 2^12 and 0.43 vs 0.32 at 2^13; unequal masses
+// (whose mass prefix one thread sums) 0.23 vs 0.40 at 2^10 and 0.43 vs 0.33 at
+// 2^11.
 constexpr u64 SMALL_MAX_EQUAL = 6144;
 constexpr u64 SMALL_MAX_UNEQUAL = 1536;
-// Sheets one wave holds in registers for a whole interval: 8 per lane.
+// Sheets one wave holds in registers for a whole interval: 8 per lane.  At 512
+// sheets a 20-step interval takes 20 us with equal masses and 104 with unequal
+// ones (whose prefix stays a sequential sum), at 1000 sheets the windows' single
+// workgroup 21 and 25.
 constexpr u64 SMALL_WAVE_MAX = 512;
+// Largest n the multi-step windows are set up for (beyond, a window of 4096
+// sheets is mostly halo at the step sizes in use).
+constexpr u64 SPAN_MAX = 1u << 22;
 int launch_small_advance(wdy_sim *s, double h, int nleap, double *acc_out,
                          double *cum_out);
 int launch_energy(wdy_sim *s, double twopiG, double omega2, double *e_out);
@@ -318,6 +335,24 @@ int warm_current_shape(wdy_sim *s);
 bool warm_config(wdy_sim *s, int *shape, u32 *T, u32 *W);
 // wait (without checking) for the warm interval in flight, if any
 void warm_wait(wdy_sim *s);
+// sets up the warm path if the sim may have one and has none yet
+int warm_ensure(wdy_sim *s);
+// multi-step windows (wdy_span.hip): a plan for an interval of nleap steps of
+// h, false when the windows do not apply or the other paths are faster
+struct SpanPlan {
+  int shape = 0;
+  u32 K = 1;  // steps per launch
+};
+bool span_plan(wdy_sim *s, double h, int nleap, SpanPlan *plan);
+// enqueues the set-up on the current (sorted) set; vmax: the largest |v|.
+// span_created: once that work has finished
+int span_create(wdy_sim *s, double vmax);
+void span_created(wdy_sim *s);
+void span_free(wdy_sim *s);
+void span_off(wdy_sim *s);
+int span_prefix(wdy_sim *s);
+int span_interval(wdy_sim *s, double h, int nleap, const SpanPlan &p);
+int span_settle(wdy_sim *s, bool *failed, double *h, int *nleap);
 // the events bracketing the last interval when it ran in a gang
 bool warm_gang_events(wdy_sim *s, hipEvent_t *start, hipEvent_t *done);
 // the next interval runs outside a gang: drop the settled gang record

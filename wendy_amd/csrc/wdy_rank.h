@@ -1,9 +1,16 @@
 // Sorting of nearly sorted sheets on chip, for kernels that run several
-// leapfrog steps without going back to memory: one wave holds up to 64 * PER
-// sheets in registers, PER consecutive ranks per lane, and re-sorts them after
-// each drift by odd-even transposition, ending as soon as the order is right:
-// no LDS, no barrier, ~10 instructions per sheet and rank of displacement.
-// Exact for any input (positions, then sheet index).
+// leapfrog steps without going back to memory.  Both forms are exact for any
+// input (positions, then sheet index).
+//
+// * WaveSort: one wave holds up to 64 * PER sheets in registers, PER
+//   consecutive ranks per lane, and re-sorts them after each drift by odd-even
+//   transposition, ending as soon as the order is right: no LDS, no barrier,
+//   ~10 instructions per sheet and rank of displacement.  For steps that move
+//   sheets a few ranks.
+// * BinRank: a workgroup's sheets stay in the registers of the threads that
+//   loaded them and only their ranks change: a counting pass over position
+//   bins in LDS, then each sheet ranks itself in its bin.  Its cost does not
+//   depend on the displacement.
 #pragma once
 
 #include "wdy_lds.h"
@@ -132,6 +139,296 @@ struct WaveSheets {
       for (int q = 0; q + 1 < PER; ++q) o = o || after(x[q], id[q], x[q + 1], id[q + 1]);
       if (__ballot(o) == 0) return moved;
       round<true>(xn);
+    }
+  }
+};
+
+// ---- BinRank -----------------------------------------------------------------
+template <int WT_, int PER_>
+struct RankShape {
+  static constexpr int WT = WT_, PER = PER_, CAP = WT_ * PER_, NWAVE = WT_ / 64;
+};
+
+// Bins: the window is cut into BIN_SEGS segments by rank, finer towards its
+// ends, and each segment's range of positions (when the launch starts) is cut
+// into as many bins as it has of them: outliers and tails take a few bins and
+// leave the rest theirs.  (With bins of one width over the window, 1000 sheets
+// of which two lie far out shared a few bins: 110 us a step.)  A thread keeps
+// its sheets' segments; they seldom change.  A window whose segments are about
+// as dense as each other takes bins of one width, which costs a quarter less.
+constexpr int BIN_SEGS = 16;
+struct BinSeg {
+  double lo, scale, next;  // its first position, bins per length, the next's first
+  u32 base, cnt;
+};
+// the start of segment k, out of 256
+__device__ __forceinline__ u32 bin_seg_start(u32 k) {
+  const u32 j = k <= 8 ? k : 16 - k;  // 0 1 4 16 32 56 80 104 128
+  const u32 e = j == 0 ? 0u : j <= 3 ? 1u << (2 * (j - 1)) : 24 * j - 64;
+  return k <= 8 ? e : 256 - e;
+}
+
+// LDS: positions and sheet indices in bin order, two sets of bin counters (one
+// is cleared while the other is used) and, with unequal masses, the masses in
+// bin order, then the mass below each slot.
+template <class SH, bool MASS>
+struct BinRank {
+  static constexpr int CAP = SH::CAP, PER = SH::PER, WT = SH::WT, NWAVE = SH::NWAVE;
+  static constexpr int NB = CAP, WPT = NB / WT;  // bins, bins per thread
+  static_assert(NWAVE <= 16, "one row of lanes scans the waves' totals");
+  static constexpr int PAD = 4;  // slots read past the last sheet (ms: one more)
+  static constexpr size_t BYTES = 8ull * (CAP + PAD) +
+                                  (MASS ? 8ull * (CAP + PAD + 1) : 0ull) +
+                                  16ull * 16 + 4ull * (CAP + PAD) + 4ull * CAP +
+                                  8ull * (NB + 1) + (BIN_SEGS + 1) * sizeof(BinSeg);
+  static_assert(NB % 256 == 0, "whole bins in every segment");
+  double *xs;
+  u64 *ms;  // masses in bin order, then the mass below each slot
+  u64 *red, *redm;
+  float *xf;  // place within the bin, rounded
+  i32 *id;
+  u32 *bins;  // [2][NB + 1]: one more, the end of the last bin
+  BinSeg *seg;  // [BIN_SEGS], and the window as one
+  double x0, scale;  // of the window as one segment
+  bool segs;         // else one segment
+  u32 s;
+  u32 g[PER];  // the sheets' segments
+
+  // kin: the keys of the window's w sheets, in order.  The segments go by rank
+  // as if there were eL ranks more in a length d below the first sheet and eR
+  // in d above the last (each 0 or the same): where the sheets go that leave the window.
+  __device__ BinRank(u64 *base, u32 w, const u64 *kin, u32 eL, u32 eR, double d) {
+    seg = (BinSeg *)base;
+    xs = (double *)(seg + BIN_SEGS + 1);
+    ms = (u64 *)(xs + CAP + PAD);
+    red = MASS ? ms + CAP + PAD + 1 : ms;
+    redm = red + 16;
+    xf = (float *)(redm + 16);
+    id = (i32 *)(xf + CAP + PAD);
+    bins = (u32 *)(id + CAP);
+    s = 0;
+    clear(0);
+    const u32 t = threadIdx.x;
+    if (t < BIN_SEGS) {
+      const u32 f0 = bin_seg_start(t), f1 = bin_seg_start(t + 1);
+      BinSeg q;
+      // (in signed numbers: the compiler here takes a `u < eL ? 0 : u - eL`
+      // inside a min() to mean that u >= eL)
+      const u32 e = max(eL, eR);
+      const double per = e ? d / (double)e : 0.0;
+      auto at = [&](u32 u) {
+        const i32 r = (i32)u - (i32)eL, over = r - (i32)w;
+        const double x = decode_pos(kin[max(0, min(r, (i32)w - 1))]);
+        return x + per * (double)(r < 0 ? r : max(over, 0));
+      };
+      const u32 tot = eL + w + eR;
+      q.lo = at(tot * f0 >> 8);
+      const double hi = at(tot * f1 >> 8);
+      q.next = t + 1 < BIN_SEGS ? hi : __builtin_inf();
+      q.base = (u32)NB / 256 * f0;
+      q.cnt = (u32)NB / 256 * (f1 - f0);
+      const double range = hi - q.lo;
+      q.scale = range > 1.0e-300 && range < 1.0e300 ? (double)q.cnt / range : 0.0;
+      seg[t] = q;
+      // one segment does while none of these would have six times its share
+      // of sheets per bin
+      const double first = at(0), last = at(tot), all = last - first;
+      const bool full = !((double)q.cnt * all <= 6.0 * (double)NB * range);
+      const u32 any = __ballot(full) != 0 ? 1u : 0u;
+      if (t == 0) {
+        q.lo = first;
+        q.scale = all > 1.0e-300 && all < 1.0e300 ? (double)NB / all : 0.0;
+        q.base = any;
+        seg[BIN_SEGS] = q;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const u32 e = i * WT + t;
+      g[i] = 0;
+#pragma unroll
+      for (u32 k = 1; k < BIN_SEGS; ++k)
+        g[i] += e + eL >= (eL + w + eR) * bin_seg_start(k) >> 8 ? 1u : 0u;
+    }
+    if (threadIdx.x < 16) red[threadIdx.x] = redm[threadIdx.x] = 0;
+    if (threadIdx.x < PAD) {
+      xf[w + threadIdx.x] = 2.f;
+    }
+    __syncthreads();
+    x0 = seg[BIN_SEGS].lo;
+    scale = seg[BIN_SEGS].scale;
+    segs = __builtin_amdgcn_readfirstlane(seg[BIN_SEGS].base) != 0;
+  }
+  __device__ __forceinline__ void clear(u32 b) {
+    const u32 t = threadIdx.x;
+#pragma unroll
+    for (int q = 0; q < WPT; ++q) {
+      bins[b * (NB + 1) + q * WT + t] = 0;
+    }
+  }
+  // exclusive prefix of one value per thread over the workgroup; one barrier
+  template <class T>
+  __device__ __forceinline__ T scan_excl(T v, u64 *r) {
+    const u32 lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
+    const T inc = wave_incl_add(v);
+    if (lane == 63u) r[wv] = inc;
+    return inc - v;
+  }
+  // the total of the waves before this one (after the barrier)
+  template <class T>
+  __device__ __forceinline__ T waves_before(const u64 *r) {
+    const u32 lane = threadIdx.x & 63u;
+    const u32 wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    T x = (T)r[lane & 15u];
+    x += dpp_mov<DPP_SHR1, 0xf>((T)0, x);
+    x += dpp_mov<DPP_SHR2, 0xf>((T)0, x);
+    if (NWAVE > 4) x += dpp_mov<DPP_SHR4, 0xf>((T)0, x);
+    if (NWAVE > 8) x += dpp_mov<DPP_SHR8, 0xf>((T)0, x);
+    // (lane wv - 1 holds the inclusive total of wave wv - 1)
+    const u32 src = wv ? wv - 1u : 0u;
+    T y;
+    if constexpr (sizeof(T) == 8)
+      y = ((T)(u32)__builtin_amdgcn_readlane((int)(x >> 32), src) << 32) |
+          (u32)__builtin_amdgcn_readlane((int)x, src);
+    else
+      y = (u32)__builtin_amdgcn_readlane((int)x, src);
+    return wv ? y : (T)0;
+  }
+
+  // Sheets i * WT + t < w of this thread move from x[i] to x[i] + p[i]; r[i]
+  // becomes the sheet's rank and c[i] the mass below it, base included.
+  // SEGS: as `segs` says.
+  template <bool SEGS>
+  __device__ __forceinline__ void step(u32 w, double (&x)[PER],
+                                       const double (&p)[PER], u32 (&r)[PER],
+                                       const i32 (&ids)[PER],
+                                       const u64 (&m)[PER], u64 (&c)[PER],
+                                       u64 base) {
+    const u32 t = threadIdx.x;
+    u32 *const bn = bins + (s & 1u) * (NB + 1);
+    u32 b[PER], slot[PER];
+    float f[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      slot[i] = 0;
+      x[i] = x[i] + p[i];
+      double lo = x0, sc = scale;
+      u32 first = 0, cnt = NB;
+      if constexpr (SEGS) {
+        BinSeg sg = seg[g[i]];
+        if ((x[i] < sg.lo && g[i] > 0) || x[i] >= sg.next) {
+          while (g[i] > 0 && x[i] < seg[g[i]].lo) --g[i];
+          while (g[i] < BIN_SEGS - 1 && x[i] >= seg[g[i]].next) ++g[i];
+          sg = seg[g[i]];
+        }
+        lo = sg.lo;
+        sc = sg.scale;
+        first = sg.base;
+        cnt = sg.cnt;
+      }
+      // below the first segment's start: with its first; a segment's last bin
+      // also takes what rounds beyond it
+      const double q = fmin(fmax((x[i] - lo) * sc, 0.0), (double)cnt);
+      const u32 k = (u32)q;
+      b[i] = first + min(k, cnt - 1);
+      // the place within the bin: non-decreasing in x
+      f[i] = k == cnt ? 1.f : (float)__builtin_amdgcn_fract(q);
+      if (i * WT + t < w) {
+        slot[i] = atomicAdd(&bn[b[i]], 1u);  // its place in the bin
+      }
+    }
+    __syncthreads();
+    {
+      u32 loc[WPT];
+      u32 sum = 0;
+#pragma unroll
+      for (int q = 0; q < WPT; ++q) {
+        loc[q] = bn[t * WPT + q];
+        sum += loc[q];
+      }
+      u32 run = scan_excl<u32>(sum, red);
+      __syncthreads();
+      run += waves_before<u32>(red);
+#pragma unroll
+      for (int q = 0; q < WPT; ++q) {
+        bn[t * WPT + q] = run;
+        run += loc[q];
+      }
+      if (t == 0) bn[NB] = w;
+    }
+    __syncthreads();
+    u32 lo[PER], hi[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      lo[i] = hi[i] = 0;
+      if (i * WT + t < w) {
+        lo[i] = bn[b[i]];
+        hi[i] = bn[b[i] + 1u];
+        slot[i] += lo[i];
+        xf[slot[i]] = f[i];
+        xs[slot[i]] = x[i];
+        id[slot[i]] = ids[i];
+        if (MASS) ms[slot[i]] = m[i];
+      }
+    }
+    clear((s & 1u) ^ 1u);
+    ++s;
+    __syncthreads();
+    if (MASS) {  // ms becomes the mass below each slot
+      u64 lm[PER], sum = 0;
+#pragma unroll
+      for (int q = 0; q < PER; ++q) {
+        lm[q] = t * PER + q < w ? ms[t * PER + q] : 0ull;
+        sum += lm[q];
+      }
+      u64 run = scan_excl<u64>(sum, redm);
+      __syncthreads();
+      run += base + waves_before<u64>(redm);
+#pragma unroll
+      for (int q = 0; q < PER; ++q) {
+        ms[t * PER + q] = run;
+        run += lm[q];
+      }
+      if (t == WT - 1) ms[CAP] = run;
+      __syncthreads();
+    }
+    // Rank inside the bin: the sheets of the bin placed below.  The first PAD
+    // slots are read at once without a look at where the bin ends: what lies
+    // beyond is in a later bin (f starts again from 0: masked by the end).
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      u32 k = lo[i], eq = 0;
+      float y[PAD];
+      u64 my[PAD + 1];  // mass of a slot: the difference of neighbours
+#pragma unroll
+      for (int q = 0; q < PAD; ++q) {
+        y[q] = xf[lo[i] + q];
+        if (MASS) my[q] = ms[lo[i] + q];
+      }
+      if (MASS) my[PAD] = ms[lo[i] + PAD];
+      u64 cm = MASS ? my[0] : 0ull;
+#pragma unroll
+      for (int q = 0; q < PAD; ++q) {
+        const float z = lo[i] + q < hi[i] ? y[q] : 3.f;
+        k += z < f[i] ? 1u : 0u;
+        eq += z == f[i] ? 1u : 0u;
+        if (MASS) cm += z < f[i] ? my[q + 1] - my[q] : 0ull;
+      }
+      for (u32 a = lo[i] + PAD; a < hi[i]; ++a) {
+        const float z = xf[a];
+        k += z < f[i] ? 1u : 0u;
+        eq += z == f[i] ? 1u : 0u;
+        if (MASS && z < f[i]) cm += ms[a + 1] - ms[a];
+      }
+      if (eq > 1) {  // another sheet rounds to the same place: in full
+        for (u32 a = lo[i]; a < hi[i]; ++a)
+          if (xf[a] == f[i] && (xs[a] < x[i] || (xs[a] == x[i] && id[a] < ids[i]))) {
+            k += 1;
+            if (MASS) cm += ms[a + 1] - ms[a];
+          }
+      }
+      r[i] = k;
+      if (MASS) c[i] = cm;
     }
   }
 };

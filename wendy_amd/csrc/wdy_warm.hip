@@ -1372,6 +1372,11 @@ int warm_configure(wdy_sim *s, int shape, u32 T, u32 W) {
   return WDY_OK;
 }
 
+int warm_ensure(wdy_sim *s) {
+  if (s->warm || !s->warm_ok) return WDY_OK;
+  return warm_configure(s, s->warm_shape0, 0u, (u32)WARM_WINDOW_DEFAULT);
+}
+
 // Folds the phase stamps of the last warm launch into the running means.
 static void prof_fold(wdy_sim *s) {
   WarmCtx &w = *s->warm;
@@ -1653,6 +1658,7 @@ int warm_settle(wdy_sim *s, bool *failed, double *h, int *nleap) {
   w.rd = w.p_mstart;
   w.ready = false;
   if (kind & WARM_ERR_STALL) {  // not a sizing problem: stop using it
+    s->warm_ok = false;
     warm_free(s);
     return WDY_OK;
   }
@@ -1681,7 +1687,8 @@ int warm_settle(wdy_sim *s, bool *failed, double *h, int *nleap) {
     }
   }
   if (shape == w.shape && T == w.T && W == w.W) {  // limits reached: radix
-    warm_free(s);                                  // path from now on
+    s->warm_ok = false;                            // path from now on
+    warm_free(s);
     return WDY_OK;
   }
   return warm_configure(s, shape, T, W);

@@ -75,8 +75,9 @@ class Sim:
 
     def __init__(self, x, v, m, totmass, omega2, equal_mass=None, path=None,
                  warm=True, shared=False):
-        """``path``: None (by size), 'small' (one persistent workgroup per
-        output interval) or 'large' (whole-GPU steps).  ``warm=False`` keeps
+        """``path``: None (by size and step), 'small' (one persistent
+        workgroup, or one wave, per output interval) or 'large' (whole-GPU
+        steps).  ``warm=False`` keeps
         the large path on the full radix sort every step.  ``shared=True``:
         the simulation will run in a ``Gang`` beside others, so it keeps the
         throughput tile shape at every size (WDY_SHARED_GPU)."""
@@ -160,7 +161,8 @@ class Sim:
                                        int(window)))
 
     def path_stats(self):
-        """(warm-start steps, radix steps, redone intervals) so far."""
+        """(warm-start or window steps, radix steps, redone intervals) so far
+        (see wdy_path_stats)."""
         a, b, c = ctypes.c_int64(0), ctypes.c_int64(0), ctypes.c_int64(0)
         _lib.check(_lib.lib().wdy_path_stats(self._h, ctypes.byref(a),
                                              ctypes.byref(b), ctypes.byref(c)))
