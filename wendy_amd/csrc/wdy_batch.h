@@ -13,6 +13,10 @@ struct BatchDesc {
   int cur;        // current buffer set
   int nleap;      // leapfrog steps this interval (0: skip)
   u32 eslot;      // error word of this simulation: err[eslot]
+  // windows (see SpanArgs) of T + 2 H sheets, nwin in all, K steps a launch,
+  // L launches an interval (0: not in windows)
+  u32 T, H, nwin, K, L;
+  u32 vslot;      // its word sets, with several windows
   u32 pad_;
   double h;       // leapfrog step
   double mq, totmass, omega2, fscale, finv;
@@ -30,8 +34,13 @@ struct BatchArrays {
 
 // One workgroup per descriptor; descriptors in d_descs[0..count).  A
 // simulation that fails its on-device check sets err[its eslot].
+// iv: intervals since the descriptors' upload (their `cur` is where that one
+// left each simulation).  many: also keeps what the windows need of the
+// simulations that have any (see k_batch_advance).
+struct SpanMany;
 int batch_launch(hipStream_t st, const BatchDesc *d_descs, int count,
-                 const BatchArrays &arr, u32 *err);
+                 const BatchArrays &arr, u32 *err, const SpanMany *many = nullptr,
+                 u32 iv = 0);
 
 // Descriptor fields derived from a simulation's masses (equal-mass flag,
 // fixed-point scale of the exact unequal-mass prefix).

@@ -1,10 +1,24 @@
 // Batched ensemble: thousands of independent simulations of uneven N advance
 // together, ONE launch per output interval.
 //
-// Each simulation is handled by one 512-thread workgroup that runs all of
-// its leapfrog steps of the interval without returning to the host (a
-// persistent workgroup per simulation; descriptors are ordered largest
-// first so the longest workgroups start first).  State lives in one arena:
+// A batch's first interval, and every interval of the serving pool, runs one
+// 512-thread workgroup per simulation through all of its leapfrog steps (a
+// persistent workgroup per simulation; descriptors are ordered largest first so
+// the longest workgroups start first).  Its time is that of the largest
+// simulation: 3.4 ms for 10 steps of 65536 sheets.
+//
+// From the second interval on a batch runs in windows (wdy_span.h), one
+// workgroup or wave per (simulation, window) and several steps per launch,
+// planned on the host from the densities and speeds that k_batch_form reports.
+// Nothing waits for the host within a plan: a window that cannot vouch for its
+// core marks its simulation, whose later launches then leave it alone, and
+// k_batch_advance, which ends every interval, redoes the rest of the interval
+// from the marked launch's input (its two sets alternate by launch) and brings
+// it back into the windows' form.  Measured, us per interval of 10 steps at
+// h = 1e-3, before -> with windows: 100 disks of 5000-20000 sheets 962 -> 95
+// (lognormal masses 1183 -> 142), 4 of 40000-60000 2704 -> 59, 400 of 50-60
+// 44 -> 14, 384 of 256-65536 3600 -> 410.
+//  State lives in one arena:
 // simulation k occupies [off_k, off_k + n_k) of two buffer sets of SoA arrays
 // (key = order-preserving position encoding, velocity, global sheet index,
 // mass * twopiG); `cur` in the descriptor says which set is current.
@@ -36,6 +50,7 @@
 
 #include "wdy_batch.h"
 #include "wdy_lds.h"
+#include "wdy_span.h"
 
 namespace wdy {
 
@@ -206,8 +221,109 @@ __device__ __forceinline__ bool ordered(const u64 *key, const i32 *idx,
   return ka < kb || (ka == kb && idx[a] <= idx[b]);
 }
 
+// The arena range of one simulation into sorted order, in place: block
+// odd-even merge sort, until every boundary of the offset blocks is in order.
+// False when that takes more rounds than any input needs.
+__device__ bool range_sort(Lds<BSH, false> &s, u32 n, u64 *key, double *vel, i32 *idx,
+                           double *mass, u64 *s_red, u64 *s_mm, u32 *s_flag) {
+  const u32 t = threadIdx.x, half = BLOCK / 2;
+  const u32 max_rounds = (2 * n + BLOCK - 1) / BLOCK + 1;
+  bool sorted = false;
+  for (u32 round = 0; round < max_rounds && !sorted; ++round) {
+    for (u32 lo = 0; lo < n; lo += BLOCK)
+      block_sort_inplace(s, key, vel, idx, mass, lo, min((u32)BLOCK, n - lo),
+                         s_red, s_mm);
+    for (u32 lo = half; lo < n; lo += BLOCK)
+      block_sort_inplace(s, key, vel, idx, mass, lo, min((u32)BLOCK, n - lo),
+                         s_red, s_mm);
+    // every boundary of the offset blocks in order -> the range is sorted
+    if (t == 0) *s_flag = 1;
+    __syncthreads();
+    for (u32 b = half + (u32)t * BLOCK; b < n; b += (u32)BWT * BLOCK)
+      if (!ordered(key, idx, b - 1, b)) *s_flag = 0;
+    __syncthreads();
+    sorted = *s_flag != 0;
+    __syncthreads();
+  }
+  return sorted;
+}
+
+// Brings set a into the form the windows read: sorted, with the mass below
+// each sheet and the speed words of the next launch (ep since the plan), and
+// tells the host the densities and the largest speed.
+__device__ void window_form(Lds<BSH, false> &s, const BatchDesc &d, const BatchArrays &A,
+                            const SpanMany &M, int a, u32 ep, u32 *err, u64 *s_red,
+                            u64 *s_mm, u32 *s_flag) {
+  const u32 t = threadIdx.x, n = d.n;
+  const bool eq = d.flags & 1u;
+  u64 *key = A.key[a] + d.off;
+  double *vel = A.vel[a] + d.off;
+  double *mass = eq ? nullptr : A.mass[a] + d.off;
+  if (!range_sort(s, n, key, vel, A.idx[a] + d.off, mass, s_red, s_mm, s_flag) && t == 0)
+    atomicOr(err + d.eslot, 1u);
+  if (!eq) {
+    u64 *cf = M.cf[a] + d.off;
+    u64 run = 0;
+    for (u32 lo = 0; lo < n; lo += BLOCK) {
+      u64 m[BPER], part = 0, total;
+#pragma unroll
+      for (int i = 0; i < BPER; ++i) {
+        const u32 r = lo + t * BPER + i;
+        m[i] = r < n ? mass_fix(mass[r], d.fscale) : 0ull;
+        part += m[i];
+      }
+      u64 c = run + block_excl_u64<BNWAVE>(part, s_red, &total);
+#pragma unroll
+      for (int i = 0; i < BPER; ++i) {
+        const u32 r = lo + t * BPER + i;
+        if (r < n) cf[r] = c;
+        c += m[i];
+      }
+      run += total;
+      __syncthreads();
+    }
+  }
+  // [0, SPAN_NW): ~width, so that all are maxima; then the speed
+  u64 top[SPAN_NW + 1];
+#pragma unroll
+  for (u32 k = 0; k <= SPAN_NW; ++k) top[k] = 0;
+  for (u32 i = t; i < n; i += BWT) {
+    const double x = decode_pos(key[i]);
+    top[SPAN_NW] = max(top[SPAN_NW], (u64)__double_as_longlong(fabs(vel[i])));
+#pragma unroll
+    for (u32 k = 0; k < SPAN_NW; ++k)
+      if (i + (4u << k) < n)
+        top[k] = max(top[k], ~(u64)__double_as_longlong(decode_pos(key[i + (4u << k)]) - x));
+  }
+#pragma unroll
+  for (u32 k = 0; k <= SPAN_NW; ++k) {
+    const u64 w = wave_max(top[k]);
+    __syncthreads();
+    if ((t & 63u) == 0) s_red[t >> 6] = w;
+    __syncthreads();
+    u64 m = 0;
+    for (int q = 0; q < BNWAVE; ++q) m = max(m, s_red[q]);
+    top[k] = m;
+  }
+  if (t == 0) {
+    double *info = M.info + (u64)d.eslot * SPAN_INFO;
+#pragma unroll
+    for (u32 k = 0; k < SPAN_NW; ++k)
+      info[k] = top[k] ? __longlong_as_double((long long)~top[k]) : 1e308;
+    info[SPAN_NW] = __longlong_as_double((long long)top[SPAN_NW]);
+  }
+  if (d.nwin > 1)
+    for (u32 i = t; i < 3 * SPAN_SLOTS; i += BWT)
+      M.vmax[(u64)d.vslot * 3u * SPAN_SLOTS + i] =
+          i == (ep % 3u) * SPAN_SLOTS ? top[SPAN_NW] : 0ull;
+}
+
+// WINDOWS: with windows, launched after those of interval iv.  Simulations in
+// windows only take part when one failed: the rest of the interval from the
+// failed launch's input, then window_form.
+template <bool WINDOWS>
 __global__ __launch_bounds__(BWT) void k_batch_advance(
-    const BatchDesc *__restrict__ descs, BatchArrays A, u32 *err) {
+    const BatchDesc *__restrict__ descs, BatchArrays A, u32 *err, SpanMany M, u32 iv) {
   extern __shared__ u64 lds_dyn[];
   Lds<BSH, false> s(lds_dyn);
   __shared__ u64 s_red[BNWAVE];
@@ -220,7 +336,24 @@ __global__ __launch_bounds__(BWT) void k_batch_advance(
   if (d.nleap <= 0 || n == 0) return;
   const bool eq = d.flags & 1u;
   const double hh = d.h / 2.;
-  int a = d.cur;
+  // the sets that interval iv since the descriptors' upload starts and ends in
+  const u32 per = d.L ? d.L : (u32)d.nleap;
+  int a = d.cur ^ (int)((iv * per) & 1u), step0 = 0;
+  const int end = a ^ (int)(per & 1u);
+  if (WINDOWS) {
+    if (d.L) {
+      const u32 f = M.fail[d.eslot];
+      u32 *stat = M.stat + (u64)d.vslot * SPAN_SLOTS;
+      if (d.nwin > 1 && t < 64u) {
+        const u32 m = (u32)~wave_max((u64)~stat[t]);
+        stat[t] = SPAN_STAT_INIT;
+        if (t == 0) M.slack[d.eslot] = f ? 0u : m;
+      }
+      if (f == 0) return;
+      step0 = (int)((f - 1u) * d.K);
+      a ^= (int)((f - 1u) & 1u);
+    }
+  }
 
   if (n <= (u32)BLOCK) {
     // ---- the whole simulation in LDS for the interval ------------------------
@@ -233,18 +366,19 @@ __global__ __launch_bounds__(BWT) void k_batch_advance(
       const u32 e = i * BWT + t;
       if (e < n) {
         const double v = vel[e];
-        s.key[e] = encode_pos(decode_pos(key[e]) + hh * v);  // first half drift
+        // first half drift
+        s.key[e] = step0 ? key[e] : encode_pos(decode_pos(key[e]) + hh * v);
         s.v[e] = v;
         s.id[e] = idx[e];
         s.m[e] = mass ? mass[e] : 0.0;
       }
     }
     __syncthreads();
-    for (int step = 0; step < d.nleap; ++step) {
+    for (int step = step0; step < d.nleap; ++step) {
       lds_bucket_sort<BSH, false>(s, n, s_red, s_mm, nullptr);
       (void)block_leap(s, d, n, 0, 0, step == d.nleap - 1 ? hh : d.h, s_red);
     }
-    const int b = a ^ (d.nleap & 1);
+    const int b = end;
     u64 *ko = A.key[b] + d.off;
     double *vo = A.vel[b] + d.off;
     i32 *io = A.idx[b] + d.off;
@@ -260,19 +394,22 @@ __global__ __launch_bounds__(BWT) void k_batch_advance(
         if (mo) mo[r] = s.m[e];
       }
     }
+    if (WINDOWS && d.L) {
+      __syncthreads();
+      window_form(s, d, A, M, end, (iv + 1) * d.L, err, s_red, s_mm, &s_flag);
+      if (t == 0) M.fail[d.eslot] = 0;
+    }
     return;
   }
 
   // ---- larger simulations: arena-resident, block odd-even merge sort ---------
-  {  // first half drift, in place
+  if (step0 == 0) {  // first half drift, in place
     u64 *key = A.key[a] + d.off;
     const double *vel = A.vel[a] + d.off;
     for (u32 i = t; i < n; i += BWT) key[i] = encode_pos(decode_pos(key[i]) + hh * vel[i]);
     __syncthreads();
   }
-  const u32 half = BLOCK / 2;
-  const u32 max_rounds = (2 * n + BLOCK - 1) / BLOCK + 1;
-  for (int step = 0; step < d.nleap; ++step) {
+  for (int step = step0; step < d.nleap; ++step) {
     u64 *key = A.key[a] + d.off;
     double *vel = A.vel[a] + d.off;
     i32 *idx = A.idx[a] + d.off;
@@ -288,23 +425,7 @@ __global__ __launch_bounds__(BWT) void k_batch_advance(
         continue;
       }
     }
-    bool sorted = false;
-    for (u32 round = 0; round < max_rounds && !sorted; ++round) {
-      for (u32 lo = 0; lo < n; lo += BLOCK)
-        block_sort_inplace(s, key, vel, idx, mass, lo, min((u32)BLOCK, n - lo),
-                           s_red, s_mm);
-      for (u32 lo = half; lo < n; lo += BLOCK)
-        block_sort_inplace(s, key, vel, idx, mass, lo, min((u32)BLOCK, n - lo),
-                           s_red, s_mm);
-      // every boundary of the offset blocks in order -> the range is sorted
-      if (t == 0) s_flag = 1;
-      __syncthreads();
-      for (u32 b = half + (u32)t * BLOCK; b < n; b += (u32)BWT * BLOCK)
-        if (!ordered(key, idx, b - 1, b)) s_flag = 0;
-      __syncthreads();
-      sorted = s_flag != 0;
-      __syncthreads();
-    }
+    const bool sorted = range_sort(s, n, key, vel, idx, mass, s_red, s_mm, &s_flag);
     if (!sorted && t == 0) atomicOr(err + d.eslot, 1u);  // not expected: bound above
     // force, kick, drift, block by block, into the other buffer set
     const int b = a ^ 1;
@@ -343,6 +464,41 @@ __global__ __launch_bounds__(BWT) void k_batch_advance(
     }
     a = b;
   }
+  if (WINDOWS && d.L) {
+    if (a != end) {
+      for (u32 i = t; i < n; i += BWT) {
+        const u64 p = d.off + i;
+        A.key[end][p] = A.key[a][p];
+        A.vel[end][p] = A.vel[a][p];
+        A.idx[end][p] = A.idx[a][p];
+        if (!eq) A.mass[end][p] = A.mass[a][p];
+      }
+      __syncthreads();
+    }
+    window_form(s, d, A, M, end, (iv + 1) * d.L, err, s_red, s_mm, &s_flag);
+    if (t == 0) M.fail[d.eslot] = 0;
+  }
+}
+
+// Every simulation's current set into the windows' form, before a plan's first
+// interval.
+__global__ __launch_bounds__(BWT) void k_batch_form(const BatchDesc *__restrict__ descs,
+                                                    BatchArrays A, SpanMany M, u32 *err) {
+  extern __shared__ u64 lds_dyn[];
+  Lds<BSH, false> s(lds_dyn);
+  __shared__ u64 s_red[BNWAVE];
+  __shared__ u64 s_mm[2 * BNWAVE];
+  __shared__ u32 s_flag;
+  const BatchDesc d = descs[blockIdx.x];
+  const u32 t = threadIdx.x;
+  window_form(s, d, A, M, d.cur, 0u, err, s_red, s_mm, &s_flag);
+  if (d.nwin > 1)
+    for (u32 i = t; i < SPAN_SLOTS; i += BWT)
+      M.stat[(u64)d.vslot * SPAN_SLOTS + i] = SPAN_STAT_INIT;
+  if (t == 0) {
+    M.fail[d.eslot] = 0;
+    M.slack[d.eslot] = SPAN_STAT_INIT;
+  }
 }
 
 }  // namespace
@@ -357,7 +513,7 @@ void batch_desc_fill(BatchDesc &d, const double *m, u32 n, double totmass,
   d.cur = 0;
   d.nleap = 0;
   d.eslot = 0;
-  d.pad_ = 0;
+  d.T = d.H = d.nwin = d.K = d.L = d.vslot = d.pad_ = 0;
   d.h = 0.0;
   d.mq = m[0];
   d.totmass = totmass;
@@ -370,13 +526,14 @@ void batch_desc_fill(BatchDesc &d, const double *m, u32 n, double totmass,
 }
 
 int batch_launch(hipStream_t st, const BatchDesc *d_descs, int count,
-                 const BatchArrays &arr, u32 *err) {
+                 const BatchArrays &arr, u32 *err, const SpanMany *many, u32 iv) {
   if (count <= 0) return WDY_OK;
   const size_t lds = Lds<BSH, false>::BYTES;
-  WDY_HIP(hipFuncSetAttribute((const void *)k_batch_advance,
+  auto fn = many ? k_batch_advance<true> : k_batch_advance<false>;
+  WDY_HIP(hipFuncSetAttribute((const void *)fn,
                               hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)lds));
-  k_batch_advance<<<count, BWT, lds, st>>>(d_descs, arr, err);
+  fn<<<count, BWT, lds, st>>>(d_descs, arr, err, many ? *many : SpanMany{}, iv);
   WDY_CHECK_LAUNCH();
   return WDY_OK;
 }
@@ -400,21 +557,16 @@ __global__ void k_batch_init(u64 n, const double *__restrict__ x,
 // One workgroup per descriptor: de-sort its current set into x_out, v_out
 // (arena order, i.e. each simulation's sheets in input order).
 __global__ void k_batch_desort(const BatchDesc *__restrict__ descs,
-                               BatchArrays A, double *__restrict__ xo,
+                               BatchArrays A, u32 iv, double *__restrict__ xo,
                                double *__restrict__ vo) {
   const BatchDesc d = descs[blockIdx.x];
-  const int c = d.cur;
+  const int c = d.cur ^ (int)((iv * (d.L ? d.L : (u32)d.nleap)) & 1u);
   for (u32 i = threadIdx.x; i < d.n; i += blockDim.x) {
     const u64 p = d.off + i;
     const i32 j = A.idx[c][p];
     xo[j] = decode_pos(A.key[c][p]);
     vo[j] = A.vel[c][p];
   }
-}
-
-__global__ void k_batch_flip(BatchDesc *descs, int count) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < count && descs[i].nleap > 0) descs[i].cur ^= (descs[i].nleap & 1);
 }
 
 }  // namespace
@@ -429,7 +581,16 @@ struct wdy_batch {
   u64 ntot = 0;
   BatchArrays arr{};
   BatchDesc *d_desc = nullptr;
-  std::vector<BatchDesc> h_desc;  // launch order: largest first
+  std::vector<BatchDesc> h_desc;  // launch order: largest first, as uploaded
+  u32 iv = 0;                     // intervals since that upload
+  // windows
+  SpanMany many{};
+  bool planned = false, started = false;
+  int shape = -1;        // -1: no simulation in windows
+  u32 neq = 0, nun = 0;  // windows of the equal and the unequal simulations
+  u32 launches = 0;
+  uint2 *d_list = nullptr;
+  std::vector<double> reach;  // per descriptor
   double *out_x = nullptr, *out_v = nullptr;
   u32 *err = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -445,6 +606,12 @@ static void batch_free(wdy_batch *b) {
     if (b->arr.idx[s]) (void)hipFree(b->arr.idx[s]);
     if (b->arr.mass[s]) (void)hipFree(b->arr.mass[s]);
   }
+  for (u64 *p : b->many.cf)
+    if (p) (void)hipFree(p);
+  if (b->many.vmax) (void)hipFree(b->many.vmax);
+  if (b->many.fail) (void)hipFree(b->many.fail);
+  if (b->many.info) (void)hipHostFree(b->many.info);
+  if (b->d_list) (void)hipFree(b->d_list);
   if (b->d_desc) (void)hipFree(b->d_desc);
   if (b->out_x) (void)hipFree(b->out_x);
   if (b->out_v) (void)hipFree(b->out_v);
@@ -453,6 +620,82 @@ static void batch_free(wdy_batch *b) {
   if (b->ev1) (void)hipEventDestroy(b->ev1);
   if (b->stream) (void)hipStreamDestroy(b->stream);
   delete b;
+}
+
+// New step parameters and, once the simulations are in order, windows.
+static int batch_plan(wdy_batch *b, double h, int nleap) {
+  std::vector<BatchDesc> &d = b->h_desc;
+  WDY_HIP(hipStreamSynchronize(b->stream));
+  for (size_t k = 0; k < d.size(); ++k) {
+    BatchDesc &q = d[k];
+    q.cur ^= (int)((b->iv * (q.L ? q.L : (u32)q.nleap)) & 1u);
+    if (b->shape >= 0 && q.L) {
+      float f;
+      __builtin_memcpy(&f, &b->many.slack[k], 4);
+      if (f < 1.05f) b->reach[k] *= f > 0.f ? 1.25 : 1.6;
+    }
+    q.L = q.nwin = 0;
+    q.h = h;
+    q.nleap = nleap;
+  }
+  b->iv = 0;
+  b->h = h;
+  b->nleap = nleap;
+  b->shape = -1;
+  const size_t bytes = d.size() * sizeof(BatchDesc);
+  auto upload = [&]() -> int {
+    WDY_HIP(hipMemcpyAsync(b->d_desc, d.data(), bytes, hipMemcpyHostToDevice, b->stream));
+    WDY_HIP(hipStreamSynchronize(b->stream));
+    return WDY_OK;
+  };
+  if (int rc = upload()) return rc;
+  b->planned = b->started;
+  if (!b->planned) return WDY_OK;
+  SpanMany &m = b->many;
+  const size_t S = d.size();
+  if (!m.fail) {
+    WDY_HIP(hipMalloc(&m.fail, S * 4));
+    WDY_HIP(hipHostMalloc((void **)&m.info, S * (SPAN_INFO * 8 + 4), hipHostMallocDefault));
+    m.slack = (u32 *)(m.info + S * SPAN_INFO);
+    if (b->arr.mass[0])
+      for (u64 *&p : m.cf) WDY_HIP(hipMalloc(&p, b->ntot * 8));
+  }
+  const size_t lds = Lds<BSH, false>::BYTES;
+  WDY_HIP(hipFuncSetAttribute((const void *)k_batch_form,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  auto form = [&]() -> int {
+    k_batch_form<<<(unsigned)S, BWT, lds, b->stream>>>(b->d_desc, b->arr, m, b->err);
+    WDY_CHECK_LAUNCH();
+    return WDY_OK;
+  };
+  if (int rc = form()) return rc;
+  WDY_HIP(hipStreamSynchronize(b->stream));
+  span_many_plan(d, m.info, b->reach, h, nleap, &b->shape);
+  if (b->shape < 0) return upload();
+  std::vector<uint2> list[2];
+  size_t words = 0;
+  b->launches = 0;
+  for (size_t k = 0; k < S; ++k) {
+    for (u32 j = 0; d[k].L && j < d[k].nwin; ++j)
+      list[d[k].flags & 1u ? 0 : 1].push_back(make_uint2((u32)k, j));
+    words += d[k].nwin > 1 ? 1 : 0;
+    b->launches = std::max(b->launches, d[k].L);
+  }
+  b->neq = (u32)list[0].size();
+  b->nun = (u32)list[1].size();
+  list[0].insert(list[0].end(), list[1].begin(), list[1].end());
+  if (b->d_list) WDY_HIP(hipFree(b->d_list));
+  b->d_list = nullptr;
+  WDY_HIP(hipMalloc(&b->d_list, list[0].size() * sizeof(uint2)));
+  WDY_HIP(hipMemcpyAsync(b->d_list, list[0].data(), list[0].size() * sizeof(uint2),
+                         hipMemcpyHostToDevice, b->stream));
+  if (m.vmax) WDY_HIP(hipFree(m.vmax));
+  m.vmax = nullptr;
+  WDY_HIP(hipMalloc(&m.vmax, (words ? words : 1) * SPAN_SLOTS * (3 * 8 + 4)));
+  m.stat = (u32 *)(m.vmax + words * SPAN_SLOTS * 3);
+  if (int rc = upload()) return rc;
+  // the speed words of the plan's first launch
+  return form();
 }
 
 extern "C" {
@@ -506,7 +749,9 @@ int wdy_batch_create(int64_t nsims, const int64_t *offsets, const double *x,
     }
     std::stable_sort(descs.begin(), descs.end(),
                      [](const BatchDesc &p, const BatchDesc &q) { return p.n > q.n; });
+    for (size_t k = 0; k < descs.size(); ++k) descs[k].eslot = (u32)k;
     b->h_desc = descs;
+    b->reach.assign(descs.size(), 1.0);
     const size_t N = (size_t)ntot;
     for (int s = 0; s < 2; ++s) {
       WDY_HIP(hipMalloc(&b->arr.key[s], N * 8));
@@ -517,8 +762,8 @@ int wdy_batch_create(int64_t nsims, const int64_t *offsets, const double *x,
     WDY_HIP(hipMalloc(&b->d_desc, descs.size() * sizeof(BatchDesc)));
     WDY_HIP(hipMalloc(&b->out_x, N * 8));
     WDY_HIP(hipMalloc(&b->out_v, N * 8));
-    WDY_HIP(hipMalloc(&b->err, 8));
-    WDY_HIP(hipMemsetAsync(b->err, 0, 8, b->stream));
+    WDY_HIP(hipMalloc(&b->err, (size_t)nsims * 4));
+    WDY_HIP(hipMemsetAsync(b->err, 0, (size_t)nsims * 4, b->stream));
     WDY_HIP(hipMemcpyAsync(b->d_desc, descs.data(), descs.size() * sizeof(BatchDesc),
                            hipMemcpyHostToDevice, b->stream));
     WDY_HIP(hipMemcpyAsync(b->out_x, x, N * 8, hipMemcpyHostToDevice, b->stream));
@@ -545,29 +790,31 @@ int wdy_batch_advance(wdy_batch *b, double h, int nleap) {
   if (nleap < 1 || !std::isfinite(h))
     return fail(WDY_EINVAL, "wdy_batch_advance: bad h or nleap");
   WDY_HIP(hipSetDevice(b->device));
-  if (h != b->h || nleap != b->nleap) {
-    // descriptors live on the device (their `cur` flips there); update the
-    // step parameters in place by re-uploading after a read of `cur`
-    std::vector<BatchDesc> cur(b->h_desc.size());
-    WDY_HIP(hipMemcpyAsync(cur.data(), b->d_desc, cur.size() * sizeof(BatchDesc),
-                           hipMemcpyDeviceToHost, b->stream));
-    WDY_HIP(hipStreamSynchronize(b->stream));
-    for (auto &d : cur) {
-      d.h = h;
-      d.nleap = nleap;
+  const bool change = h != b->h || nleap != b->nleap;
+  // A batch's first interval puts every simulation in order; from the second
+  // on it runs in windows.  A plan stays until h or nleap changes or a halo
+  // gets tight (the reports are the host's to read at any time: they only say
+  // when to look again).
+  bool plan = change || !b->planned;
+  if (!plan && b->shape >= 0)
+    for (size_t k = 0; k < b->h_desc.size() && !plan; ++k) {
+      float f;
+      __builtin_memcpy(&f, &b->many.slack[k], 4);
+      plan = b->h_desc[k].L != 0 && f < 1.05f;
     }
-    WDY_HIP(hipMemcpyAsync(b->d_desc, cur.data(), cur.size() * sizeof(BatchDesc),
-                           hipMemcpyHostToDevice, b->stream));
-    WDY_HIP(hipStreamSynchronize(b->stream));
-    b->h = h;
-    b->nleap = nleap;
-  }
+  if (plan)
+    if (int rc = batch_plan(b, h, nleap)) return rc;
   WDY_HIP(hipEventRecord(b->ev0, b->stream));
-  if (int rc = batch_launch(b->stream, b->d_desc, (int)b->nsims, b->arr, b->err))
+  if (b->shape >= 0)
+    for (u32 q = 0; q < b->launches; ++q)
+      if (int rc = span_many_launch(b->stream, b->shape, b->d_desc, b->d_list, b->neq,
+                                    b->nun, b->arr, b->many, q, b->iv))
+        return rc;
+  if (int rc = batch_launch(b->stream, b->d_desc, (int)b->nsims, b->arr, b->err,
+                            b->shape >= 0 ? &b->many : nullptr, b->iv))
     return rc;
-  k_batch_flip<<<(unsigned)((b->nsims + 255) / 256), 256, 0, b->stream>>>(
-      b->d_desc, (int)b->nsims);
-  WDY_CHECK_LAUNCH();
+  ++b->iv;
+  b->started = true;
   WDY_HIP(hipEventRecord(b->ev1, b->stream));
   return WDY_OK;
 }
@@ -578,8 +825,8 @@ int wdy_batch_read(wdy_batch *b, double *x_out, double *v_out,
   WDY_HIP(hipSetDevice(b->device));
   const size_t N = (size_t)b->ntot;
   if (x_out || v_out) {
-    k_batch_desort<<<(unsigned)b->nsims, 256, 0, b->stream>>>(b->d_desc, b->arr,
-                                                               b->out_x, b->out_v);
+    k_batch_desort<<<(unsigned)b->nsims, 256, 0, b->stream>>>(
+        b->d_desc, b->arr, b->iv, b->out_x, b->out_v);
     WDY_CHECK_LAUNCH();
     if (x_out)
       WDY_HIP(hipMemcpyAsync(x_out, b->out_x, N * 8, hipMemcpyDeviceToHost,
@@ -588,9 +835,12 @@ int wdy_batch_read(wdy_batch *b, double *x_out, double *v_out,
       WDY_HIP(hipMemcpyAsync(v_out, b->out_v, N * 8, hipMemcpyDeviceToHost,
                              b->stream));
   }
-  u32 err = 0;
-  WDY_HIP(hipMemcpyAsync(&err, b->err, 4, hipMemcpyDeviceToHost, b->stream));
+  std::vector<u32> errs((size_t)b->nsims);
+  WDY_HIP(hipMemcpyAsync(errs.data(), b->err, errs.size() * 4, hipMemcpyDeviceToHost,
+                         b->stream));
   WDY_HIP(hipStreamSynchronize(b->stream));
+  u32 err = 0;
+  for (u32 e : errs) err |= e;
   if (err)
     return fail(WDY_EVERIFY, "wdy_batch_read: a simulation did not sort within "
                 "its bound");

@@ -1,6 +1,9 @@
 // Shared declarations of the multi-step window kernels (wdy_span.hip).
 #pragma once
 
+#include <vector>
+
+#include "wdy_batch.h"
 #include "wdy_internal.h"
 
 namespace wdy {
@@ -30,14 +33,18 @@ struct SpanArgs {
   double amax0, amax1;  // |acceleration| <= amax0 + amax1 * |x|
   ExtForce ext;
   double t;              // force time of the first step
-  const u64 *vmax_in;    // [SPAN_SLOTS] bits of the largest |v| of the state read
-  u64 *vmax_out;         // of the state written (cleared by an earlier launch)
-  u64 *vmax_clr;         // cleared for the next launch
+  // [SPAN_SLOTS] bits of the largest |v| of the state read, of the state
+  // written (cleared by an earlier launch), and words cleared for the next
+  // launch; all null where one window takes the whole simulation for good
+  const u64 *vmax_in;
+  u64 *vmax_out;
+  u64 *vmax_clr;
   u32 *stat;             // [SPAN_SLOTS] float bits of the smallest halo width /
-                         // reach; 0: a window could not vouch for its core
-  u32 *stat_host;        // one window: set to 0 if a sheet is no longer finite
-                         // (pinned host memory)
-  u32 *stat_clr;         // stat words of the next interval, to be reset
+                         // reach, with several windows
+  u32 *stat_clr;         // stat words of the next interval, to be reset (or null)
+  u32 *stat_host;        // copies of stat in pinned host memory (or null)
+  u32 *fail;             // set to fail_value if a window could not vouch for its
+  u32 fail_value;        // core, or a sheet is no longer finite
 };
 
 // Window shapes: one wave (WaveSort), or a workgroup (BinRank).
@@ -48,5 +55,28 @@ struct SpanShape {
 constexpr int SPAN_NSHAPES = 10;
 const SpanShape &span_shape(int i);
 int span_launch(hipStream_t st, int shape, bool eq, const SpanArgs &a);
+
+// ---- many simulations per launch (a batch) -----------------------------------
+// What the device keeps and reports of a batch's simulations.
+struct SpanMany {
+  u64 *cf[2];   // fixed-point mass below each sheet, per set (null: none unequal)
+  u64 *vmax;    // [vslot][3][SPAN_SLOTS]: the word sets of SpanArgs
+  u32 *stat;    // [vslot][SPAN_SLOTS]
+  u32 *fail;    // [simulation] 0, or 1 + the launch of the interval that failed
+  u32 *slack;   // [simulation] pinned: the interval's smallest stat, 0: repaired
+  double *info; // [simulation][SPAN_INFO] pinned: SPAN_NW widths, max |v|
+};
+constexpr u32 SPAN_NW = 10;
+constexpr u32 SPAN_INFO = 12;
+// Sets shape and each simulation's T, H, nwin, K, L, vslot for intervals of
+// nleap steps of h from what the device reported; L = 0 where the windows do
+// not hold.  reach[i] scales simulation i's halo.
+void span_many_plan(std::vector<BatchDesc> &d, const double *info,
+                    const std::vector<double> &reach, double h, int nleap, int *shape);
+// Launch q of interval iv since the plan; list: (simulation, window) of nwin
+// windows, those of simulations with equal masses before the others.
+int span_many_launch(hipStream_t st, int shape, const BatchDesc *descs,
+                     const uint2 *list, u32 neq, u32 nun, const BatchArrays &arr,
+                     const SpanMany &m, u32 q, u32 iv);
 
 }  // namespace wdy

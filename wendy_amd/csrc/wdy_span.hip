@@ -56,7 +56,7 @@ __device__ __forceinline__ Reach span_reach(const SpanArgs &A, const u32 j) {
   const double xm = fmax(fabs(decode_pos(A.kin[0])), fabs(decode_pos(A.kin[A.n - 1])));
   const double amax = A.amax0 + A.amax1 * xm;  // of any sheet, all forces
   const double S = fabs(A.pre) + (double)(A.K - 1) * fabs(A.h) + fabs(A.hlast);
-  const u64 vin = wave_max(A.vmax_in[threadIdx.x & (SPAN_SLOTS - 1)]);
+  const u64 vin = A.vmax_in ? wave_max(A.vmax_in[threadIdx.x & (SPAN_SLOTS - 1)]) : 0ull;
   R.V = 1.03 * (bits_double(vin) + (double)A.K * fabs(A.h) * amax);
   R.D = R.V * S * 1.0001 + (double)(A.K + 2) * 3.0e-16 * xm;
   if (A.nwin == 1) R.V = 1.7976931348623157e308;  // no outside: finite is enough
@@ -74,8 +74,8 @@ __device__ __forceinline__ Reach span_reach(const SpanArgs &A, const u32 j) {
     R.slack = fminf(R.slack, (float)(d / R.D));
   }
   if (j == 0 && threadIdx.x < SPAN_SLOTS) {
-    A.vmax_clr[threadIdx.x] = 0;
-    A.stat_clr[threadIdx.x] = SPAN_STAT_INIT;
+    if (A.vmax_clr) A.vmax_clr[threadIdx.x] = 0;
+    if (A.stat_clr) A.stat_clr[threadIdx.x] = SPAN_STAT_INIT;
   }
   return R;
 }
@@ -102,20 +102,25 @@ __device__ __forceinline__ void span_store(const SpanArgs &A, Reach &R, u32 r,
   }
 }
 
-// One thread of the window reports: sb, its verdict as stat holds it; vm, the
-// bits of the core's largest speed.
+// One thread of the window reports: sb, its verdict (the float bits of its
+// slack, 0: it cannot vouch for its core); vm, the bits of the core's largest
+// speed.
 __device__ __forceinline__ u32 span_verdict(const Reach &R) {
   return R.ok ? min(__float_as_uint(fmaxf(R.slack, 0.f)), SPAN_STAT_INIT) : 0u;
 }
 __device__ __forceinline__ void span_report(const SpanArgs &A, u32 j, u32 sb, u64 vm) {
   const u32 q = j & (SPAN_SLOTS - 1);
-  // (a stale word only costs an atomic that changes nothing)
-  if (A.nwin > 1) {
-    if (sb < A.stat[q]) atomicMin(A.stat + q, sb);
-  } else if (sb == 0) {
-    *A.stat_host = 0;
+  if (sb == 0) {
+    *A.fail = A.fail_value;
+    return;
   }
-  if (vm > A.vmax_out[q])
+  // (a stale word only costs an atomic that changes nothing; the host's copies
+  // are for the next plan's halos, where a lost race does not matter)
+  if (A.nwin > 1 && sb < A.stat[q]) {
+    atomicMin(A.stat + q, sb);
+    if (A.stat_host) A.stat_host[q] = sb;
+  }
+  if (A.vmax_out && vm > A.vmax_out[q])
     atomicMax((unsigned long long *)A.vmax_out + q, (unsigned long long)vm);
 }
 
@@ -332,6 +337,78 @@ int launch_block(hipStream_t st, bool eq, const SpanArgs &a) {
             : launch_block_one<SH, false, false>(st, a);
 }
 
+// Windows of many simulations: one wave (PER > 0: PER sheets per lane) or
+// workgroup per (simulation, window).
+template <int PER, class SH, bool EQ>
+__global__ __launch_bounds__(PER ? 64 : SH::WT) void k_span_many(
+    const BatchDesc *__restrict__ descs, const uint2 *__restrict__ list, BatchArrays arr,
+    SpanMany M, u32 q, u32 iv) {
+  const uint2 e = list[blockIdx.x];
+  const BatchDesc d = descs[e.x];
+  const int done = (int)(q * d.K);
+  if (M.fail[d.eslot] != 0 || done >= d.nleap) return;
+  const int K = min((int)d.K, d.nleap - done);
+  const u32 ep = iv * d.L + q;  // launches since the plan
+  const int in = d.cur ^ (int)(ep & 1u), out = in ^ 1;
+  SpanArgs A;
+  A.n = d.n;
+  A.T = d.T;
+  A.H = d.H;
+  A.nwin = d.nwin;
+  A.K = (u32)K;
+  A.kin = arr.key[in] + d.off;
+  A.vin = arr.vel[in] + d.off;
+  A.iin = arr.idx[in] + d.off;
+  A.kout = arr.key[out] + d.off;
+  A.vout = arr.vel[out] + d.off;
+  A.iout = arr.idx[out] + d.off;
+  if (!EQ) {
+    A.min = arr.mass[in] + d.off;
+    A.cin = M.cf[in] + d.off;
+    A.mout = arr.mass[out] + d.off;
+    A.cout = M.cf[out] + d.off;
+  }
+  A.pre = done == 0 ? d.h / 2. : 0.0;
+  A.h = d.h;
+  A.hlast = done + K == d.nleap ? d.h / 2. : d.h;
+  A.mq = d.mq;
+  A.totmass = d.totmass;
+  A.omega2 = d.flags & 2u ? d.omega2 : 0.0;
+  A.fscale = d.fscale;
+  A.finv = d.finv;
+  A.amax0 = fabs(d.totmass);
+  A.amax1 = A.omega2;
+  A.t = 0.0;
+  u64 *const vm = d.nwin > 1 ? M.vmax + (u64)d.vslot * 3u * SPAN_SLOTS : nullptr;
+  A.vmax_in = vm ? vm + (ep % 3u) * SPAN_SLOTS : nullptr;
+  A.vmax_out = vm ? vm + ((ep + 1u) % 3u) * SPAN_SLOTS : nullptr;
+  A.vmax_clr = vm ? vm + ((ep + 2u) % 3u) * SPAN_SLOTS : nullptr;
+  A.stat = d.nwin > 1 ? M.stat + (u64)d.vslot * SPAN_SLOTS : nullptr;
+  A.stat_clr = nullptr;
+  A.stat_host = nullptr;
+  A.fail = M.fail + d.eslot;
+  A.fail_value = q + 1u;
+  if constexpr (PER > 0)
+    span_wave<PER, EQ, false>(A, e.y);
+  else
+    span_block<SH, EQ, false>(A, e.y);
+}
+
+template <int PER, class SH, bool EQ>
+int launch_many(hipStream_t st, const BatchDesc *descs, const uint2 *list, u32 nblk,
+                const BatchArrays &arr, const SpanMany &m, u32 q, u32 iv) {
+  if (nblk == 0) return WDY_OK;
+  auto fn = k_span_many<PER, SH, EQ>;
+  const size_t lds = PER ? 0 : BinRank<SH, !EQ>::BYTES;
+  if (lds > 65536)
+    WDY_HIP(hipFuncSetAttribute((const void *)fn,
+                                hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)lds));
+  fn<<<nblk, PER ? 64 : SH::WT, lds, st>>>(descs, list, arr, m, q, iv);
+  WDY_CHECK_LAUNCH();
+  return WDY_OK;
+}
+
 }  // namespace
 
 // Window shapes and what they cost, in us, measured on the sech^2 disk with
@@ -359,6 +436,14 @@ static const SpanCost kCost[SPAN_NSHAPES] = {
     {{3.80, 6.60}, {0., 0.}, {3.80, 6.60}, 1.0, 1. / 256., 5.5, {0.025, 0.055}},
     {{6.00, 0.}, {0., 0.}, {6.00, 0.}, 1.0, 1. / 256., 5.5, {0.025, 0.}}};
 
+// Halo ranks taken over ranks the reach is expected to cross; that follows
+// the smallest halo width the windows report.
+constexpr double SPAN_MARGIN = 1.15;
+// (a batch's plan stays for many intervals)
+constexpr double SPAN_MANY_MARGIN = 1.3;
+constexpr int SPAN_KBIN = 64;  // steps per launch of the binned shapes (their
+                               // bins are those of its start)
+
 const SpanShape &span_shape(int i) { return kShapes[i]; }
 
 int span_launch(hipStream_t st, int shape, bool eq, const SpanArgs &a) {
@@ -385,6 +470,113 @@ int span_launch(hipStream_t st, int shape, bool eq, const SpanArgs &a) {
   if (!eq) return fail(WDY_ERUNTIME, "span_launch: shape %d with unequal masses", shape);
   return a.ext.kind ? launch_block_one<SH, true, true>(st, a)
                     : launch_block_one<SH, true, false>(st, a);
+}
+
+template <int PER, class SH>
+static int launch_many_both(hipStream_t st, const BatchDesc *descs, const uint2 *list,
+                            u32 neq, u32 nun, const BatchArrays &arr, const SpanMany &m,
+                            u32 q, u32 iv) {
+  if (int rc = launch_many<PER, SH, true>(st, descs, list, neq, arr, m, q, iv)) return rc;
+  return launch_many<PER, SH, false>(st, descs, list + neq, nun, arr, m, q, iv);
+}
+
+int span_many_launch(hipStream_t st, int shape, const BatchDesc *descs,
+                     const uint2 *list, u32 neq, u32 nun, const BatchArrays &arr,
+                     const SpanMany &m, u32 q, u32 iv) {
+  auto go = [&](auto fn) { return fn(st, descs, list, neq, nun, arr, m, q, iv); };
+  switch (shape) {
+    case 0: return go(launch_many_both<2, RankShape<256, 1>>);
+    case 1: return go(launch_many_both<4, RankShape<256, 1>>);
+    case 3: return go(launch_many_both<0, RankShape<256, 2>>);
+    case 5: return go(launch_many_both<0, RankShape<512, 2>>);
+    case 7: return go(launch_many_both<0, RankShape<512, 4>>);
+    case 8: return go(launch_many_both<0, RankShape<1024, 4>>);
+    default: return fail(WDY_ERUNTIME, "span_many_launch: shape %d", shape);
+  }
+}
+
+// Ranks that a distance takes where sheets are densest; width[k]: the smallest
+// width of 2^(k + 2) ranks (1e308: fewer sheets than that).
+static double ranks_of(const double *width, double dx) {
+  double w0 = 0.0, r0 = 0.0;
+  for (u32 k = 0; k < SPAN_NW; ++k) {
+    const double w = width[k], r = (double)(4u << k);
+    if (!(w < 1e300)) break;
+    if (w >= dx) return r0 + (r - r0) * (dx - w0) / (w - w0);
+    w0 = w;
+    r0 = r;
+  }
+  return w0 > 0.0 ? r0 * (dx / w0) : 1e12;
+}
+
+// One shape and K serve the whole batch.  Simulations too dense for them stay
+// with the workgroup-per-simulation kernel, whose time is that of the largest:
+// measured, us per step, 100 sheets 3.4, 1000 4.9, 2000 6.9, above 2048 (a
+// sliding pass) 5.2 ns per sheet.
+void span_many_plan(std::vector<BatchDesc> &d, const double *info,
+                    const std::vector<double> &reach, double h, int nleap, int *shape) {
+  const double ah = std::fabs(h);
+  u32 maxn = 0;
+  bool un = false;
+  for (const BatchDesc &q : d) {
+    maxn = std::max(maxn, q.n);
+    un = un || !(q.flags & 1u);
+  }
+  auto other = [&](u32 n) {
+    return nleap * (n <= 2048 ? 3.4 + 1.7e-3 * n : 5.2e-3 * n);
+  };
+  double best = other(maxn);
+  int bs = -1, bk = 0;
+  auto halo = [&](size_t i, int K) {
+    const double *w = info + i * SPAN_INFO;
+    const double dx = 1.04 * (w[SPAN_NW] + ah * K * std::fabs(d[i].totmass)) * ah * (K + 0.5);
+    return std::ceil(SPAN_MANY_MARGIN * reach[i] * ranks_of(w, dx)) + 2.0;
+  };
+  double disp = 0.0;  // ranks of displacement per step
+  for (size_t i = 0; i < d.size(); ++i) {
+    const double *w = info + i * SPAN_INFO;
+    disp = std::max(disp, ranks_of(w, ah * (w[SPAN_NW] + ah * std::fabs(d[i].totmass))));
+  }
+  if (h != 0.0)
+    for (int L = 1; L <= nleap; L = L < 8 ? L + 1 : L + L / 4) {
+      const int K = (nleap + L - 1) / L;
+      const int launches = (nleap + K - 1) / K;
+      for (int s : {0, 1, 3, 5, 7, 8}) {
+        if (kShapes[s].bin && K > SPAN_KBIN) continue;
+        const double cap = kShapes[s].cap;
+        const SpanCost &k = kCost[s];
+        double W = 0.0, rest = 0.0;
+        for (size_t i = 0; i < d.size(); ++i) {
+          const double H = d[i].n <= cap ? 0.0 : halo(i, K);
+          if (2.0 * H + cap / 16 <= cap) W += std::ceil(d[i].n / (cap - 2.0 * H));
+          else rest = std::max(rest, other(d[i].n));
+        }
+        double step = k.lat[un] + k.latd[un] * std::sqrt(disp);
+        if (W > 256.0)
+          step = std::max(step * k.two, (kShapes[s].bin ? 1.0 : 1.0 + std::sqrt(disp)) * k.sat[un] * std::ceil(W * k.per) / (256.0 * k.per));
+        const double cost = launches * (k.base + k.basew[un] * W + K * step) + rest + 5.0;
+        if (cost < best) {
+          best = cost;
+          bs = s;
+          bk = K;
+        }
+      }
+    }
+  *shape = bs;
+  u32 vslot = 0;
+  for (size_t i = 0; i < d.size(); ++i) {
+    BatchDesc &q = d[i];
+    q.L = q.K = q.T = q.H = q.nwin = q.vslot = 0;
+    if (bs < 0) continue;
+    const double cap = kShapes[bs].cap, H = q.n <= cap ? 0.0 : halo(i, bk);
+    if (!(2.0 * H + cap / 16 <= cap)) continue;
+    q.H = (u32)H;
+    q.T = q.n <= cap ? q.n : (u32)cap - 2 * q.H;
+    q.nwin = (q.n + q.T - 1) / q.T;
+    q.K = (u32)bk;
+    q.L = (u32)((nleap + bk - 1) / bk);
+    if (q.nwin > 1) q.vslot = vslot++;
+  }
 }
 
 // ---- a simulation's intervals --------------------------------------------------
@@ -415,7 +607,6 @@ __global__ __launch_bounds__(256) void k_span_absmax(u32 n, const double *__rest
 // The smallest widths of 2^(k + 2) consecutive ranks, k < SPAN_NW: how far
 // apart the sheets are where they are densest, at every halo size.  One
 // thread per `stride` ranks.
-constexpr u32 SPAN_NW = 10;
 __global__ __launch_bounds__(256) void k_span_widths(u32 n, u32 stride,
                                                      const u64 *__restrict__ key,
                                                      u64 *__restrict__ out) {
@@ -500,8 +691,7 @@ struct SpanCtx {
   u64 *vmax = nullptr;    // [3][SPAN_SLOTS], then stat [2][SPAN_SLOTS]
   u32 *stat = nullptr;
   u64 *h_buf = nullptr;   // pinned: [16] words of the widths, then
-  u32 *h_stat = nullptr;  // [SPAN_SLOTS]
-  hipEvent_t ev = nullptr;
+  u32 *h_stat = nullptr;  // [SPAN_SLOTS], then the fail word
   double fscale = 1.0, finv = 1.0;
   double width[16] = {};  // smallest width of 2^(k + 2) ranks at the start
   double vmax_h = 0.0;    // largest |v| at the start
@@ -517,12 +707,6 @@ struct SpanCtx {
   u32 p_nwin = 0;
   double p_ratio = 0.0;  // halo ranks taken over ranks expected
 };
-
-// Halo ranks taken over ranks the reach is expected to cross; that follows
-// the smallest halo width the windows report.
-constexpr double SPAN_MARGIN = 1.15;
-constexpr int SPAN_KBIN = 64;  // steps per launch of the binned shapes (their
-                               // bins are those of its start)
 
 // |acceleration| of a sheet at x <= a0 + a1 * |x|
 static void span_amax(const wdy_sim *s, double *a0, double *a1) {
@@ -542,16 +726,7 @@ static double span_reach_x(const wdy_sim *s, double drift, double kicks) {
   return 1.04 * (s->span->vmax_h + kicks * a0) * drift;
 }
 static double span_ranks(const wdy_sim *s, double dx) {
-  const SpanCtx &c = *s->span;
-  double w0 = 0.0, r0 = 0.0;
-  for (u32 k = 0; k < SPAN_NW; ++k) {
-    const double w = c.width[k], r = (double)(4u << k);
-    if (!(w < 1e300)) break;  // fewer sheets than that
-    if (w >= dx) return r0 + (r - r0) * (dx - w0) / (w - w0);
-    w0 = w;
-    r0 = r;
-  }
-  return w0 > 0.0 ? r0 * (dx / w0) : 1e12;
+  return ranks_of(s->span->width, dx);
 }
 
 // The windows of a launch that drifts `drift` time units in all and kicks for
@@ -645,9 +820,8 @@ int span_create(wdy_sim *s, double vmax) {
   WDY_HIP(hipMalloc(&c->vmax, (3 * SPAN_SLOTS + 16) * 8 + 2 * SPAN_SLOTS * 4));
   u64 *const width = c->vmax + 3 * SPAN_SLOTS;
   c->stat = (u32 *)(width + 16);
-  WDY_HIP(hipHostMalloc((void **)&c->h_buf, 16 * 8 + SPAN_SLOTS * 4, hipHostMallocDefault));
+  WDY_HIP(hipHostMalloc((void **)&c->h_buf, 16 * 8 + (SPAN_SLOTS + 1) * 4, hipHostMallocDefault));
   c->h_stat = (u32 *)(c->h_buf + 16);
-  WDY_HIP(hipEventCreateWithFlags(&c->ev, hipEventDisableTiming));
   if (!s->equal_mass)
     for (int b = 0; b < 3; ++b) WDY_HIP(hipMalloc(&c->cf[b], N * 8));
   u64 bits;
@@ -679,7 +853,6 @@ void span_free(wdy_sim *s) {
     if (p) (void)hipFree(p);
   if (c->vmax) (void)hipFree(c->vmax);
   if (c->h_buf) (void)hipHostFree(c->h_buf);
-  if (c->ev) (void)hipEventDestroy(c->ev);
   delete c;
   s->span = nullptr;
 }
@@ -730,7 +903,8 @@ static int span_resort(wdy_sim *s) {
   return span_vmax(s);
 }
 
-// Enqueues one output interval; checked by span_settle.  It starts from the
+// Enqueues one output interval, which span_settle checks once the caller has
+// recorded ev1 behind it.  It starts from the
 // current set and writes only the two others, so a failure found later can
 // go back to its start.
 int span_interval(wdy_sim *s, double h, int nleap, const SpanPlan &p) {
@@ -749,8 +923,12 @@ int span_interval(wdy_sim *s, double h, int nleap, const SpanPlan &p) {
   a.finv = c.finv;
   a.ext = s->ext;
   span_amax(s, &a.amax0, &a.amax1);
+  // (the interval before has been settled: nothing writes there now)
+  for (u32 q = 0; q < SPAN_SLOTS; ++q) c.h_stat[q] = SPAN_STAT_INIT;
+  c.h_stat[SPAN_SLOTS] = 0;
   a.stat_host = c.h_stat;
-  c.h_stat[0] = SPAN_STAT_INIT;
+  a.fail = c.h_stat + SPAN_SLOTS;
+  a.fail_value = 1;
   a.stat = c.stat + SPAN_SLOTS * (c.iv & 1u);
   a.stat_clr = c.stat + SPAN_SLOTS * ((c.iv + 1u) & 1u);
   double t = s->t0;
@@ -795,10 +973,6 @@ int span_interval(wdy_sim *s, double h, int nleap, const SpanPlan &p) {
     done += K;
     in = out;
   }
-  if (c.p_nwin > 1)
-    WDY_HIP(hipMemcpyAsync(c.h_stat, a.stat, SPAN_SLOTS * 4, hipMemcpyDeviceToHost,
-                           s->stream));
-  WDY_HIP(hipEventRecord(c.ev, s->stream));
   ++c.iv;
   c.pending = true;
   c.p_start = start;
@@ -817,12 +991,11 @@ int span_settle(wdy_sim *s, bool *failed, double *h, int *nleap) {
   SpanCtx *cp = s->span;
   if (!cp || !cp->pending) return WDY_OK;
   SpanCtx &c = *cp;
-  WDY_HIP(hipEventSynchronize(c.ev));
+  WDY_HIP(hipEventSynchronize(s->ev1));
   c.pending = false;
-  u32 st = c.h_stat[0];
-  if (c.p_nwin > 1)
-    for (u32 q = 1; q < SPAN_SLOTS; ++q) st = std::min(st, c.h_stat[q]);
-  if (st != 0) {
+  u32 st = SPAN_STAT_INIT;
+  for (u32 q = 0; q < SPAN_SLOTS; ++q) st = std::min(st, c.h_stat[q]);
+  if (c.h_stat[SPAN_SLOTS] == 0) {
     c.fails = 0;
     if (!s->small_class) s->warm_steps += c.p_nleap;
     if (c.p_nwin > 1 && st < SPAN_STAT_INIT) {
