@@ -69,7 +69,7 @@ def test_windows(gpu_lib, n, mass):
     x, v, m = disk(n, mass)
     for dt, nleap in ((0.0005, 1), (0.0023, 23), (0.02, 13)):
         st, _ = check(x, v, m, dt, nleap, 2, omega=0.1, exact=mass == 'equal')
-        if n > 6144 and nleap > 1:
+        if n > 6144:
             assert st == (2 * nleap, 0, 0)  # no radix interval, nothing redone
 
 
@@ -137,3 +137,35 @@ def test_overflow_as_on_the_other_paths(gpu_lib, n):
     assert numpy.isnan(out[0][0]).any()
     for a, b in zip(*out):
         assert numpy.array_equal(a, b, equal_nan=True)
+
+
+@pytest.mark.parametrize('n', [3, 512, 513, 4097, 30000, 65537])
+def test_outputs_of_pipelined_reads(gpu_lib, n):
+    """read_and_advance: pinned and pageable arrays, one of the two left out,
+    reads and an energy in between, a collapse that is redone."""
+    x, v, m = disk(n, 'equal')
+    if n == 30000:
+        v = numpy.where(numpy.abs(x) < 0.05, -10. * x, 0.)
+    st = O.ApproxState(x, v, m, 0.05, 10, omega=0.1)
+    sim = wendy_amd.Sim(x, v, m, numpy.sum(m), 0.1 ** 2.)
+    bufs = [(wendy_amd._lib.pinned_empty(n), wendy_amd._lib.pinned_empty(n)),
+            (numpy.empty(n), numpy.empty(n))]
+    gx, gv = numpy.empty(n), numpy.empty(n)
+    try:
+        sim.advance(0.005, 10)
+        for k in range(8):
+            xo, vo = bufs[(k // 2) % 2]
+            if k == 3:
+                sim.energy()
+            if k == 5:
+                sim.read(gx, gv)
+            sim.read_and_advance(xo, vo if k != 6 else None, 0.005, 10)
+            wx, wv = st.onestep()[:2]
+            assert bits_equal(xo, wx), k
+            assert k == 6 or bits_equal(vo, wv), k
+            assert k != 5 or (bits_equal(gx, wx) and bits_equal(gv, wv))
+        sim.read(gx, gv)
+        wx, wv = st.onestep()[:2]
+        assert bits_equal(gx, wx) and bits_equal(gv, wv)
+    finally:
+        sim.close()

@@ -132,6 +132,8 @@ static void free_sim(wdy_sim *s) {
   if (s->red) (void)hipFree(s->red);
   if (s->out_x) (void)hipFree(s->out_x);
   if (s->out_v) (void)hipFree(s->out_v);
+  if (s->out_x2) (void)hipFree(s->out_x2);
+  if (s->out_v2) (void)hipFree(s->out_v2);
   if (s->ext_tab) (void)hipFree(s->ext_tab);
   radix_free(&s->radix);
   if (s->ev0) (void)hipEventDestroy(s->ev0);
@@ -456,16 +458,18 @@ static int settle(wdy_sim *s) {
     bool failed = false;
     double h = 0.0;
     int nleap = 0;
-    if (int rc = span_settle(s, &failed, &h, &nleap)) return rc;
+    double *xo = nullptr, *vo = nullptr;
+    if (int rc = span_settle(s, &failed, &h, &nleap, &xo, &vo)) return rc;
     while (failed) {  // again with wider halos, or on the other paths
       s->redos += 1;
       SpanPlan p;
       if (span_plan(s, h, nleap, &p)) {
-        if (int rc = span_interval(s, h, nleap, p)) return rc;
+        if (int rc = span_interval(s, h, nleap, p, xo, vo)) return rc;
         WDY_HIP(hipEventRecord(s->ev1, s->stream));
-        if (int rc = span_settle(s, &failed, &h, &nleap)) return rc;
+        if (int rc = span_settle(s, &failed, &h, &nleap, &xo, &vo)) return rc;
       } else {
         failed = false;
+        s->staged = -1;
         if (int rc = cold_interval(s, h, nleap, nullptr, nullptr)) return rc;
         WDY_HIP(hipEventRecord(s->ev1, s->stream));
         if (int rc = radix_check_enqueue(s)) return rc;
@@ -484,10 +488,14 @@ static int settle(wdy_sim *s) {
   return WDY_OK;
 }
 
+// outputs: have them written by the interval's last launch where its path can
 static int advance_impl(wdy_sim *s, double h, int nleap, double *acc_last,
-                        double *cum_last) {
+                        double *cum_last, bool outputs = false) {
   WDY_HIP(hipSetDevice(s->device));
   if (int rc = settle(s)) return rc;
+  s->staged = -1;
+  double *const xo = !outputs ? nullptr : s->stage_next ? s->out_x2 : s->out_x;
+  double *const vo = !outputs ? nullptr : s->stage_next ? s->out_v2 : s->out_v;
   warm_gang_release(s);  // ev0/ev1 bracket this interval
   WDY_HIP(hipEventRecord(s->ev0, s->stream));
   SpanPlan plan;
@@ -495,13 +503,15 @@ static int advance_impl(wdy_sim *s, double h, int nleap, double *acc_last,
     if (int rc = advance_host_force(s, h, nleap, acc_last, cum_last)) return rc;
     if (int rc = radix_check_enqueue(s)) return rc;
   } else if (s->small) {
-    int rc = launch_small_advance(s, h, nleap, acc_last, cum_last);
+    int rc = launch_small_advance(s, h, nleap, acc_last, cum_last, xo, vo);
     if (rc) return rc;
+    if (outputs && (u64)s->n <= SMALL_WAVE_MAX) s->staged = s->stage_next;
     if (s->ext.kind)  // the kernel's clock, replayed (wendy/wendy.c:401-408)
       for (int ii = 0; ii < nleap; ++ii) s->t0 = s->t0 + h;
   } else if (!acc_last && !cum_last && span_plan(s, h, nleap, &plan)) {
     const bool resorts = !s->span_sorted;
-    if (int rc = span_interval(s, h, nleap, plan)) return rc;
+    if (int rc = span_interval(s, h, nleap, plan, xo, vo)) return rc;
+    if (outputs) s->staged = s->stage_next;
     if (resorts)
       if (int rc = radix_check_enqueue(s)) return rc;
   } else if (!acc_last && !cum_last && warm_ready_for(s, h)) {
@@ -576,19 +586,55 @@ int wdy_read(wdy_sim *sim, double *x_out, double *v_out, double *seconds_out) {
   WDY_HIP(hipSetDevice(sim->device));
   const size_t N = (size_t)sim->n;
   if (x_out || v_out) {
-    if (int rc = launch_desort(sim, sim->out_x, sim->out_v, nullptr, nullptr,
-                               nullptr))
+    const double *xs = sim->out_x;
+    const double *vs = sim->small ? sim->vel[0] : sim->out_v;
+    if (sim->staged >= 0) {
+      xs = sim->staged ? sim->out_x2 : sim->out_x;
+      vs = sim->staged ? sim->out_v2 : sim->out_v;
+    } else if (int rc = launch_desort(sim, sim->out_x, sim->out_v, nullptr, nullptr,
+                                      nullptr)) {
       return rc;
+    }
     if (x_out)
-      WDY_HIP(hipMemcpyAsync(x_out, sim->out_x, N * 8, hipMemcpyDeviceToHost,
+      WDY_HIP(hipMemcpyAsync(x_out, xs, N * 8, hipMemcpyDeviceToHost,
                              sim->stream));
     if (v_out)
-      WDY_HIP(hipMemcpyAsync(v_out, sim->small ? sim->vel[0] : sim->out_v,
-                             N * 8, hipMemcpyDeviceToHost, sim->stream));
+      WDY_HIP(hipMemcpyAsync(v_out, vs, N * 8, hipMemcpyDeviceToHost, sim->stream));
   }
   WDY_HIP(hipStreamSynchronize(sim->stream));
   if (seconds_out) *seconds_out = interval_ms(sim) * 1e-3;
   return WDY_OK;
+}
+
+// Both output arrays to pinned host memory in one launch.  Up to 2^16 sheets
+// that costs less than two copy calls; above, their larger stores win.  us per
+// output of the generator (two steps each), two copies / this kernel: 10^4
+// sheets 31 / 24, 65536 47 / 44, 131072 65 / 66, 2^19 177 / 189.
+__global__ __launch_bounds__(256) void k_copy_out(u32 n, const double *__restrict__ xs,
+                                                  const double *__restrict__ vs,
+                                                  double *__restrict__ xd,
+                                                  double *__restrict__ vd) {
+  const u32 step = gridDim.x * 256;
+  for (u32 i = blockIdx.x * 256 + threadIdx.x; i < n; i += step) {
+    xd[i] = xs[i];
+    vd[i] = vs[i];
+  }
+}
+
+constexpr size_t COPY_KERNEL_MAX = (size_t)1 << 16;
+
+// Whether a kernel may write these bytes of host memory at their own address.
+static bool device_visible(const void *p, size_t bytes) {
+  const char *const q = (const char *)p;
+  for (const char *b : {q, q + bytes - 1}) {
+    hipPointerAttribute_t at;
+    if (hipPointerGetAttributes(&at, b) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    if (at.type != hipMemoryTypeHost || at.devicePointer != (const void *)b) return false;
+  }
+  return true;
 }
 
 int wdy_read_and_advance(wdy_sim *sim, double *x_out, double *v_out, double h,
@@ -596,29 +642,53 @@ int wdy_read_and_advance(wdy_sim *sim, double *x_out, double *v_out, double h,
   if (int rc = check_settled(sim, "wdy_read_and_advance")) return rc;
   if (nleap < 1) return fail(WDY_EINVAL, "wdy_read_and_advance: nleap=%d < 1", nleap);
   if (!std::isfinite(h)) return fail(WDY_EINVAL, "wdy_read_and_advance: h not finite");
-  if (sim->small) {  // velocities live in the state buffer: read, then advance
-    if (int rc = wdy_read(sim, x_out, v_out, seconds_out)) return rc;
-    return wdy_advance(sim, h, nleap);
-  }
   WDY_HIP(hipSetDevice(sim->device));
   const size_t N = (size_t)sim->n;
+  // From the second interval on, the last launch of an interval has written the
+  // outputs by itself, so the copy starts at once (before, a de-sorting launch
+  // and an event stood in front of it: 10^4 sheets at 10 steps an output took
+  // 60 us against 27, 30000 at one step 63 against 26).
+  const bool stages = sim->small ? (u64)sim->n <= SMALL_WAVE_MAX : sim->span != nullptr;
+  if (stages && !sim->out_v2) {
+    if (!sim->out_x2) WDY_HIP(hipMalloc(&sim->out_x2, N * 8));
+    WDY_HIP(hipMalloc(&sim->out_v2, N * 8));
+  }
+  if (sim->small && sim->staged < 0) {
+    // velocities live in the state buffer: read, then advance
+    if (int rc = wdy_read(sim, x_out, v_out, seconds_out)) return rc;
+    return advance_impl(sim, h, nleap, nullptr, nullptr, stages);
+  }
   WDY_HIP(hipEventSynchronize(sim->ev1));  // the interval being read
   if (seconds_out) *seconds_out = interval_ms(sim) * 1e-3;
   if (x_out || v_out) {
-    if (int rc = launch_desort(sim, sim->out_x, sim->out_v, nullptr, nullptr, nullptr))
-      return rc;
-    WDY_HIP(hipEventRecord(sim->ev_out, sim->stream));
-    WDY_HIP(hipStreamWaitEvent(sim->copy_stream, sim->ev_out, 0));
-    if (x_out)
-      WDY_HIP(hipMemcpyAsync(x_out, sim->out_x, N * 8, hipMemcpyDeviceToHost,
-                             sim->copy_stream));
-    if (v_out)
-      WDY_HIP(hipMemcpyAsync(v_out, sim->out_v, N * 8, hipMemcpyDeviceToHost,
-                             sim->copy_stream));
+    const double *xs = sim->out_x, *vs = sim->out_v;
+    if (sim->staged >= 0) {
+      if (sim->staged) xs = sim->out_x2, vs = sim->out_v2;
+      sim->stage_next = sim->staged ^ 1;
+    } else {
+      if (int rc = launch_desort(sim, sim->out_x, sim->out_v, nullptr, nullptr, nullptr))
+        return rc;
+      WDY_HIP(hipEventRecord(sim->ev_out, sim->stream));
+      WDY_HIP(hipStreamWaitEvent(sim->copy_stream, sim->ev_out, 0));
+      sim->stage_next = 1;
+    }
+    if (N <= COPY_KERNEL_MAX && x_out && v_out && device_visible(x_out, N * 8) &&
+        device_visible(v_out, N * 8)) {
+      const u32 grid = std::min<u32>(((u32)N + 511) / 512, 64u);
+      k_copy_out<<<grid, 256, 0, sim->copy_stream>>>((u32)N, xs, vs, x_out, v_out);
+      WDY_CHECK_LAUNCH();
+    } else {
+      if (x_out)
+        WDY_HIP(hipMemcpyAsync(x_out, xs, N * 8, hipMemcpyDeviceToHost,
+                               sim->copy_stream));
+      if (v_out)
+        WDY_HIP(hipMemcpyAsync(v_out, vs, N * 8, hipMemcpyDeviceToHost,
+                               sim->copy_stream));
+    }
     WDY_HIP(hipEventRecord(sim->ev_copied, sim->copy_stream));
   }
-  // the next interval never touches the output staging buffers
-  const int rc = advance_impl(sim, h, nleap, nullptr, nullptr);
+  // the next interval never touches the staging pair being copied
+  const int rc = advance_impl(sim, h, nleap, nullptr, nullptr, stages);
   if (x_out || v_out) WDY_HIP(hipEventSynchronize(sim->ev_copied));
   return rc;
 }
@@ -752,6 +822,8 @@ int wdy_gang_advance(wdy_gang *gang, wdy_sim *const *sims, int count,
     wdy_sim *s = sims[i];
     if (int rc = settle(s)) return rc;
     if (warm_gang_eligible(s, h[i])) {
+      s->staged = -1;
+      s->span_sorted = false;
       gs.push_back(s);
       gh.push_back(h[i]);
       gn.push_back(nleap[i]);

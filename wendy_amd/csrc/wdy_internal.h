@@ -213,6 +213,12 @@ struct wdy_sim {
   double *red = nullptr;         // reduction partials (energy, momentum)
   double *out_x = nullptr;       // de-sorted output staging
   double *out_v = nullptr;
+  // A program that reads every interval (wdy_read_and_advance) has the last
+  // launch of an interval write its de-sorted outputs too, into the staging
+  // pair the copy of the interval before is not reading: out_x, out_v and these
+  double *out_x2 = nullptr, *out_v2 = nullptr;
+  int stage_next = 0;  // the pair the next interval would write
+  int staged = -1;     // the pair that holds the current state's outputs
   wdy::RadixWork radix;
   wdy::WarmCtx *warm = nullptr;  // null: no warm path, or not set up yet
   bool warm_ok = false;          // the warm path may be set up
@@ -309,8 +315,9 @@ constexpr u64 SMALL_WAVE_MAX = 512;
 // Largest n the multi-step windows are set up for (beyond, a window of 4096
 // sheets is mostly halo at the step sizes in use).
 constexpr u64 SPAN_MAX = 1u << 22;
+// xo, vo (or null): also the de-sorted outputs, for n <= SMALL_WAVE_MAX
 int launch_small_advance(wdy_sim *s, double h, int nleap, double *acc_out,
-                         double *cum_out);
+                         double *cum_out, double *xo = nullptr, double *vo = nullptr);
 int launch_energy(wdy_sim *s, double twopiG, double omega2, double *e_out);
 // warm-start step (wdy_warm.hip)
 int warm_configure(wdy_sim *s, int shape, u32 T, u32 W);
@@ -351,8 +358,10 @@ void span_created(wdy_sim *s);
 void span_free(wdy_sim *s);
 void span_off(wdy_sim *s);
 int span_prefix(wdy_sim *s);
-int span_interval(wdy_sim *s, double h, int nleap, const SpanPlan &p);
-int span_settle(wdy_sim *s, bool *failed, double *h, int *nleap);
+// xo, vo: the de-sorted outputs, or null
+int span_interval(wdy_sim *s, double h, int nleap, const SpanPlan &p, double *xo,
+                  double *vo);
+int span_settle(wdy_sim *s, bool *failed, double *h, int *nleap, double **xo, double **vo);
 // the events bracketing the last interval when it ran in a gang
 bool warm_gang_events(wdy_sim *s, hipEvent_t *start, hipEvent_t *done);
 // the next interval runs outside a gang: drop the settled gang record

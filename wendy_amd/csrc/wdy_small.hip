@@ -172,7 +172,7 @@ __global__ __launch_bounds__(64) void k_small_wave(
     double *__restrict__ vel, const double *__restrict__ mass,
     double *__restrict__ cum, double mq, double totmass, double omega2, double h,
     int nleap, double *__restrict__ acc_out, double *__restrict__ cum_out,
-    ExtForce ext, double t0) {
+    ExtForce ext, double t0, double *__restrict__ xo, double *__restrict__ vo) {
   extern __shared__ u64 smem[];
   __shared__ double s_m[EQ ? 1 : 64 * PER + 8];  // masses in sorted order
   __shared__ double s_id[EQ ? 1 : 64 * PER];     // masses by sheet index
@@ -274,6 +274,11 @@ __global__ __launch_bounds__(64) void k_small_wave(
   if (__builtin_expect(__ballot(over) != 0, 0)) {
     small_interval<EQ, HARM>(n, key_g, id_g, vel, mass, cum, mq, totmass, omega2, h,
                              nleap, acc_out, cum_out, ext, t0, smem, nullptr);
+    __syncthreads();
+    for (u32 i = lane; xo && i < n; i += 64) {
+      xo[id_g[i]] = decode_pos(key_g[i]);
+      vo[i] = vel[i];
+    }
     return;
   }
 #pragma unroll
@@ -282,18 +287,24 @@ __global__ __launch_bounds__(64) void k_small_wave(
       key_g[e0 + q] = encode_pos(s.x[q]);
       id_g[e0 + q] = s.id[q];
       vel[s.id[q]] = s.v[q];
+      if (xo) {
+        xo[s.id[q]] = s.x[q];
+        vo[s.id[q]] = s.v[q];
+      }
       if (acc_out) acc_out[s.id[q]] = a[q];
       if (cum_out) cum_out[e0 + q] = C[q];
     }
 }
 
 template <int PER, bool EXT>
-int launch_wave(wdy_sim *s, double h, int nleap, double *acc, double *cum) {
+int launch_wave(wdy_sim *s, double h, int nleap, double *acc, double *cum, double *xo,
+                double *vo) {
   const bool harm = s->omega2 >= 0.0;
 #define WDY_WAVE(EQ, HARM)                                                    \
   k_small_wave<PER, EQ, HARM, EXT><<<1, 64, (size_t)s->n * 12 + 16, s->stream>>>( \
       (u32)s->n, s->key[0], s->idx[0], s->vel[0], s->mass[0], s->cum,         \
-      s->m_equal, s->totmass, s->omega2, h, nleap, acc, cum, s->ext, s->t0)
+      s->m_equal, s->totmass, s->omega2, h, nleap, acc, cum, s->ext, s->t0,   \
+      xo, vo)
   if (s->equal_mass) {
     if (harm) WDY_WAVE(true, true); else WDY_WAVE(true, false);
   } else {
@@ -305,10 +316,11 @@ int launch_wave(wdy_sim *s, double h, int nleap, double *acc, double *cum) {
 }
 
 template <bool EXT>
-int launch_wave_per(wdy_sim *s, double h, int nleap, double *acc, double *cum) {
-  if (s->n <= 128) return launch_wave<2, EXT>(s, h, nleap, acc, cum);
-  if (s->n <= 256) return launch_wave<4, EXT>(s, h, nleap, acc, cum);
-  return launch_wave<8, EXT>(s, h, nleap, acc, cum);
+int launch_wave_per(wdy_sim *s, double h, int nleap, double *acc, double *cum,
+                    double *xo, double *vo) {
+  if (s->n <= 128) return launch_wave<2, EXT>(s, h, nleap, acc, cum, xo, vo);
+  if (s->n <= 256) return launch_wave<4, EXT>(s, h, nleap, acc, cum, xo, vo);
+  return launch_wave<8, EXT>(s, h, nleap, acc, cum, xo, vo);
 }
 
 }  // namespace
@@ -324,12 +336,13 @@ u32 small_max_n(int device) {
 }
 
 int launch_small_advance(wdy_sim *s, double h, int nleap, double *acc_out,
-                         double *cum_out) {
+                         double *cum_out, double *xo, double *vo) {
   const u32 n = (u32)s->n;
   if (n <= SMALL_WAVE_MAX) {
     if (s->timing) timer_begin(s->timer, s->stream, KC_LEAP);
-    const int rc = s->ext.kind ? launch_wave_per<true>(s, h, nleap, acc_out, cum_out)
-                               : launch_wave_per<false>(s, h, nleap, acc_out, cum_out);
+    const int rc =
+        s->ext.kind ? launch_wave_per<true>(s, h, nleap, acc_out, cum_out, xo, vo)
+                    : launch_wave_per<false>(s, h, nleap, acc_out, cum_out, xo, vo);
     if (s->timing) timer_end(s->timer, s->stream, KC_LEAP);
     return rc;
   }

@@ -28,6 +28,7 @@ struct SpanArgs {
   i32 *iout;
   double *mout;
   u64 *cout;
+  double *xo, *vo;  // de-sorted positions and velocities as well (or null)
   double pre, h, hlast;  // drift before the first force; step; last drift
   double mq, totmass, omega2, fscale, finv;  // omega2: 0 without the term
   double amax0, amax1;  // |acceleration| <= amax0 + amax1 * |x|

@@ -99,6 +99,10 @@ __device__ __forceinline__ void span_store(const SpanArgs &A, Reach &R, u32 r,
       A.mout[r] = m;
       A.cout[r] = c;
     }
+    if (A.xo) {
+      A.xo[id] = x;
+      A.vo[id] = v;
+    }
   }
 }
 
@@ -368,6 +372,7 @@ __global__ __launch_bounds__(PER ? 64 : SH::WT) void k_span_many(
     A.mout = arr.mass[out] + d.off;
     A.cout = M.cf[out] + d.off;
   }
+  A.xo = A.vo = nullptr;
   A.pre = done == 0 ? d.h / 2. : 0.0;
   A.h = d.h;
   A.hlast = done + K == d.nleap ? d.h / 2. : d.h;
@@ -706,6 +711,7 @@ struct SpanCtx {
   double p_h = 0.0, p_t0 = 0.0;
   u32 p_nwin = 0;
   double p_ratio = 0.0;  // halo ranks taken over ranks expected
+  double *p_xo = nullptr, *p_vo = nullptr;
 };
 
 // |acceleration| of a sheet at x <= a0 + a1 * |x|
@@ -763,10 +769,6 @@ static double span_drift(double ah, int done, int K, int nleap) {
 
 bool span_plan(wdy_sim *s, double h, int nleap, SpanPlan *plan) {
   if (!s->span || s->span->off || !(h != 0.0) || !std::isfinite(h)) return false;
-  // A single step per interval: the windows' 14 us against 24 of the one-step
-  // kernel are hidden behind the outputs' copies, which they disturb more
-  // (30000 sheets: 66 us an output against 63)
-  if (nleap == 1 && !s->small_class) return false;
   const u32 n = (u32)s->n;
   const int un = s->equal_mass ? 0 : 1;
   const double ah = std::fabs(h);
@@ -907,7 +909,8 @@ static int span_resort(wdy_sim *s) {
 // recorded ev1 behind it.  It starts from the
 // current set and writes only the two others, so a failure found later can
 // go back to its start.
-int span_interval(wdy_sim *s, double h, int nleap, const SpanPlan &p) {
+int span_interval(wdy_sim *s, double h, int nleap, const SpanPlan &p, double *xo,
+                  double *vo) {
   SpanCtx &c = *s->span;
   if (!s->span_sorted)
     if (int rc = span_resort(s)) return rc;
@@ -958,6 +961,8 @@ int span_interval(wdy_sim *s, double h, int nleap, const SpanPlan &p) {
     a.iout = s->idx[out];
     a.mout = s->mass[out];
     a.cout = c.cf[out];
+    a.xo = done + K == nleap ? xo : nullptr;
+    a.vo = done + K == nleap ? vo : nullptr;
     a.pre = done == 0 ? h / 2. : 0.0;
     a.hlast = done + K == nleap ? h / 2. : h;
     a.t = t;
@@ -979,6 +984,8 @@ int span_interval(wdy_sim *s, double h, int nleap, const SpanPlan &p) {
   c.p_h = h;
   c.p_nleap = nleap;
   c.p_t0 = s->t0;
+  c.p_xo = xo;
+  c.p_vo = vo;
   s->cur = in;
   if (s->ext.kind) s->t0 = t;
   return WDY_OK;
@@ -986,7 +993,8 @@ int span_interval(wdy_sim *s, double h, int nleap, const SpanPlan &p) {
 
 // Waits for and checks the interval in flight; *failed: the state is back at
 // its start and (h, nleap) must be redone, with the halo estimate widened.
-int span_settle(wdy_sim *s, bool *failed, double *h, int *nleap) {
+int span_settle(wdy_sim *s, bool *failed, double *h, int *nleap, double **xo,
+                double **vo) {
   *failed = false;
   SpanCtx *cp = s->span;
   if (!cp || !cp->pending) return WDY_OK;
@@ -1011,6 +1019,8 @@ int span_settle(wdy_sim *s, bool *failed, double *h, int *nleap) {
   *failed = true;
   *h = c.p_h;
   *nleap = c.p_nleap;
+  *xo = c.p_xo;
+  *vo = c.p_vo;
   s->cur = c.p_start;
   s->t0 = c.p_t0;
   s->fail_overflow += 1;
