@@ -12,6 +12,7 @@
 // where C is the exclusive prefix of masses in sorted order
 // (wendy/wendy.c:359-360).  Equal-mass runs use C = rank * m, the exact
 // value of the reference's running sum whenever m is a power of two.
+#include <algorithm>
 #include <climits>
 #include <cmath>
 
@@ -313,39 +314,93 @@ __global__ __launch_bounds__(BLOCK) void k_sum_partials(
   if (threadIdx.x == 0) out[0] = (err && *err) ? __builtin_nan("") : t;
 }
 
-// out[k] = [omega2 * y_k^2 / 2] + twopiG * sum_j m_j |x_j - y_k|
-// (wendy/wendy.py:512-517).  One block per query point.
-__global__ __launch_bounds__(BLOCK) void k_potential(
-    u32 n, const double *__restrict__ x, const double *__restrict__ m,
-    const double *__restrict__ y, double twopiG, double omega2,
+// What is made of the sum S_k = sum_j m_j |x_j - y_k|:
+// * potential (v null): [omega2 * y_k^2 / 2] + twopiG * S_k
+//   (wendy/wendy.py:512-517)
+// * energy of sheet k, at y_k: [m_k omega^2 y_k^2 / 2] + twopiG m_k S_k
+//   + m_k v_k^2 / 2 (wendy/wendy.py:458-466)
+struct PairEnd {
+  const double *v;
+  double twopiG, omega2;
+};
+__device__ __forceinline__ double pair_end(const PairEnd &e, const double *y,
+                                           const double *m, u32 k, double S) {
+  const double yk = y[k];
+  if (!e.v) {
+    const double o = e.omega2 >= 0.0 ? e.omega2 * (yk * yk) / 2.0 : 0.0;
+    return o + e.twopiG * S;
+  }
+  const double mk = m[k], vk = e.v[k];
+  const double o = e.omega2 >= 0.0 ? mk * e.omega2 * (yk * yk) / 2.0 : 0.0;
+  return (o + e.twopiG * mk * S) + mk * (vk * vk) / 2.0;
+}
+
+// S_k for QP points y per block over one stretch of
+// sheets: a thread's sheets are read once for all of its QP points, whose sums
+// it keeps in registers, so the sheets' traffic from L2 (16 B for QP pairs of
+// two f64 instructions) falls behind the arithmetic.  With one point per block
+// the loads were what bound it: 30000 x 30000 pairs 808 us, with QP = 16
+// 105 us (the two instructions alone take 46).  A thread adds up a stretch's
+// n / splits / 256 terms, the rest is a tree, in a fixed order.
+// out: [splits][ny] sums, or, with one stretch, the results made of them.
+template <int QP>
+__global__ __launch_bounds__(BLOCK) void k_pair_sums(
+    u32 n, u32 ny, u32 per, const double *__restrict__ x,
+    const double *__restrict__ m, const double *__restrict__ y, PairEnd end,
     double *__restrict__ out) {
-  __shared__ double s_w[BLOCK / 64];
-  const double yk = y[blockIdx.x];
-  double acc = 0.0;
-  for (u32 j = threadIdx.x; j < n; j += BLOCK) acc = acc + m[j] * fabs(x[j] - yk);
-  const double t = block_sum_f64(acc, s_w);
-  if (threadIdx.x == 0) {
-    const double o = omega2 >= 0.0 ? omega2 * (yk * yk) / 2.0 : 0.0;
-    out[blockIdx.x] = o + twopiG * t;
+  __shared__ double s_w[BLOCK / 64][QP];
+  const u32 k0 = blockIdx.x * QP, t = threadIdx.x, lane = t & 63u;
+  double yk[QP], acc[QP];
+#pragma unroll
+  for (int q = 0; q < QP; ++q) {
+    yk[q] = y[min(k0 + q, ny - 1u)];
+    acc[q] = 0.0;
+  }
+  const u32 lo = blockIdx.y * per, hi = min(n, lo + per);
+#pragma unroll 4
+  for (u32 j = lo + t; j < hi; j += BLOCK) {
+    const double xj = x[j], mj = m[j];
+#pragma unroll
+    for (int q = 0; q < QP; ++q) acc[q] = __builtin_fma(mj, fabs(xj - yk[q]), acc[q]);
+  }
+  // over the lanes: half of the sums go to the other half of the lanes as long
+  // as there are several
+  int o = 32;
+#pragma unroll
+  for (int w = QP / 2; w >= 1; w /= 2, o /= 2) {
+    const bool up = lane & (u32)o;
+#pragma unroll
+    for (int q = 0; q < w; ++q) {
+      const double send = up ? acc[q] : acc[q + w];
+      acc[q] = (up ? acc[q + w] : acc[q]) + __shfl_xor(send, o, 64);
+    }
+  }
+  u32 mine = 0;  // the lane's point: its upper bits, as they were chosen
+#pragma unroll
+  for (int w = QP / 2, b = 32; w >= 1; w /= 2, b /= 2) mine += lane & (u32)b ? (u32)w : 0u;
+  for (; o >= 1; o /= 2) acc[0] = acc[0] + __shfl_xor(acc[0], o, 64);
+  if ((lane & (64u / QP - 1u)) == 0) s_w[t >> 6][mine] = acc[0];
+  __syncthreads();
+  if (t < QP && k0 + t < ny) {
+    double tot = 0.0;
+    for (int w = 0; w < BLOCK / 64; ++w) tot = tot + s_w[w][t];
+    out[(size_t)blockIdx.y * ny + k0 + t] =
+        gridDim.y == 1 ? pair_end(end, y, m, k0 + t, tot) : tot;
   }
 }
 
-// E_i = [m_i omega^2 x_i^2 / 2] + twopiG m_i sum_j m_j |x_i - x_j|
-//       + m_i v_i^2 / 2   (wendy/wendy.py:458-466).  One block per sheet.
-__global__ __launch_bounds__(BLOCK) void k_energy_individual(
-    u32 n, const double *__restrict__ x, const double *__restrict__ v,
-    const double *__restrict__ m, double twopiG, double omega2,
-    double *__restrict__ out) {
-  __shared__ double s_w[BLOCK / 64];
-  const u32 i = blockIdx.x;
-  const double xi = x[i];
-  double acc = 0.0;
-  for (u32 j = threadIdx.x; j < n; j += BLOCK) acc = acc + m[j] * fabs(x[j] - xi);
-  const double t = block_sum_f64(acc, s_w);
-  if (threadIdx.x == 0) {
-    const double o = omega2 >= 0.0 ? m[i] * omega2 * (xi * xi) / 2.0 : 0.0;
-    out[i] = (o + twopiG * m[i] * t) + m[i] * (v[i] * v[i]) / 2.0;
-  }
+// The same from the sums of several stretches.
+__global__ __launch_bounds__(BLOCK) void k_pair_end(u32 ny, u32 splits,
+                                                    const double *__restrict__ sums,
+                                                    const double *__restrict__ m,
+                                                    const double *__restrict__ y,
+                                                    PairEnd end,
+                                                    double *__restrict__ out) {
+  const u32 k = blockIdx.x * BLOCK + threadIdx.x;
+  if (k >= ny) return;
+  double t = 0.0;
+  for (u32 s = 0; s < splits; ++s) t = t + sums[(size_t)s * ny + k];
+  out[k] = pair_end(end, y, m, k, t);
 }
 
 __global__ __launch_bounds__(BLOCK) void k_encode(u32 n,
@@ -635,21 +690,60 @@ int launch_momentum_arrays(int64_t n64, const double *v, const double *m,
   return WDY_OK;
 }
 
+namespace {
+
+// How the pair sums of ny points over n sheets are launched: enough blocks to
+// fill the GPU, stretches no shorter than 4 sheets per thread and at most 128 of
+// them (one thread adds up their sums).  Few points
+// (under 4096) take 4 to a block: their sheets come from L2 anyway, and 16
+// would leave too few blocks.
+struct PairPlan {
+  u32 qp, splits, per;
+};
+PairPlan pair_plan(u32 n, u32 ny) {
+  PairPlan p;
+  p.qp = ny >= 4096 ? 16 : 4;
+  const u32 bx = (ny + p.qp - 1) / p.qp;
+  const u32 most = std::min<u32>(128, std::max<u32>(1, n / (4 * BLOCK)));
+  p.splits = std::min(most, std::max<u32>(1, (1024 + bx - 1) / bx));
+  p.per = (n + p.splits - 1) / p.splits;
+  p.splits = (n + p.per - 1) / p.per;
+  return p;
+}
+
+int launch_pairs(const PairPlan &p, u32 n, u32 ny, const double *x, const double *m,
+                 const double *y, const PairEnd &end, double *sums, double *out) {
+  const dim3 grid((ny + p.qp - 1) / p.qp, p.splits);
+  double *const o = p.splits == 1 ? out : sums;
+  if (p.qp == 16)
+    k_pair_sums<16><<<grid, BLOCK>>>(n, ny, p.per, x, m, y, end, o);
+  else
+    k_pair_sums<4><<<grid, BLOCK>>>(n, ny, p.per, x, m, y, end, o);
+  WDY_CHECK_LAUNCH();
+  if (p.splits > 1) {
+    k_pair_end<<<grid_for(ny), BLOCK>>>(ny, p.splits, sums, m, y, end, out);
+    WDY_CHECK_LAUNCH();
+  }
+  return WDY_OK;
+}
+
+}  // namespace
+
 int launch_potential_arrays(int64_t ny, const double *y, int64_t n64,
                             const double *x, const double *m, double twopiG,
                             double omega2, double *out) {
   const u32 n = (u32)n64;
+  const PairPlan p = pair_plan(n, (u32)ny);
   DevBufs b;
-  double *dy, *dx, *dm, *dout;
-  WDY_HIP(b.alloc(&dy, ny));
-  WDY_HIP(b.alloc(&dx, n));
-  WDY_HIP(b.alloc(&dm, n));
-  WDY_HIP(b.alloc(&dout, ny));
+  double *dx;
+  WDY_HIP(b.alloc(&dx, 2 * (size_t)n + (2 + p.splits) * (size_t)ny));
+  double *const dm = dx + n, *const dy = dm + n, *const dout = dy + ny;
+  double *const sums = dout + ny;
   WDY_HIP(hipMemcpy(dy, y, 8 * (size_t)ny, hipMemcpyHostToDevice));
   WDY_HIP(hipMemcpy(dx, x, 8 * (size_t)n, hipMemcpyHostToDevice));
   WDY_HIP(hipMemcpy(dm, m, 8 * (size_t)n, hipMemcpyHostToDevice));
-  k_potential<<<(unsigned)ny, BLOCK>>>(n, dx, dm, dy, twopiG, omega2, dout);
-  WDY_CHECK_LAUNCH();
+  const PairEnd end{nullptr, twopiG, omega2};
+  if (int rc = launch_pairs(p, n, (u32)ny, dx, dm, dy, end, sums, dout)) return rc;
   WDY_HIP(hipMemcpy(out, dout, 8 * (size_t)ny, hipMemcpyDeviceToHost));
   return WDY_OK;
 }
@@ -658,20 +752,19 @@ int launch_energy_individual_arrays(int64_t n64, const double *x,
                                     const double *v, const double *m,
                                     double twopiG, double omega2, double *out) {
   const u32 n = (u32)n64;
+  const PairPlan p = pair_plan(n, n);
   DevBufs b;
-  double *dx, *dv, *dm, *dout;
-  WDY_HIP(b.alloc(&dx, n));
-  WDY_HIP(b.alloc(&dv, n));
-  WDY_HIP(b.alloc(&dm, n));
-  WDY_HIP(b.alloc(&dout, n));
+  double *dx;
+  WDY_HIP(b.alloc(&dx, (4 + p.splits) * (size_t)n));
+  double *const dv = dx + n, *const dm = dv + n, *const dout = dm + n;
+  double *const sums = dout + n;
   WDY_HIP(hipMemcpy(dx, x, 8 * (size_t)n, hipMemcpyHostToDevice));
   WDY_HIP(hipMemcpy(dv, v, 8 * (size_t)n, hipMemcpyHostToDevice));
   WDY_HIP(hipMemcpy(dm, m, 8 * (size_t)n, hipMemcpyHostToDevice));
-  k_energy_individual<<<n, BLOCK>>>(n, dx, dv, dm, twopiG, omega2, dout);
-  WDY_CHECK_LAUNCH();
+  const PairEnd end{dv, twopiG, omega2};
+  if (int rc = launch_pairs(p, n, n, dx, dm, dx, end, sums, dout)) return rc;
   WDY_HIP(hipMemcpy(out, dout, 8 * (size_t)n, hipMemcpyDeviceToHost));
   return WDY_OK;
 }
 
 }  // namespace wdy
-
