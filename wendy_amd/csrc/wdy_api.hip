@@ -116,30 +116,15 @@ __global__ void k_iota(u32 n, i32 *__restrict__ idx) {
 
 static void free_sim(wdy_sim *s) {
   if (!s) return;
-  for (int b = 0; b < 3; ++b) {
-    if (s->key[b]) (void)hipFree(s->key[b]);
-    if (s->vel[b]) (void)hipFree(s->vel[b]);
-    if (s->idx[b]) (void)hipFree(s->idx[b]);
-    if (s->mass[b]) (void)hipFree(s->mass[b]);
-  }
-  for (int b = 0; b < 2; ++b)
-    if (s->perm[b]) (void)hipFree(s->perm[b]);
   warm_free(s);
   span_free(s);
-  if (s->skey) (void)hipFree(s->skey);
-  if (s->cum) (void)hipFree(s->cum);
-  if (s->tile_sums) (void)hipFree(s->tile_sums);
-  if (s->red) (void)hipFree(s->red);
-  if (s->out_x) (void)hipFree(s->out_x);
-  if (s->out_v) (void)hipFree(s->out_v);
+  if (s->block) (void)hipFree(s->block);
   if (s->out_x2) (void)hipFree(s->out_x2);
-  if (s->out_v2) (void)hipFree(s->out_v2);
   if (s->ext_tab) (void)hipFree(s->ext_tab);
-  radix_free(&s->radix);
   if (s->ev0) (void)hipEventDestroy(s->ev0);
   if (s->ev1) (void)hipEventDestroy(s->ev1);
   if (s->ev_rerr) (void)hipEventDestroy(s->ev_rerr);
-  if (s->h_rerr) (void)hipHostFree(s->h_rerr);
+  if (s->h_block) (void)hipHostFree(s->h_block);
   if (s->ev_out) (void)hipEventDestroy(s->ev_out);
   if (s->ev_copied) (void)hipEventDestroy(s->ev_copied);
   if (s->copy_stream) (void)hipStreamDestroy(s->copy_stream);
@@ -228,13 +213,13 @@ static int create_impl(int64_t n, const double *x_slot, const i32 *id_slot,
                      (!(flags & WDY_FORCE_LARGE) && (u64)n <= slim);
     s->small = s->small_class && !span;
     WDY_HIP(hipStreamCreate(&s->stream));
-    WDY_HIP(hipStreamCreate(&s->copy_stream));
     WDY_HIP(hipEventCreate(&s->ev0));
     WDY_HIP(hipEventCreate(&s->ev1));
     WDY_HIP(hipEventCreateWithFlags(&s->ev_out, hipEventDisableTiming));
     WDY_HIP(hipEventCreateWithFlags(&s->ev_copied, hipEventDisableTiming));
     WDY_HIP(hipEventCreateWithFlags(&s->ev_rerr, hipEventDisableTiming));
-    WDY_HIP(hipHostMalloc((void **)&s->h_rerr, 8, hipHostMallocDefault));
+    WDY_HIP(hipHostMalloc((void **)&s->h_block, 1024, hipHostMallocDefault));
+    s->h_rerr = (u32 *)s->h_block;
     *s->h_rerr = 0;
     s->timer = timer_create();
     if (!s->timer) return fail(WDY_ENOMEM, "wdy_create: timer allocation failed");
@@ -244,24 +229,35 @@ static int create_impl(int64_t n, const double *x_slot, const i32 *id_slot,
     s->totmass = totmass;
     s->omega2 = omega2 < 0.0 ? -1.0 : omega2;
     const size_t N = (size_t)n;
-    for (int b = 0; b < 3; ++b) {
-      if (s->small && b == 2) break;
-      WDY_HIP(hipMalloc(&s->key[b], N * sizeof(u64)));
-      WDY_HIP(hipMalloc(&s->idx[b], N * sizeof(i32)));
-      if (b == 0 || !s->small) {
-        WDY_HIP(hipMalloc(&s->vel[b], N * sizeof(double)));
-        if (!eq) WDY_HIP(hipMalloc(&s->mass[b], N * sizeof(double)));
+    auto arrays = [&](Carve &c) {
+      for (int b = 0; b < 3; ++b) {
+        if (s->small && b == 2) break;
+        c.take(s->key[b], N);
+        c.take(s->idx[b], N);
+        if (b == 0 || !s->small) {
+          c.take(s->vel[b], N);
+          if (!eq) c.take(s->mass[b], N);
+        }
       }
-    }
-    for (int b = 0; b < 2; ++b)
-      WDY_HIP(hipMalloc(&s->perm[b], N * sizeof(u32)));
-    WDY_HIP(hipMalloc(&s->skey, N * sizeof(u64)));
-    WDY_HIP(hipMalloc(&s->cum, N * sizeof(double)));
-    WDY_HIP(hipMalloc(&s->tile_sums, (N / 4096 + 2) * sizeof(double)));
-    WDY_HIP(hipMalloc(&s->red, (N / 256 + 4) * sizeof(double)));
-    WDY_HIP(hipMalloc(&s->out_x, N * sizeof(double)));
-    WDY_HIP(hipMalloc(&s->out_v, N * sizeof(double)));
-    int r = radix_alloc(&s->radix, (u32)n, s->stream);
+      for (int b = 0; b < 2; ++b) c.take(s->perm[b], N);
+      c.take(s->skey, N);
+      c.take(s->cum, N);
+      c.take(s->tile_sums, N / 4096 + 2);
+      c.take(s->red, N / 256 + 4);
+      c.take(s->out_x, N);
+      c.take(s->out_v, N);
+      c.take(s->warm_words, 16);
+      radix_take(&s->radix, (u32)n, c);
+      if (span) span_take(s, c);
+    };
+    if (span && !span_context(s))
+      return fail(WDY_ENOMEM, "span context allocation failed");
+    Carve size, at;
+    arrays(size);
+    WDY_HIP(hipMalloc(&s->block, size.size));
+    at.base = (char *)s->block;
+    arrays(at);
+    int r = radix_init(&s->radix, (u32)n, s->stream);
     if (r) return r;
     // staging: x -> out_x, v -> out_v, m -> cum, sheet ids -> idx[1]
     WDY_HIP(hipMemcpyAsync(s->out_x, x_slot, N * 8, hipMemcpyHostToDevice,
@@ -649,9 +645,10 @@ int wdy_read_and_advance(wdy_sim *sim, double *x_out, double *v_out, double h,
   // and an event stood in front of it: 10^4 sheets at 10 steps an output took
   // 60 us against 27, 30000 at one step 63 against 26).
   const bool stages = sim->small ? (u64)sim->n <= SMALL_WAVE_MAX : sim->span != nullptr;
+  if (!sim->copy_stream) WDY_HIP(hipStreamCreate(&sim->copy_stream));
   if (stages && !sim->out_v2) {
-    if (!sim->out_x2) WDY_HIP(hipMalloc(&sim->out_x2, N * 8));
-    WDY_HIP(hipMalloc(&sim->out_v2, N * 8));
+    WDY_HIP(hipMalloc(&sim->out_x2, 2 * N * 8));
+    sim->out_v2 = sim->out_x2 + N;
   }
   if (sim->small && sim->staged < 0) {
     // velocities live in the state buffer: read, then advance

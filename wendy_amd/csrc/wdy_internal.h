@@ -126,6 +126,21 @@ void timer_begin(Timer *t, hipStream_t s, int kc);
 void timer_end(Timer *t, hipStream_t s, int kc);
 int timer_collect(Timer *t, int kc, double *ms_total, int64_t *count);
 
+// Several device arrays in one allocation: a first pass over the same take()
+// calls (base null) sums up the size, a second one hands out the addresses.
+// (A simulation used to make up to 55 allocations; each free waits for the
+// whole device, 25 ms for all of a simulation's beside busy ones.)
+struct Carve {
+  char *base = nullptr;
+  size_t size = 0;
+  template <class T>
+  void take(T *&p, size_t count) {
+    if (base) p = (T *)(base + size);
+    size += (count * sizeof(T) + 255) & ~(size_t)255;
+  }
+};
+
+
 // --------------------------------------------------------------------------
 // Radix sort of (uint64 key, uint32 payload) pairs: LSD, 8 passes of 8 bits,
 // one all-digit histogram pass plus one onesweep scatter pass per digit.
@@ -154,8 +169,9 @@ u32 radix_tiles(u32 n);
 size_t radix_hist_bytes();
 size_t radix_counter_bytes();
 size_t radix_status_bytes(u32 n);  // look-back words: zero before first use
-// zeroes its counters and look-back words on stream st
-int radix_alloc(RadixWork *w, u32 n, hipStream_t st);
+// the scratch, then: zeroes the counters and look-back words on stream st
+void radix_take(RadixWork *w, u32 n, Carve &c);
+int radix_init(RadixWork *w, u32 n, hipStream_t st);
 // Source slot of sorted position i.  A sort whose look-back wait gave up can
 // leave slots of its payload unwritten (arbitrary values); clamping keeps
 // every access that follows inside the arrays until the host reports the
@@ -167,7 +183,6 @@ __device__ __forceinline__ u32 sorted_slot(const u32 *perm, u32 i, u32 n) {
 // Device word set nonzero when a look-back wait of a sort gave up (its
 // results are then wrong; every kernel still finishes).
 u32 *radix_err_word(RadixWork *w);
-void radix_free(RadixWork *w);
 // Sorts keys[0..n) ascending, stably; keys ping-pong between k0 and k1 and
 // end in k0 (8 passes).  The payload ends in p0: if identity_payload, the
 // first pass generates p = source position and p0's prior contents are
@@ -211,6 +226,9 @@ struct wdy_sim {
   wdy::u64 *skey = nullptr;      // sort ping-pong partner of the key array
   double *tile_sums = nullptr;   // mass-prefix tile partials
   double *red = nullptr;         // reduction partials (energy, momentum)
+  void *block = nullptr;         // the allocation that holds the arrays here
+  char *h_block = nullptr;       // pinned: h_rerr, then 8 bytes for the warm
+                                 // path's error word, from 64 on the windows'
   double *out_x = nullptr;       // de-sorted output staging
   double *out_v = nullptr;
   // A program that reads every interval (wdy_read_and_advance) has the last
@@ -221,6 +239,7 @@ struct wdy_sim {
   int staged = -1;     // the pair that holds the current state's outputs
   wdy::RadixWork radix;
   wdy::WarmCtx *warm = nullptr;  // null: no warm path, or not set up yet
+  wdy::u32 *warm_words = nullptr;  // [16] its error words and tickets
   bool warm_ok = false;          // the warm path may be set up
   int warm_shape0 = 0;           // the tile shape it starts from
   // several steps per launch over windows of sheets (null: not for this
@@ -353,6 +372,10 @@ struct SpanPlan {
 bool span_plan(wdy_sim *s, double h, int nleap, SpanPlan *plan);
 // enqueues the set-up on the current (sorted) set; vmax: the largest |v|.
 // span_created: once that work has finished
+// (its device arrays are part of the simulation's allocation: span_context,
+// then span_take, before it)
+bool span_context(wdy_sim *s);
+void span_take(wdy_sim *s, Carve &c);
 int span_create(wdy_sim *s, double vmax);
 void span_created(wdy_sim *s);
 void span_free(wdy_sim *s);

@@ -266,27 +266,20 @@ size_t radix_status_bytes(u32 n) {
   return (size_t)radix_tiles(n) * RADIX * sizeof(u64);
 }
 
-int radix_alloc(RadixWork *w, u32 n, hipStream_t st) {
+void radix_take(RadixWork *w, u32 n, Carve &c) {
+  c.take(w->hist, PASSES * RADIX);
+  c.take(w->counters, 64);
+  c.take(w->status, (size_t)radix_tiles(n) * RADIX);
+}
+
+int radix_init(RadixWork *w, u32 n, hipStream_t st) {
   w->n = n;
-  w->ntiles = (n + TILE - 1) / TILE;
-  if (w->ntiles == 0) w->ntiles = 1;
-  WDY_HIP(hipMalloc(&w->hist, PASSES * RADIX * sizeof(u32)));
-  WDY_HIP(hipMalloc(&w->counters, 64 * sizeof(u32)));
+  w->ntiles = radix_tiles(n);
   WDY_HIP(hipMemsetAsync(w->counters, 0, 64 * sizeof(u32), st));
-  WDY_HIP(hipMalloc(&w->status, (size_t)w->ntiles * RADIX * sizeof(u64)));
   WDY_HIP(hipMemsetAsync(w->status, 0, (size_t)w->ntiles * RADIX * sizeof(u64),
                          st));
   w->epoch = 1;
   return WDY_OK;
-}
-
-void radix_free(RadixWork *w) {
-  if (w->hist) (void)hipFree(w->hist);
-  if (w->counters) (void)hipFree(w->counters);
-  if (w->status) (void)hipFree(w->status);
-  w->hist = nullptr;
-  w->counters = nullptr;
-  w->status = nullptr;
 }
 
 int radix_sort_pairs(RadixWork *w, hipStream_t s, Timer *tm, u64 *k0, u64 *k1,

@@ -809,23 +809,30 @@ bool span_plan(wdy_sim *s, double h, int nleap, SpanPlan *plan) {
   return 1.15 * best < nleap * (un ? 15.0 + 3.2e-5 * n : 14.0 + 2.0e-5 * n);
 }
 
+bool span_context(wdy_sim *s) {
+  s->span = new (std::nothrow) SpanCtx();
+  return s->span != nullptr;
+}
+
+void span_take(wdy_sim *s, Carve &k) {
+  SpanCtx &c = *s->span;
+  const size_t N = (size_t)s->n;
+  k.take(c.vmax, 3 * SPAN_SLOTS + 16);
+  k.take(c.stat, 2 * SPAN_SLOTS);
+  if (!s->equal_mass)
+    for (int b = 0; b < 3; ++b) k.take(c.cf[b], N);
+}
+
 int span_create(wdy_sim *s, double vmax) {
-  SpanCtx *c = new (std::nothrow) SpanCtx();
-  if (!c) return fail(WDY_ENOMEM, "span context allocation failed");
-  s->span = c;
+  SpanCtx *c = s->span;
   c->vmax_h = vmax;
   int e = 0;  // the fixed-point scale of the other paths: 2^k * totmass <= 2^62
   (void)frexp(s->totmass > 0.0 ? s->totmass : 1.0, &e);
   c->fscale = ldexp(1.0, 62 - e);
   c->finv = ldexp(1.0, e - 62);
-  const size_t N = (size_t)s->n;
-  WDY_HIP(hipMalloc(&c->vmax, (3 * SPAN_SLOTS + 16) * 8 + 2 * SPAN_SLOTS * 4));
   u64 *const width = c->vmax + 3 * SPAN_SLOTS;
-  c->stat = (u32 *)(width + 16);
-  WDY_HIP(hipHostMalloc((void **)&c->h_buf, 16 * 8 + (SPAN_SLOTS + 1) * 4, hipHostMallocDefault));
+  c->h_buf = (u64 *)(s->h_block + 64);
   c->h_stat = (u32 *)(c->h_buf + 16);
-  if (!s->equal_mass)
-    for (int b = 0; b < 3; ++b) WDY_HIP(hipMalloc(&c->cf[b], N * 8));
   u64 bits;
   __builtin_memcpy(&bits, &vmax, 8);
   k_span_init<<<1, 256, 0, s->stream>>>(c->vmax, c->stat, c->epoch % 3u, bits, width);
@@ -851,10 +858,6 @@ void span_created(wdy_sim *s) {
 void span_free(wdy_sim *s) {
   SpanCtx *c = s->span;
   if (!c) return;
-  for (u64 *p : c->cf)
-    if (p) (void)hipFree(p);
-  if (c->vmax) (void)hipFree(c->vmax);
-  if (c->h_buf) (void)hipHostFree(c->h_buf);
   delete c;
   s->span = nullptr;
 }

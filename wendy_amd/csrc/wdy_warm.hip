@@ -1235,10 +1235,11 @@ struct WarmCtx {
   int shape = WARM_SHAPE_DEFAULT;
   u32 *ring = nullptr;   // [8] ticket ring, overflow-count ring
   size_t seg_alloc = 0, nb_alloc = 0;  // allocated entries
+  void *block = nullptr;  // holds meta and status
   WarmMeta meta[3];
   u64 *status = nullptr;
-  u32 *err = nullptr;
-  u32 *h_err = nullptr;  // pinned copy of err
+  u32 *err = nullptr;     // in the simulation's allocation, like ring
+  u32 *h_err = nullptr;  // pinned copy of err (in the simulation's h_block)
   // the last warm interval, enqueued but not yet checked: its error word is
   // copied to h_err and ev_err marks the copy's completion; until checked,
   // the interval's start set and metadata (p_start, p_mstart) stay intact
@@ -1264,25 +1265,20 @@ struct WarmCtx {
   double clk_khz = 100000.0;
 };
 
-static void meta_free(WarmMeta &m) {
-  void *ps[] = {m.segcnt, m.segoff, m.boff, m.spl,
-                m.okey, m.ov, m.oid, m.om, m.odst};
-  for (void *p : ps)
-    if (p) (void)hipFree(p);
-  m = WarmMeta();
-}
-
-static int meta_alloc(WarmMeta &m, size_t nseg, size_t nbp1) {
-  WDY_HIP(hipMalloc(&m.segcnt, nseg * 4));
-  WDY_HIP(hipMalloc(&m.segoff, nseg * 4));
-  WDY_HIP(hipMalloc(&m.boff, nbp1 * 4));
-  WDY_HIP(hipMalloc(&m.spl, nbp1 * 8));
-  WDY_HIP(hipMalloc(&m.okey, (size_t)WARM_OVF_CAP * 8));
-  WDY_HIP(hipMalloc(&m.ov, (size_t)WARM_OVF_CAP * 8));
-  WDY_HIP(hipMalloc(&m.oid, (size_t)WARM_OVF_CAP * 4));
-  WDY_HIP(hipMalloc(&m.om, (size_t)WARM_OVF_CAP * 8));
-  WDY_HIP(hipMalloc(&m.odst, (size_t)WARM_OVF_CAP * 4));
-  return WDY_OK;
+// The three metadata sets and the look-back words.
+static void meta_take(WarmCtx &w, size_t nseg, size_t nbp1, Carve &c) {
+  for (WarmMeta &m : w.meta) {
+    c.take(m.segcnt, nseg);
+    c.take(m.segoff, nseg);
+    c.take(m.boff, nbp1);
+    c.take(m.spl, nbp1);
+    c.take(m.okey, WARM_OVF_CAP);
+    c.take(m.ov, WARM_OVF_CAP);
+    c.take(m.oid, WARM_OVF_CAP);
+    c.take(m.om, WARM_OVF_CAP);
+    c.take(m.odst, WARM_OVF_CAP);
+  }
+  c.take(w.status, nbp1 * 5);
 }
 
 void warm_free(wdy_sim *s) {
@@ -1305,11 +1301,7 @@ void warm_free(wdy_sim *s) {
     }
     (void)hipFree(w->prof);
   }
-  for (auto &m : w->meta) meta_free(m);
-  if (w->status) (void)hipFree(w->status);
-  if (w->err) (void)hipFree(w->err);
-  if (w->ring) (void)hipFree(w->ring);
-  if (w->h_err) (void)hipHostFree(w->h_err);
+  if (w->block) (void)hipFree(w->block);
   if (w->ev_err) (void)hipEventDestroy(w->ev_err);
   delete w;
   s->warm = nullptr;
@@ -1321,11 +1313,10 @@ int warm_configure(wdy_sim *s, int shape, u32 T, u32 W) {
   if (!s->warm) {
     s->warm = new (std::nothrow) WarmCtx();
     if (!s->warm) return fail(WDY_ENOMEM, "warm context allocation failed");
-    WDY_HIP(hipMalloc(&s->warm->err, 8));
-    WDY_HIP(hipMemsetAsync(s->warm->err, 0, 8, s->stream));
-    WDY_HIP(hipMalloc(&s->warm->ring, 32));
-    WDY_HIP(hipMemsetAsync(s->warm->ring, 0, 32, s->stream));
-    WDY_HIP(hipHostMalloc((void **)&s->warm->h_err, 8, hipHostMallocDefault));
+    s->warm->err = s->warm_words;
+    WDY_HIP(hipMemsetAsync(s->warm->err, 0, 64, s->stream));
+    s->warm->ring = s->warm->err + 8;
+    s->warm->h_err = (u32 *)(s->h_block + 8);
     WDY_HIP(hipEventCreateWithFlags(&s->warm->ev_err, hipEventDisableTiming));
     // fixed-point scale: 2^k * totmass <= 2^62
     int e = 0;
@@ -1348,12 +1339,15 @@ int warm_configure(wdy_sim *s, int shape, u32 T, u32 W) {
   w.nb = (n + T - 1) / T;
   const size_t nseg = (size_t)w.nb * (w.S + 1), nbp1 = (size_t)w.nb + 1;
   if (nseg > w.seg_alloc || nbp1 > w.nb_alloc) {
-    for (auto &m : w.meta) meta_free(m);
-    if (w.status) (void)hipFree(w.status);
-    w.status = nullptr;
-    for (auto &m : w.meta)
-      if (int rc = meta_alloc(m, nseg, nbp1)) return rc;
-    WDY_HIP(hipMalloc(&w.status, nbp1 * 5 * 8));
+    w.ready = false;
+    if (w.block) (void)hipFree(w.block);
+    w.block = nullptr;
+    w.seg_alloc = w.nb_alloc = 0;
+    Carve size, at;
+    meta_take(w, nseg, nbp1, size);
+    WDY_HIP(hipMalloc(&w.block, size.size));
+    at.base = (char *)w.block;
+    meta_take(w, nseg, nbp1, at);
     WDY_HIP(hipMemsetAsync(w.status, 0, nbp1 * 5 * 8, s->stream));
     w.seg_alloc = nseg;
     w.nb_alloc = nbp1;
