@@ -610,21 +610,36 @@ __global__ __launch_bounds__(256) void k_span_absmax(u32 n, const double *__rest
 }
 
 // The smallest widths of 2^(k + 2) consecutive ranks, k < SPAN_NW: how far
-// apart the sheets are where they are densest, at every halo size.  One
-// thread per `stride` ranks.
-__global__ __launch_bounds__(256) void k_span_widths(u32 n, u32 stride,
+// apart the sheets are where they are densest, at every halo size.  `starts`
+// windows, `stride` ranks apart.  A few blocks, each with one atomic per width:
+// with one per wave and width they took 128 us at 10^5 sheets.
+__global__ __launch_bounds__(256) void k_span_widths(u32 n, u32 starts, u32 stride,
                                                      const u64 *__restrict__ key,
                                                      u64 *__restrict__ out) {
-  const u64 i = (u64)(blockIdx.x * 256 + threadIdx.x) * stride;
-  const double x0 = i < n ? decode_pos(key[i]) : 0.0;
+  __shared__ u64 s_w[4][SPAN_NW];
+  u64 w[SPAN_NW];
+#pragma unroll
+  for (u32 k = 0; k < SPAN_NW; ++k) w[k] = ~0ull;
+  for (u32 q = blockIdx.x * 256 + threadIdx.x; q < starts; q += gridDim.x * 256) {
+    const u32 i = q * stride;
+    const double x0 = decode_pos(key[i]);
+#pragma unroll
+    for (u32 k = 0; k < SPAN_NW; ++k)
+      if (i + (4u << k) < n) {
+        const u64 d = (u64)__double_as_longlong(decode_pos(key[i + (4u << k)]) - x0);
+        w[k] = d < w[k] ? d : w[k];
+      }
+  }
 #pragma unroll
   for (u32 k = 0; k < SPAN_NW; ++k) {
-    u64 w = ~0ull;
-    if (i + (4u << k) < n)
-      w = (u64)__double_as_longlong(decode_pos(key[i + (4u << k)]) - x0);
-    w = wave_min(w);
-    if ((threadIdx.x & 63u) == 0 && w < out[k])
-      atomicMin((unsigned long long *)out + k, (unsigned long long)w);
+    const u64 m = wave_min(w[k]);
+    if ((threadIdx.x & 63u) == 0) s_w[threadIdx.x >> 6][k] = m;
+  }
+  __syncthreads();
+  if (threadIdx.x < SPAN_NW) {
+    u64 m = s_w[0][threadIdx.x];
+    for (int q = 1; q < 4; ++q) m = s_w[q][threadIdx.x] < m ? s_w[q][threadIdx.x] : m;
+    if (m < out[threadIdx.x]) atomicMin((unsigned long long *)out + threadIdx.x, m);
   }
 }
 
@@ -839,8 +854,8 @@ int span_create(wdy_sim *s, double vmax) {
   // (2^18 starting ranks are enough for a density)
   const u32 n = (u32)s->n, stride = (n + (1u << 18) - 1) >> 18;
   const u32 starts = (n + stride - 1) / stride;
-  k_span_widths<<<(starts + 255) / 256, 256, 0, s->stream>>>(n, stride, s->key[s->cur],
-                                                             width);
+  k_span_widths<<<std::min<u32>((starts + 255) / 256, 128), 256, 0, s->stream>>>(
+      n, starts, stride, s->key[s->cur], width);
   WDY_CHECK_LAUNCH();
   WDY_HIP(hipMemcpyAsync(c->h_buf, width, 16 * 8, hipMemcpyDeviceToHost, s->stream));
   return span_prefix(s);
