@@ -602,10 +602,12 @@ int wdy_read(wdy_sim *sim, double *x_out, double *v_out, double *seconds_out) {
   return WDY_OK;
 }
 
-// Both output arrays to pinned host memory in one launch.  Up to 2^16 sheets
-// that costs less than two copy calls; above, their larger stores win.  us per
-// output of the generator (two steps each), two copies / this kernel: 10^4
-// sheets 31 / 24, 65536 47 / 44, 131072 65 / 66, 2^19 177 / 189.
+// Both output arrays to pinned host memory in one launch, where the copy is what
+// an output waits for: 2^14 sheets or fewer, and up to 2^16 with one or two
+// steps an output.  Beside a longer interval the two copy calls disturb it less
+// and are hidden behind it.  us per output of the generator, two copies / this
+// kernel: 10^4 sheets at 2 steps 31 / 24, at 10 steps 33 / 34; 30000 at 1 step
+// 36 / 32, at 20 steps 55 / 59; 65536 at 2 steps 47 / 44, at 20 steps 69 / 83.
 __global__ __launch_bounds__(256) void k_copy_out(u32 n, const double *__restrict__ xs,
                                                   const double *__restrict__ vs,
                                                   double *__restrict__ xd,
@@ -617,7 +619,9 @@ __global__ __launch_bounds__(256) void k_copy_out(u32 n, const double *__restric
   }
 }
 
-constexpr size_t COPY_KERNEL_MAX = (size_t)1 << 16;
+static bool copy_kernel(size_t n, int nleap) {
+  return n <= (size_t)1 << 14 || (n <= (size_t)1 << 16 && nleap <= 2);
+}
 
 // Whether a kernel may write these bytes of host memory at their own address.
 static bool device_visible(const void *p, size_t bytes) {
@@ -669,7 +673,7 @@ int wdy_read_and_advance(wdy_sim *sim, double *x_out, double *v_out, double h,
       WDY_HIP(hipStreamWaitEvent(sim->copy_stream, sim->ev_out, 0));
       sim->stage_next = 1;
     }
-    if (N <= COPY_KERNEL_MAX && x_out && v_out && device_visible(x_out, N * 8) &&
+    if (copy_kernel(N, nleap) && x_out && v_out && device_visible(x_out, N * 8) &&
         device_visible(v_out, N * 8)) {
       const u32 grid = std::min<u32>(((u32)N + 511) / 512, 64u);
       k_copy_out<<<grid, 256, 0, sim->copy_stream>>>((u32)N, xs, vs, x_out, v_out);
