@@ -161,11 +161,10 @@ __global__ __launch_bounds__(1024) void k_small_advance(
 // within the interval.  A step is a chain of dependent instructions (force,
 // kick, drift, the test of the order), so what bounds it is their latency:
 // measured, us per step, before (k_small_advance) -> now: 3 sheets 0.77 ->
-// 0.11, 101 sheets with tracers 4.4 -> 0.35, 512 sheets that move ~2 ranks a
-// step 2.2 -> 1.0 with equal masses.  The rounds of the sort grow with the
+// 0.058, 101 sheets with tracers 4.4 -> 0.22, 512 sheets that move ~2 ranks a
+// step 2.2 -> 0.9 with equal masses.  The rounds of the sort grow with the
 // displacement as before, at about half the time each.
-// The unequal masses' prefix stays the reference's sequential sum, bit for
-// bit, but is only summed again from the lowest rank whose mass changed.
+// The unequal masses' prefix stays the reference's sequential sum, bit for bit.
 template <int PER, bool EQ, bool HARM, bool EXT>
 __global__ __launch_bounds__(64) void k_small_wave(
     u32 n, u64 *__restrict__ key_g, i32 *__restrict__ id_g,
@@ -178,7 +177,7 @@ __global__ __launch_bounds__(64) void k_small_wave(
   __shared__ double s_id[EQ ? 1 : 64 * PER];     // masses by sheet index
   const u32 lane = threadIdx.x & 63u, e0 = lane * PER;
   WaveSheets<PER, false> s;
-  double m[EQ ? 1 : PER], C[PER], g[PER], a[PER];
+  double m[PER], C[PER], g[PER], a[PER];
   const double hh = h / 2.;
 #pragma unroll
   for (int q = 0; q < PER; ++q) {
@@ -187,6 +186,7 @@ __global__ __launch_bounds__(64) void k_small_wave(
     s.id[q] = 0;
     a[q] = 0.0;
     C[q] = 0.0;
+    m[q] = 0.0;
     if (e0 + q < n) {
       s.id[q] = id_g[e0 + q];
       s.v[q] = vel[s.id[q]];
@@ -203,29 +203,21 @@ __global__ __launch_bounds__(64) void k_small_wave(
     if (lane < 8) s_m[64 * PER + lane] = 0.0;
     __syncthreads();
   }
-  bool first = true;
-  auto prefix = [&] {  // unequal masses, after a change of order
-    bool diff = false;
-#pragma unroll
-    for (int q = 0; q < PER; ++q) {
-      m[q] = e0 + q < n ? s_id[s.id[q]] : 0.0;
-      if (!first) diff = diff || m[q] != s_m[e0 + q];
-    }
-    u32 k0 = 0;  // the lane that holds the lowest rank whose mass changed
-    double run = 0.0;
-    if (!first) {
-      const u64 b = __ballot(diff);
-      if (b == 0) return;
-      k0 = (u32)__ffsll((long long)b) - 1u;
-      const u64 c = (u64)__double_as_longlong(C[0]);
-      run = __longlong_as_double((long long)(
-          ((u64)(u32)__builtin_amdgcn_readlane((int)(c >> 32), k0) << 32) |
-          (u32)__builtin_amdgcn_readlane((int)c, k0)));
-    }
-    first = false;
+  // The masses below: C[0] of a lane and its masses give its C and its end; the
+  // whole is the sequential sum, bit for bit, exactly when every lane's end is
+  // the next one's C[0].  After a change of order that mostly holds with the
+  // starts as they were (where it does not, rounding went the other way and the
+  // starts move on lane by lane for a few rounds; then everything is summed
+  // again from the first lane in doubt).
+  u32 k0 = 0;  // lanes up to here have the right C[0]
+  auto sum_from_k0 = [&] {
 #pragma unroll
     for (int q = 0; q < PER; ++q) s_m[e0 + q] = m[q];
     __syncthreads();
+    const u64 c = (u64)__double_as_longlong(C[0]);
+    double run = __longlong_as_double((long long)(
+        ((u64)(u32)__builtin_amdgcn_readlane((int)(c >> 32), k0) << 32) |
+        (u32)__builtin_amdgcn_readlane((int)c, k0)));
     // each lane adds up every mass from lane k0's first to its own first (the
     // loads ahead of the chain of additions, zeros from its own on)
     for (u32 k = k0 * PER; k < n; k += 8) {
@@ -235,15 +227,40 @@ __global__ __launch_bounds__(64) void k_small_wave(
 #pragma unroll
       for (int q = 0; q < 8; ++q) run = run + (k + q < e0 ? w[q] : 0.0);
     }
-    if (lane >= k0) {
+    if (lane >= k0) C[0] = run;
+    __syncthreads();
+  };
+  bool first = true;
+  auto prefix = [&] {  // unequal masses, after a change of order
+    bool diff = first;
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+      const double mq_ = e0 + q < n ? s_id[s.id[q]] : 0.0;
+      diff = diff || mq_ != m[q];
+      m[q] = mq_;
+    }
+    if (__ballot(diff) == 0) return;
+    if (first) sum_from_k0();
+    first = false;
+    for (int round = 0;; ++round) {
+      double run = C[0];
 #pragma unroll
       for (int q = 0; q < PER; ++q) {
         C[q] = run;
-        g[q] = (totmass - 2.0 * run) - m[q];
         run = run + m[q];
       }
+      const double next = dpp_mov_f64<DPP_WAVE_SHL1>(run, C[0]);
+      const u64 bad = __ballot(run != next);
+      if (bad == 0 || round > 6) break;
+      if (round == 6) {
+        k0 = (u32)__ffsll((long long)bad) - 1u;
+        sum_from_k0();
+      } else {
+        C[0] = dpp_mov_f64<DPP_WAVE_SHR1>(0.0, run);
+      }
     }
-    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < PER; ++q) g[q] = (totmass - 2.0 * C[q]) - m[q];
   };
   (void)s.sort();
   if constexpr (!EQ) prefix();

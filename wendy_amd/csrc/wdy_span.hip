@@ -430,15 +430,15 @@ static const SpanShape kShapes[SPAN_NSHAPES] = {
     {256, 512, true}, {512, 512, true}, {512, 1024, true},
     {1024, 2048, true}, {512, 2048, true}, {1024, 4096, true}, {1024, 6144, true}};
 static const SpanCost kCost[SPAN_NSHAPES] = {
-    {{0.20, 0.38}, {0.25, 0.34}, {0.025, 0.05}, 1.0, 1.0, 5.5, {0.0042, 0.0042}},
-    {{0.33, 0.50}, {0.34, 0.52}, {0.05, 0.10}, 1.0, 1.0, 5.5, {0.005, 0.005}},
+    {{0.16, 0.32}, {0.20, 0.29}, {0.025, 0.05}, 1.0, 1.0, 5.5, {0.0042, 0.0042}},
+    {{0.27, 0.45}, {0.28, 0.45}, {0.05, 0.10}, 1.0, 1.0, 5.5, {0.005, 0.005}},
     {{0.95, 1.50}, {0., 0.}, {0.19, 0.36}, 1.0, 1.0, 5.5, {0.0035, 0.0035}},
     {{1.20, 1.90}, {0., 0.}, {0.34, 0.65}, 1.0, 1.0, 5.5, {0.004, 0.004}},
     {{1.00, 1.70}, {0., 0.}, {0.42, 0.90}, 1.1, 1.0, 5.5, {0.0045, 0.0045}},
     {{1.35, 2.30}, {0., 0.}, {0.72, 1.40}, 1.2, 1.0, 5.5, {0.0045, 0.0055}},
     {{1.95, 3.40}, {0., 0.}, {1.80, 3.40}, 1.7, 1.0, 5.5, {0.009, 0.015}},
     {{2.30, 3.90}, {0., 0.}, {1.90, 2.80}, 1.6, 1.0, 5.5, {0.008, 0.012}},
-    {{3.80, 6.60}, {0., 0.}, {3.80, 6.60}, 1.0, 1. / 256., 5.5, {0.025, 0.055}},
+    {{3.80, 7.60}, {0., 0.}, {3.80, 7.00}, 1.0, 1. / 256., 5.5, {0.025, 0.055}},
     {{6.00, 0.}, {0., 0.}, {6.00, 0.}, 1.0, 1. / 256., 5.5, {0.025, 0.}}};
 
 // Halo ranks taken over ranks the reach is expected to cross; that follows
