@@ -169,3 +169,20 @@ def test_outputs_of_pipelined_reads(gpu_lib, n):
         assert bits_equal(gx, wx) and bits_equal(gv, wv)
     finally:
         sim.close()
+
+
+@pytest.mark.parametrize('mass', ['equal', 'lognormal'])
+@pytest.mark.parametrize('n', [150001, 300001, 700001])
+def test_large_windows_as_on_the_large_path(gpu_lib, n, mass):
+    """Step sizes up to where the windows no longer pay, so every window shape
+    of this range; both paths' mass prefixes are exact, so the same bits."""
+    x, v, m = disk(n, mass)
+    for h, nleap in ((2.5e-4, 20), (5e-4, 7), (1e-3, 10), (2e-3, 5), (3e-3, 1)):
+        sims = [wendy_amd.Sim(x, v, m, numpy.sum(m), 0.01, path=p) for p in (None, 'large')]
+        out = [(numpy.empty(n), numpy.empty(n)) for _ in sims]
+        for sim, (gx, gv) in zip(sims, out):
+            for _ in range(2):
+                sim.advance(h, nleap)
+            sim.read(gx, gv)
+            sim.close()
+        assert bits_equal(out[0][0], out[1][0]) and bits_equal(out[0][1], out[1][1]), h

@@ -15,9 +15,9 @@
 // k_batch_advance, which ends every interval, redoes the rest of the interval
 // from the marked launch's input (its two sets alternate by launch) and brings
 // it back into the windows' form.  Measured, us per interval of 10 steps at
-// h = 1e-3, before -> with windows: 100 disks of 5000-20000 sheets 962 -> 95
-// (lognormal masses 1183 -> 142), 4 of 40000-60000 2704 -> 59, 400 of 50-60
-// 44 -> 14, 384 of 256-65536 3600 -> 410.
+// h = 1e-3, before -> with windows: 100 disks of 5000-20000 sheets 962 -> 99
+// (lognormal masses 1183 -> 146), 4 of 40000-60000 2704 -> 58, 400 of 50-60
+// 44 -> 13, 2000 of 64-512 156 -> 29, 384 of 256-65536 3600 -> 410.
 //  State lives in one arena:
 // simulation k occupies [off_k, off_k + n_k) of two buffer sets of SoA arrays
 // (key = order-preserving position encoding, velocity, global sheet index,
@@ -343,13 +343,8 @@ __global__ __launch_bounds__(BWT) void k_batch_advance(
   if (WINDOWS) {
     if (d.L) {
       const u32 f = M.fail[d.eslot];
-      u32 *stat = M.stat + (u64)d.vslot * SPAN_SLOTS;
-      if (d.nwin > 1 && t < 64u) {
-        const u32 m = (u32)~wave_max((u64)~stat[t]);
-        stat[t] = SPAN_STAT_INIT;
-        if (t == 0) M.slack[d.eslot] = f ? 0u : m;
-      }
       if (f == 0) return;
+      if (t == 0 && d.nwin > 1) M.intact[d.eslot] = 0;
       step0 = (int)((f - 1u) * d.K);
       a ^= (int)((f - 1u) & 1u);
     }
@@ -492,12 +487,9 @@ __global__ __launch_bounds__(BWT) void k_batch_form(const BatchDesc *__restrict_
   const BatchDesc d = descs[blockIdx.x];
   const u32 t = threadIdx.x;
   window_form(s, d, A, M, d.cur, 0u, err, s_red, s_mm, &s_flag);
-  if (d.nwin > 1)
-    for (u32 i = t; i < SPAN_SLOTS; i += BWT)
-      M.stat[(u64)d.vslot * SPAN_SLOTS + i] = SPAN_STAT_INIT;
   if (t == 0) {
     M.fail[d.eslot] = 0;
-    M.slack[d.eslot] = SPAN_STAT_INIT;
+    M.intact[d.eslot] = 1;
   }
 }
 
@@ -630,9 +622,7 @@ static int batch_plan(wdy_batch *b, double h, int nleap) {
     BatchDesc &q = d[k];
     q.cur ^= (int)((b->iv * (q.L ? q.L : (u32)q.nleap)) & 1u);
     if (b->shape >= 0 && q.L) {
-      float f;
-      __builtin_memcpy(&f, &b->many.slack[k], 4);
-      if (f < 1.05f) b->reach[k] *= f > 0.f ? 1.25 : 1.6;
+      if (b->many.intact[k] == 0) b->reach[k] *= 1.6;
     }
     q.L = q.nwin = 0;
     q.h = h;
@@ -656,7 +646,7 @@ static int batch_plan(wdy_batch *b, double h, int nleap) {
   if (!m.fail) {
     WDY_HIP(hipMalloc(&m.fail, S * 4));
     WDY_HIP(hipHostMalloc((void **)&m.info, S * (SPAN_INFO * 8 + 4), hipHostMallocDefault));
-    m.slack = (u32 *)(m.info + S * SPAN_INFO);
+    m.intact = (u32 *)(m.info + S * SPAN_INFO);
     if (b->arr.mass[0])
       for (u64 *&p : m.cf) WDY_HIP(hipMalloc(&p, b->ntot * 8));
   }
@@ -691,8 +681,7 @@ static int batch_plan(wdy_batch *b, double h, int nleap) {
                          hipMemcpyHostToDevice, b->stream));
   if (m.vmax) WDY_HIP(hipFree(m.vmax));
   m.vmax = nullptr;
-  WDY_HIP(hipMalloc(&m.vmax, (words ? words : 1) * SPAN_SLOTS * (3 * 8 + 4)));
-  m.stat = (u32 *)(m.vmax + words * SPAN_SLOTS * 3);
+  WDY_HIP(hipMalloc(&m.vmax, (words ? words : 1) * SPAN_SLOTS * 3 * 8));
   if (int rc = upload()) return rc;
   // the speed words of the plan's first launch
   return form();
@@ -792,16 +781,13 @@ int wdy_batch_advance(wdy_batch *b, double h, int nleap) {
   WDY_HIP(hipSetDevice(b->device));
   const bool change = h != b->h || nleap != b->nleap;
   // A batch's first interval puts every simulation in order; from the second
-  // on it runs in windows.  A plan stays until h or nleap changes or a halo
-  // gets tight (the reports are the host's to read at any time: they only say
-  // when to look again).
+  // on it runs in windows.  A plan stays until h or nleap changes or a window
+  // failed (the reports are the host's to read at any time: they only say when
+  // to look again).
   bool plan = change || !b->planned;
   if (!plan && b->shape >= 0)
-    for (size_t k = 0; k < b->h_desc.size() && !plan; ++k) {
-      float f;
-      __builtin_memcpy(&f, &b->many.slack[k], 4);
-      plan = b->h_desc[k].L != 0 && f < 1.05f;
-    }
+    for (size_t k = 0; k < b->h_desc.size() && !plan; ++k)
+      plan = b->h_desc[k].L != 0 && b->many.intact[k] == 0;
   if (plan)
     if (int rc = batch_plan(b, h, nleap)) return rc;
   WDY_HIP(hipEventRecord(b->ev0, b->stream));

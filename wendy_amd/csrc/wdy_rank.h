@@ -182,7 +182,14 @@ __device__ __forceinline__ u32 bin_seg_start(u32 k) {
 
 // LDS: positions and sheet indices in bin order, two sets of bin counters (one
 // is cleared while the other is used) and, with unequal masses, the masses in
-// bin order, then the mass below each slot.
+// bin order, then the mass below each slot: 20 and 28 B per sheet.
+//
+// A step is a chain of four to five barriers; with every window on a CU of its
+// own their latency bounds it (256 sheets 0.85 us, 1024 1.2, 4096 3.6), else the
+// CUs' issue rate, ~100 instructions per sheet and step.  A sheet is compared
+// with its bin's positions themselves: with the places in the bin, rounded to
+// 32 bits and masked at the bin's end, a step took a quarter longer, and the
+// LDS held 4096 sheets where it now holds 7168.
 template <class SH, bool MASS>
 struct BinRank {
   static constexpr int CAP = SH::CAP, PER = SH::PER, WT = SH::WT, NWAVE = SH::NWAVE;
@@ -191,13 +198,12 @@ struct BinRank {
   static constexpr int PAD = 4;  // slots read past the last sheet (ms: one more)
   static constexpr size_t BYTES = 8ull * (CAP + PAD) +
                                   (MASS ? 8ull * (CAP + PAD + 1) : 0ull) +
-                                  16ull * 16 + 4ull * (CAP + PAD) + 4ull * CAP +
+                                  16ull * 16 + 4ull * CAP +
                                   8ull * (NB + 1) + (BIN_SEGS + 1) * sizeof(BinSeg);
   static_assert(NB % 256 == 0, "whole bins in every segment");
   double *xs;
   u64 *ms;  // masses in bin order, then the mass below each slot
   u64 *red, *redm;
-  float *xf;  // place within the bin, rounded
   i32 *id;
   u32 *bins;  // [2][NB + 1]: one more, the end of the last bin
   BinSeg *seg;  // [BIN_SEGS], and the window as one
@@ -215,8 +221,7 @@ struct BinRank {
     ms = (u64 *)(xs + CAP + PAD);
     red = MASS ? ms + CAP + PAD + 1 : ms;
     redm = red + 16;
-    xf = (float *)(redm + 16);
-    id = (i32 *)(xf + CAP + PAD);
+    id = (i32 *)(redm + 16);
     bins = (u32 *)(id + CAP);
     s = 0;
     clear(0);
@@ -263,9 +268,7 @@ struct BinRank {
         g[i] += e + eL >= (eL + w + eR) * bin_seg_start(k) >> 8 ? 1u : 0u;
     }
     if (threadIdx.x < 16) red[threadIdx.x] = redm[threadIdx.x] = 0;
-    if (threadIdx.x < PAD) {
-      xf[w + threadIdx.x] = 2.f;
-    }
+    if (threadIdx.x < PAD) xs[w + threadIdx.x] = __builtin_inf();
     __syncthreads();
     x0 = seg[BIN_SEGS].lo;
     scale = seg[BIN_SEGS].scale;
@@ -319,7 +322,6 @@ struct BinRank {
     const u32 t = threadIdx.x;
     u32 *const bn = bins + (s & 1u) * (NB + 1);
     u32 b[PER], slot[PER];
-    float f[PER];
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       slot[i] = 0;
@@ -338,13 +340,10 @@ struct BinRank {
         first = sg.base;
         cnt = sg.cnt;
       }
-      // below the first segment's start: with its first; a segment's last bin
-      // also takes what rounds beyond it
+      // non-decreasing in x; below the first segment's start: with its first; a
+      // segment's last bin also takes what rounds beyond it
       const double q = fmin(fmax((x[i] - lo) * sc, 0.0), (double)cnt);
-      const u32 k = (u32)q;
-      b[i] = first + min(k, cnt - 1);
-      // the place within the bin: non-decreasing in x
-      f[i] = k == cnt ? 1.f : (float)__builtin_amdgcn_fract(q);
+      b[i] = first + min((u32)q, cnt - 1);
       if (i * WT + t < w) {
         slot[i] = atomicAdd(&bn[b[i]], 1u);  // its place in the bin
       }
@@ -377,7 +376,6 @@ struct BinRank {
         lo[i] = bn[b[i]];
         hi[i] = bn[b[i] + 1u];
         slot[i] += lo[i];
-        xf[slot[i]] = f[i];
         xs[slot[i]] = x[i];
         id[slot[i]] = ids[i];
         if (MASS) ms[slot[i]] = m[i];
@@ -404,37 +402,36 @@ struct BinRank {
       if (t == WT - 1) ms[CAP] = run;
       __syncthreads();
     }
-    // Rank inside the bin: the sheets of the bin placed below.  The first PAD
-    // slots are read at once without a look at where the bin ends: what lies
-    // beyond is in a later bin (f starts again from 0: masked by the end).
+    // Rank inside the bin: the sheets of the bin below.  The first PAD slots are
+    // read at once without a look at where the bin ends: what lies beyond is in
+    // a later bin, so above.
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       u32 k = lo[i], eq = 0;
-      float y[PAD];
+      double y[PAD];
       u64 my[PAD + 1];  // mass of a slot: the difference of neighbours
 #pragma unroll
       for (int q = 0; q < PAD; ++q) {
-        y[q] = xf[lo[i] + q];
+        y[q] = xs[lo[i] + q];
         if (MASS) my[q] = ms[lo[i] + q];
       }
       if (MASS) my[PAD] = ms[lo[i] + PAD];
       u64 cm = MASS ? my[0] : 0ull;
 #pragma unroll
       for (int q = 0; q < PAD; ++q) {
-        const float z = lo[i] + q < hi[i] ? y[q] : 3.f;
-        k += z < f[i] ? 1u : 0u;
-        eq += z == f[i] ? 1u : 0u;
-        if (MASS) cm += z < f[i] ? my[q + 1] - my[q] : 0ull;
+        k += y[q] < x[i] ? 1u : 0u;
+        eq += y[q] == x[i] ? 1u : 0u;
+        if (MASS) cm += y[q] < x[i] ? my[q + 1] - my[q] : 0ull;
       }
       for (u32 a = lo[i] + PAD; a < hi[i]; ++a) {
-        const float z = xf[a];
-        k += z < f[i] ? 1u : 0u;
-        eq += z == f[i] ? 1u : 0u;
-        if (MASS && z < f[i]) cm += ms[a + 1] - ms[a];
+        const double z = xs[a];
+        k += z < x[i] ? 1u : 0u;
+        eq += z == x[i] ? 1u : 0u;
+        if (MASS && z < x[i]) cm += ms[a + 1] - ms[a];
       }
-      if (eq > 1) {  // another sheet rounds to the same place: in full
+      if (eq > 1) {  // exactly equal positions go by sheet index
         for (u32 a = lo[i]; a < hi[i]; ++a)
-          if (xf[a] == f[i] && (xs[a] < x[i] || (xs[a] == x[i] && id[a] < ids[i]))) {
+          if (xs[a] == x[i] && id[a] < ids[i]) {
             k += 1;
             if (MASS) cm += ms[a + 1] - ms[a];
           }

@@ -41,7 +41,7 @@ struct SpanArgs {
   u64 *vmax_out;
   u64 *vmax_clr;
   u32 *stat;             // [SPAN_SLOTS] float bits of the smallest halo width /
-                         // reach, with several windows
+                         // reach, with several windows (or null)
   u32 *stat_clr;         // stat words of the next interval, to be reset (or null)
   u32 *stat_host;        // copies of stat in pinned host memory (or null)
   u32 *fail;             // set to fail_value if a window could not vouch for its
@@ -50,11 +50,10 @@ struct SpanArgs {
 
 // Window shapes: one wave (WaveSort), or a workgroup (BinRank).
 struct SpanShape {
-  int threads, cap;
+  int threads, cap, cap_un;  // sheets, with equal and with unequal masses
   bool bin;
 };
 constexpr int SPAN_NSHAPES = 10;
-const SpanShape &span_shape(int i);
 int span_launch(hipStream_t st, int shape, bool eq, const SpanArgs &a);
 
 // ---- many simulations per launch (a batch) -----------------------------------
@@ -62,9 +61,8 @@ int span_launch(hipStream_t st, int shape, bool eq, const SpanArgs &a);
 struct SpanMany {
   u64 *cf[2];   // fixed-point mass below each sheet, per set (null: none unequal)
   u64 *vmax;    // [vslot][3][SPAN_SLOTS]: the word sets of SpanArgs
-  u32 *stat;    // [vslot][SPAN_SLOTS]
   u32 *fail;    // [simulation] 0, or 1 + the launch of the interval that failed
-  u32 *slack;   // [simulation] pinned: the interval's smallest stat, 0: repaired
+  u32 *intact;  // [simulation] pinned: 0 once a window failed (multi-window ones)
   double *info; // [simulation][SPAN_INFO] pinned: SPAN_NW widths, max |v|
 };
 constexpr u32 SPAN_NW = 10;

@@ -12,8 +12,8 @@
 // What bounds the one-step kernel at these sizes is not the GPU's rates but a
 // launch per step, ~12 us of dependent phases each.  Measured, us per interval
 // of 20 steps on the sech^2 disk, before (one launch per step) -> with windows,
-// equal / unequal masses: 2^14 239 -> 37 / 266 -> 49, 2^16 265 -> 58 / 306 ->
-// 75, 2^18 412 -> 108 / 479 -> 147, 2^20 851 -> 407 / 950 -> 580.  What bounds
+// equal / unequal masses: 2^14 239 -> 30 / 266 -> 43, 2^16 265 -> 51 / 306 ->
+// 70, 2^18 412 -> 99 / 479 -> 145, 2^20 851 -> 284 / 950 -> 578.  What bounds
 // a window is the latency of its step, ~1 us of LDS round trips and barriers
 // (0.2-0.5 us for one wave), and from ~256 windows on the CUs' issue rate.
 #include <algorithm>
@@ -120,7 +120,7 @@ __device__ __forceinline__ void span_report(const SpanArgs &A, u32 j, u32 sb, u6
   }
   // (a stale word only costs an atomic that changes nothing; the host's copies
   // are for the next plan's halos, where a lost race does not matter)
-  if (A.nwin > 1 && sb < A.stat[q]) {
+  if (A.nwin > 1 && A.stat && sb < A.stat[q]) {
     atomicMin(A.stat + q, sb);
     if (A.stat_host) A.stat_host[q] = sb;
   }
@@ -388,7 +388,7 @@ __global__ __launch_bounds__(PER ? 64 : SH::WT) void k_span_many(
   A.vmax_in = vm ? vm + (ep % 3u) * SPAN_SLOTS : nullptr;
   A.vmax_out = vm ? vm + ((ep + 1u) % 3u) * SPAN_SLOTS : nullptr;
   A.vmax_clr = vm ? vm + ((ep + 2u) % 3u) * SPAN_SLOTS : nullptr;
-  A.stat = d.nwin > 1 ? M.stat + (u64)d.vslot * SPAN_SLOTS : nullptr;
+  A.stat = nullptr;
   A.stat_clr = nullptr;
   A.stat_host = nullptr;
   A.fail = M.fail + d.eslot;
@@ -417,29 +417,30 @@ int launch_many(hipStream_t st, const BatchDesc *descs, const uint2 *list, u32 n
 }  // namespace
 
 // Window shapes and what they cost, in us, measured on the sech^2 disk with
-// step sizes of 0.1 to 700 ranks: a step takes `lat` + `latd` * sqrt(ranks of
-// displacement per step) while every window has a CU to itself, `two` times
-// that or `sat` per 256 windows when they share the CUs (in steps of one
-// window per CU for the largest shape: `per`); a launch `base` plus `basew`
-// per window.  [0] equal masses, [1] unequal.
+// step sizes of 0.1 to 700 ranks: a step (and the sort that opens an interval)
+// takes `lat` + `latd` * sqrt(ranks of displacement per step) while every window
+// has a CU to itself, `two` times that or `sat` per 256 windows when they share
+// the CUs (in steps of one window per CU for the two largest shapes: `per`); a
+// launch `base` plus `basew` per window.  [0] equal masses, [1] unequal.
 struct SpanCost {
-  double lat[2], latd[2], sat[2], two, per, base, basew[2];
+  double lat[2], latd[2], sat[2], two, per, base[2], basew[2];
 };
 static const SpanShape kShapes[SPAN_NSHAPES] = {
-    {64, 128, false}, {64, 256, false}, {256, 256, true},
-    {256, 512, true}, {512, 512, true}, {512, 1024, true},
-    {1024, 2048, true}, {512, 2048, true}, {1024, 4096, true}, {1024, 6144, true}};
+    {64, 128, 128, false}, {64, 256, 256, false}, {256, 256, 256, true},
+    {256, 512, 512, true}, {512, 512, 512, true}, {512, 1024, 1024, true},
+    {1024, 2048, 2048, true}, {512, 2048, 2048, true}, {1024, 4096, 4096, true},
+    {1024, 7168, 5120, true}};
 static const SpanCost kCost[SPAN_NSHAPES] = {
-    {{0.16, 0.32}, {0.20, 0.29}, {0.025, 0.05}, 1.0, 1.0, 5.5, {0.0042, 0.0042}},
-    {{0.27, 0.45}, {0.28, 0.45}, {0.05, 0.10}, 1.0, 1.0, 5.5, {0.005, 0.005}},
-    {{0.95, 1.50}, {0., 0.}, {0.19, 0.36}, 1.0, 1.0, 5.5, {0.0035, 0.0035}},
-    {{1.20, 1.90}, {0., 0.}, {0.34, 0.65}, 1.0, 1.0, 5.5, {0.004, 0.004}},
-    {{1.00, 1.70}, {0., 0.}, {0.42, 0.90}, 1.1, 1.0, 5.5, {0.0045, 0.0045}},
-    {{1.35, 2.30}, {0., 0.}, {0.72, 1.40}, 1.2, 1.0, 5.5, {0.0045, 0.0055}},
-    {{1.95, 3.40}, {0., 0.}, {1.80, 3.40}, 1.7, 1.0, 5.5, {0.009, 0.015}},
-    {{2.30, 3.90}, {0., 0.}, {1.90, 2.80}, 1.6, 1.0, 5.5, {0.008, 0.012}},
-    {{3.80, 7.60}, {0., 0.}, {3.80, 7.00}, 1.0, 1. / 256., 5.5, {0.025, 0.055}},
-    {{6.00, 0.}, {0., 0.}, {6.00, 0.}, 1.0, 1. / 256., 5.5, {0.025, 0.}}};
+    {{0.16, 0.32}, {0.20, 0.29}, {0.025, 0.05}, 1.0, 1.0, {5.5, 5.5}, {0.0042, 0.0042}},
+    {{0.27, 0.45}, {0.28, 0.45}, {0.05, 0.10}, 1.0, 1.0, {5.5, 5.5}, {0.005, 0.005}},
+    {{0.85, 1.45}, {0., 0.}, {0.16, 0.32}, 1.0, 1.0, {6.5, 7.0}, {0.0035, 0.0035}},
+    {{1.05, 1.80}, {0., 0.}, {0.45, 0.90}, 1.4, 1.0, {6.5, 7.0}, {0.004, 0.004}},
+    {{0.90, 1.60}, {0., 0.}, {0.70, 1.40}, 1.6, 1.0, {6.5, 7.0}, {0.0045, 0.0045}},
+    {{1.20, 2.15}, {0., 0.}, {1.20, 2.20}, 2.0, 1.0, {6.5, 7.0}, {0.0045, 0.0055}},
+    {{1.90, 3.60}, {0., 0.}, {1.90, 3.60}, 1.8, 1.0, {6.5, 8.0}, {0.009, 0.015}},
+    {{2.50, 4.60}, {0., 0.}, {2.20, 4.00}, 1.6, 1.0, {6.5, 8.5}, {0.008, 0.012}},
+    {{3.55, 6.50}, {0., 0.}, {3.55, 6.50}, 1.0, 1. / 256., {7.0, 8.0}, {0.025, 0.04}},
+    {{6.00, 7.30}, {0., 0.}, {6.00, 7.30}, 1.0, 1. / 256., {11., 11.}, {0.043, 0.05}}};
 
 // Halo ranks taken over ranks the reach is expected to cross; that follows
 // the smallest halo width the windows report.
@@ -449,13 +450,14 @@ constexpr double SPAN_MANY_MARGIN = 1.3;
 constexpr int SPAN_KBIN = 64;  // steps per launch of the binned shapes (their
                                // bins are those of its start)
 
-const SpanShape &span_shape(int i) { return kShapes[i]; }
+static int cap_of(int shape, bool eq) {
+  return eq ? kShapes[shape].cap : kShapes[shape].cap_un;
+}
 
 int span_launch(hipStream_t st, int shape, bool eq, const SpanArgs &a) {
-  const SpanShape &sh = kShapes[shape];
   // every window within the shape's capacity, every sheet in one core
   const u32 span = a.nwin > 1 ? a.T + 2 * a.H : a.n;
-  if (span > (u32)sh.cap || a.T < 1 || a.nwin < 1 || a.K < 1 ||
+  if (span > (u32)cap_of(shape, eq) || a.T < 1 || a.nwin < 1 || a.K < 1 ||
       (u64)a.nwin * a.T < (u64)a.n || (u64)(a.nwin - 1) * a.T >= (u64)a.n || (a.nwin > 1 && a.H < 1))
     return fail(WDY_ERUNTIME, "span_launch: %u windows of %u + 2 * %u sheets do "
                 "not fit shape %d (n = %u)", a.nwin, a.T, a.H, shape, a.n);
@@ -471,10 +473,14 @@ int span_launch(hipStream_t st, int shape, bool eq, const SpanArgs &a) {
     case 8: return launch_block<RankShape<1024, 4>>(st, eq, a);
     default: break;
   }
-  using SH = RankShape<1024, 6>;  // fits the LDS with equal masses only
-  if (!eq) return fail(WDY_ERUNTIME, "span_launch: shape %d with unequal masses", shape);
-  return a.ext.kind ? launch_block_one<SH, true, true>(st, a)
-                    : launch_block_one<SH, true, false>(st, a);
+  // what the LDS holds: 20 B per sheet with equal masses, else 28
+  using E = RankShape<1024, 7>;
+  using U = RankShape<1024, 5>;
+  if (a.ext.kind)
+    return eq ? launch_block_one<E, true, true>(st, a)
+              : launch_block_one<U, false, true>(st, a);
+  return eq ? launch_block_one<E, true, false>(st, a)
+            : launch_block_one<U, false, false>(st, a);
 }
 
 template <int PER, class SH>
@@ -496,6 +502,7 @@ int span_many_launch(hipStream_t st, int shape, const BatchDesc *descs,
     case 5: return go(launch_many_both<0, RankShape<512, 2>>);
     case 7: return go(launch_many_both<0, RankShape<512, 4>>);
     case 8: return go(launch_many_both<0, RankShape<1024, 4>>);
+    case 9: return launch_many<0, RankShape<1024, 7>, true>(st, descs, list, neq, arr, m, q, iv);
     default: return fail(WDY_ERUNTIME, "span_many_launch: shape %d", shape);
   }
 }
@@ -530,7 +537,9 @@ void span_many_plan(std::vector<BatchDesc> &d, const double *info,
   auto other = [&](u32 n) {
     return nleap * (n <= 2048 ? 3.4 + 1.7e-3 * n : 5.2e-3 * n);
   };
-  double best = other(maxn);
+  double all = 0.0;  // 512 of its workgroups run at a time
+  for (const BatchDesc &q : d) all += other(q.n) / 512.0;
+  double best = std::max(other(maxn), all);
   int bs = -1, bk = 0;
   auto halo = [&](size_t i, int K) {
     const double *w = info + i * SPAN_INFO;
@@ -546,12 +555,12 @@ void span_many_plan(std::vector<BatchDesc> &d, const double *info,
     for (int L = 1; L <= nleap; L = L < 8 ? L + 1 : L + L / 4) {
       const int K = (nleap + L - 1) / L;
       const int launches = (nleap + K - 1) / K;
-      for (int s : {0, 1, 3, 5, 7, 8}) {
-        if (kShapes[s].bin && K > SPAN_KBIN) continue;
-        const double cap = kShapes[s].cap;
+      for (int s : {0, 1, 3, 5, 7, 8, 9}) {
+        if ((kShapes[s].bin && K > SPAN_KBIN) || (s == 9 && un)) continue;
         const SpanCost &k = kCost[s];
         double W = 0.0, rest = 0.0;
         for (size_t i = 0; i < d.size(); ++i) {
+          const double cap = cap_of(s, d[i].flags & 1u);
           const double H = d[i].n <= cap ? 0.0 : halo(i, K);
           if (2.0 * H + cap / 16 <= cap) W += std::ceil(d[i].n / (cap - 2.0 * H));
           else rest = std::max(rest, other(d[i].n));
@@ -559,7 +568,8 @@ void span_many_plan(std::vector<BatchDesc> &d, const double *info,
         double step = k.lat[un] + k.latd[un] * std::sqrt(disp);
         if (W > 256.0)
           step = std::max(step * k.two, (kShapes[s].bin ? 1.0 : 1.0 + std::sqrt(disp)) * k.sat[un] * std::ceil(W * k.per) / (256.0 * k.per));
-        const double cost = launches * (k.base + k.basew[un] * W + K * step) + rest + 5.0;
+        const double cost =
+            launches * (k.base[un] + k.basew[un] * W + K * step) + step + rest + 5.0;
         if (cost < best) {
           best = cost;
           bs = s;
@@ -573,7 +583,7 @@ void span_many_plan(std::vector<BatchDesc> &d, const double *info,
     BatchDesc &q = d[i];
     q.L = q.K = q.T = q.H = q.nwin = q.vslot = 0;
     if (bs < 0) continue;
-    const double cap = kShapes[bs].cap, H = q.n <= cap ? 0.0 : halo(i, bk);
+    const double cap = cap_of(bs, q.flags & 1u), H = q.n <= cap ? 0.0 : halo(i, bk);
     if (!(2.0 * H + cap / 16 <= cap)) continue;
     q.H = (u32)H;
     q.T = q.n <= cap ? q.n : (u32)cap - 2 * q.H;
@@ -758,9 +768,8 @@ struct SpanGeom {
 };
 static bool span_geom(const wdy_sim *s, int shape, double drift, double kicks,
                       SpanGeom *g) {
-  const u32 n = (u32)s->n, cap = (u32)kShapes[shape].cap;
+  const u32 n = (u32)s->n, cap = (u32)cap_of(shape, s->equal_mass);
   g->est = span_ranks(s, span_reach_x(s, drift, kicks));
-  if (shape == SPAN_NSHAPES - 1 && (!s->equal_mass || n > cap)) return false;
   if (n <= cap) {  // one window, no halo
     g->T = n;
     g->H = 0;
@@ -808,7 +817,7 @@ bool span_plan(wdy_sim *s, double h, int nleap, SpanPlan *plan) {
         double step = k.lat[un] + k.latd[un] * std::sqrt(d);
         if (g.nwin > 256)
           step = std::max(step * k.two, k.sat[un] * std::ceil(g.nwin * k.per) / (256.0 * k.per));
-        cost += count * (k.base + k.basew[un] * g.nwin + K * step);
+        cost += count * (k.base[un] + k.basew[un] * g.nwin + K * step) + (q == 0 ? step : 0.0);
       }
       if (cost < best) {
         best = cost;
@@ -821,7 +830,7 @@ bool span_plan(wdy_sim *s, double h, int nleap, SpanPlan *plan) {
   // the one-step kernel over the whole GPU, measured on the sech^2 disk (us
   // per step, equal / unequal masses; the windows have to win clearly): 14 / 15 at 2^16, 21 / 24 at 2^18, 43 /
   // 48 at 2^20, 59 / 82 at 2^21, 92 / 130 at 2^22
-  return 1.15 * best < nleap * (un ? 15.0 + 3.2e-5 * n : 14.0 + 2.0e-5 * n);
+  return 1.1 * best < nleap * (un ? 15.0 + 3.2e-5 * n : 14.0 + 2.0e-5 * n);
 }
 
 bool span_context(wdy_sim *s) {
