@@ -16,7 +16,7 @@
 // from the marked launch's input (its two sets alternate by launch) and brings
 // it back into the windows' form.  Measured, us per interval of 10 steps at
 // h = 1e-3, before -> with windows: 100 disks of 5000-20000 sheets 962 -> 99
-// (lognormal masses 1183 -> 146), 4 of 40000-60000 2704 -> 58, 400 of 50-60
+// (lognormal masses 1183 -> 131), 4 of 40000-60000 2704 -> 58, 400 of 50-60
 // 44 -> 13, 2000 of 64-512 156 -> 29, 384 of 256-65536 3600 -> 410.
 //  State lives in one arena:
 // simulation k occupies [off_k, off_k + n_k) of two buffer sets of SoA arrays

@@ -182,11 +182,13 @@ __device__ __forceinline__ u32 bin_seg_start(u32 k) {
 
 // LDS: positions and sheet indices in bin order, two sets of bin counters (one
 // is cleared while the other is used) and, with unequal masses, the masses in
-// bin order, then the mass below each slot: 20 and 28 B per sheet.
+// rank order, then the mass below each rank: 20 and 28 B per sheet.
 //
-// A step is a chain of four to five barriers; with every window on a CU of its
+// A step is a chain of four barriers, seven with unequal masses; with every window on a CU of its
 // own their latency bounds it (256 sheets 0.85 us, 1024 1.2, 4096 3.6), else the
-// CUs' issue rate, ~100 instructions per sheet and step.  A sheet is compared
+// CUs' issue rate, ~100 instructions per sheet and step.  Unequal masses go to
+// LDS in the new order after the ranking (4096 sheets: 5.4 us; with a prefix over
+// the bins' slots and the mass summed while ranking, 6.5).  A sheet is compared
 // with its bin's positions themselves: with the places in the bin, rounded to
 // 32 bits and masked at the bin's end, a step took a quarter longer, and the
 // LDS held 4096 sheets where it now holds 7168.
@@ -195,14 +197,14 @@ struct BinRank {
   static constexpr int CAP = SH::CAP, PER = SH::PER, WT = SH::WT, NWAVE = SH::NWAVE;
   static constexpr int NB = CAP, WPT = NB / WT;  // bins, bins per thread
   static_assert(NWAVE <= 16, "one row of lanes scans the waves' totals");
-  static constexpr int PAD = 4;  // slots read past the last sheet (ms: one more)
+  static constexpr int PAD = 4;  // slots read past the last sheet
   static constexpr size_t BYTES = 8ull * (CAP + PAD) +
-                                  (MASS ? 8ull * (CAP + PAD + 1) : 0ull) +
+                                  (MASS ? 8ull * CAP : 0ull) +
                                   16ull * 16 + 4ull * CAP +
                                   8ull * (NB + 1) + (BIN_SEGS + 1) * sizeof(BinSeg);
   static_assert(NB % 256 == 0, "whole bins in every segment");
   double *xs;
-  u64 *ms;  // masses in bin order, then the mass below each slot
+  u64 *ms;  // masses in rank order, then the mass below each rank
   u64 *red, *redm;
   i32 *id;
   u32 *bins;  // [2][NB + 1]: one more, the end of the last bin
@@ -219,7 +221,7 @@ struct BinRank {
     seg = (BinSeg *)base;
     xs = (double *)(seg + BIN_SEGS + 1);
     ms = (u64 *)(xs + CAP + PAD);
-    red = MASS ? ms + CAP + PAD + 1 : ms;
+    red = MASS ? ms + CAP : ms;
     redm = red + 16;
     id = (i32 *)(redm + 16);
     bins = (u32 *)(id + CAP);
@@ -378,13 +380,41 @@ struct BinRank {
         slot[i] += lo[i];
         xs[slot[i]] = x[i];
         id[slot[i]] = ids[i];
-        if (MASS) ms[slot[i]] = m[i];
       }
     }
     clear((s & 1u) ^ 1u);
     ++s;
     __syncthreads();
-    if (MASS) {  // ms becomes the mass below each slot
+    // Rank inside the bin: the sheets of the bin below.  The first PAD slots are
+    // read at once without a look at where the bin ends: what lies beyond is in
+    // a later bin, so above.
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      u32 k = lo[i], eq = 0;
+      double y[PAD];
+#pragma unroll
+      for (int q = 0; q < PAD; ++q) y[q] = xs[lo[i] + q];
+#pragma unroll
+      for (int q = 0; q < PAD; ++q) {
+        k += y[q] < x[i] ? 1u : 0u;
+        eq += y[q] == x[i] ? 1u : 0u;
+      }
+      for (u32 a = lo[i] + PAD; a < hi[i]; ++a) {
+        const double z = xs[a];
+        k += z < x[i] ? 1u : 0u;
+        eq += z == x[i] ? 1u : 0u;
+      }
+      if (eq > 1) {  // exactly equal positions go by sheet index
+        for (u32 a = lo[i]; a < hi[i]; ++a)
+          if (xs[a] == x[i] && id[a] < ids[i]) k += 1;
+      }
+      r[i] = k;
+    }
+    if constexpr (MASS) {  // the masses in the new order, then what is below
+#pragma unroll
+      for (int i = 0; i < PER; ++i)
+        if (i * WT + t < w) ms[r[i]] = m[i];
+      __syncthreads();
       u64 lm[PER], sum = 0;
 #pragma unroll
       for (int q = 0; q < PER; ++q) {
@@ -399,45 +429,9 @@ struct BinRank {
         ms[t * PER + q] = run;
         run += lm[q];
       }
-      if (t == WT - 1) ms[CAP] = run;
       __syncthreads();
-    }
-    // Rank inside the bin: the sheets of the bin below.  The first PAD slots are
-    // read at once without a look at where the bin ends: what lies beyond is in
-    // a later bin, so above.
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      u32 k = lo[i], eq = 0;
-      double y[PAD];
-      u64 my[PAD + 1];  // mass of a slot: the difference of neighbours
-#pragma unroll
-      for (int q = 0; q < PAD; ++q) {
-        y[q] = xs[lo[i] + q];
-        if (MASS) my[q] = ms[lo[i] + q];
-      }
-      if (MASS) my[PAD] = ms[lo[i] + PAD];
-      u64 cm = MASS ? my[0] : 0ull;
-#pragma unroll
-      for (int q = 0; q < PAD; ++q) {
-        k += y[q] < x[i] ? 1u : 0u;
-        eq += y[q] == x[i] ? 1u : 0u;
-        if (MASS) cm += y[q] < x[i] ? my[q + 1] - my[q] : 0ull;
-      }
-      for (u32 a = lo[i] + PAD; a < hi[i]; ++a) {
-        const double z = xs[a];
-        k += z < x[i] ? 1u : 0u;
-        eq += z == x[i] ? 1u : 0u;
-        if (MASS && z < x[i]) cm += ms[a + 1] - ms[a];
-      }
-      if (eq > 1) {  // exactly equal positions go by sheet index
-        for (u32 a = lo[i]; a < hi[i]; ++a)
-          if (xs[a] == x[i] && id[a] < ids[i]) {
-            k += 1;
-            if (MASS) cm += ms[a + 1] - ms[a];
-          }
-      }
-      r[i] = k;
-      if (MASS) c[i] = cm;
+      for (int i = 0; i < PER; ++i) c[i] = ms[r[i]];
     }
   }
 };

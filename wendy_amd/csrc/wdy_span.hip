@@ -12,8 +12,8 @@
 // What bounds the one-step kernel at these sizes is not the GPU's rates but a
 // launch per step, ~12 us of dependent phases each.  Measured, us per interval
 // of 20 steps on the sech^2 disk, before (one launch per step) -> with windows,
-// equal / unequal masses: 2^14 239 -> 30 / 266 -> 43, 2^16 265 -> 51 / 306 ->
-// 70, 2^18 412 -> 99 / 479 -> 145, 2^20 851 -> 284 / 950 -> 578.  What bounds
+// equal / unequal masses: 2^14 239 -> 30 / 266 -> 40, 2^16 265 -> 51 / 306 ->
+// 66, 2^18 412 -> 100 / 479 -> 132, 2^20 851 -> 283 / 950 -> 500.  What bounds
 // a window is the latency of its step, ~1 us of LDS round trips and barriers
 // (0.2-0.5 us for one wave), and from ~256 windows on the CUs' issue rate.
 #include <algorithm>
@@ -433,14 +433,14 @@ static const SpanShape kShapes[SPAN_NSHAPES] = {
 static const SpanCost kCost[SPAN_NSHAPES] = {
     {{0.16, 0.32}, {0.20, 0.29}, {0.025, 0.05}, 1.0, 1.0, {5.5, 5.5}, {0.0042, 0.0042}},
     {{0.27, 0.45}, {0.28, 0.45}, {0.05, 0.10}, 1.0, 1.0, {5.5, 5.5}, {0.005, 0.005}},
-    {{0.85, 1.45}, {0., 0.}, {0.16, 0.32}, 1.0, 1.0, {6.5, 7.0}, {0.0035, 0.0035}},
-    {{1.05, 1.80}, {0., 0.}, {0.45, 0.90}, 1.4, 1.0, {6.5, 7.0}, {0.004, 0.004}},
-    {{0.90, 1.60}, {0., 0.}, {0.70, 1.40}, 1.6, 1.0, {6.5, 7.0}, {0.0045, 0.0045}},
-    {{1.20, 2.15}, {0., 0.}, {1.20, 2.20}, 2.0, 1.0, {6.5, 7.0}, {0.0045, 0.0055}},
-    {{1.90, 3.60}, {0., 0.}, {1.90, 3.60}, 1.8, 1.0, {6.5, 8.0}, {0.009, 0.015}},
-    {{2.50, 4.60}, {0., 0.}, {2.20, 4.00}, 1.6, 1.0, {6.5, 8.5}, {0.008, 0.012}},
-    {{3.55, 6.50}, {0., 0.}, {3.55, 6.50}, 1.0, 1. / 256., {7.0, 8.0}, {0.025, 0.04}},
-    {{6.00, 7.30}, {0., 0.}, {6.00, 7.30}, 1.0, 1. / 256., {11., 11.}, {0.043, 0.05}}};
+    {{0.85, 1.30}, {0., 0.}, {0.16, 0.30}, 1.0, 1.0, {6.5, 7.0}, {0.0035, 0.0035}},
+    {{1.05, 1.60}, {0., 0.}, {0.45, 0.80}, 1.4, 1.0, {6.5, 7.0}, {0.004, 0.004}},
+    {{0.90, 1.40}, {0., 0.}, {0.70, 1.20}, 1.6, 1.0, {6.5, 7.0}, {0.0045, 0.0045}},
+    {{1.20, 1.90}, {0., 0.}, {1.20, 1.90}, 2.0, 1.0, {6.5, 7.0}, {0.0045, 0.0055}},
+    {{1.90, 3.10}, {0., 0.}, {1.90, 3.10}, 1.8, 1.0, {6.5, 8.0}, {0.009, 0.015}},
+    {{2.50, 3.90}, {0., 0.}, {2.20, 3.40}, 1.6, 1.0, {6.5, 8.5}, {0.008, 0.012}},
+    {{3.55, 5.40}, {0., 0.}, {3.55, 5.40}, 1.0, 1. / 256., {7.0, 8.0}, {0.025, 0.04}},
+    {{6.00, 6.30}, {0., 0.}, {6.00, 6.30}, 1.0, 1. / 256., {11., 11.}, {0.043, 0.05}}};
 
 // Halo ranks taken over ranks the reach is expected to cross; that follows
 // the smallest halo width the windows report.
