@@ -213,6 +213,9 @@ static int create_impl(int64_t n, const double *x_slot, const i32 *id_slot,
                      (!(flags & WDY_FORCE_LARGE) && (u64)n <= slim);
     s->small = s->small_class && !span;
     WDY_HIP(hipStreamCreate(&s->stream));
+    // (a gang's member is not read while it runs: its is made if it is needed)
+    if (n > (int64_t)1 << 14 && !(flags & WDY_SHARED_GPU))
+      WDY_HIP(hipStreamCreate(&s->copy_stream));
     WDY_HIP(hipEventCreate(&s->ev0));
     WDY_HIP(hipEventCreate(&s->ev1));
     WDY_HIP(hipEventCreateWithFlags(&s->ev_out, hipEventDisableTiming));
