@@ -643,13 +643,12 @@ static int batch_plan(wdy_batch *b, double h, int nleap) {
   if (!b->planned) return WDY_OK;
   SpanMany &m = b->many;
   const size_t S = d.size();
-  if (!m.fail) {
-    WDY_HIP(hipMalloc(&m.fail, S * 4));
+  if (!m.fail) WDY_HIP(hipMalloc(&m.fail, S * 4));
+  if (!m.info)
     WDY_HIP(hipHostMalloc((void **)&m.info, S * (SPAN_INFO * 8 + 4), hipHostMallocDefault));
-    m.intact = (u32 *)(m.info + S * SPAN_INFO);
-    if (b->arr.mass[0])
-      for (u64 *&p : m.cf) WDY_HIP(hipMalloc(&p, b->ntot * 8));
-  }
+  m.intact = (u32 *)(m.info + S * SPAN_INFO);
+  for (u64 *&p : m.cf)
+    if (b->arr.mass[0] && !p) WDY_HIP(hipMalloc(&p, b->ntot * 8));
   const size_t lds = Lds<BSH, false>::BYTES;
   WDY_HIP(hipFuncSetAttribute((const void *)k_batch_form,
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -660,29 +659,37 @@ static int batch_plan(wdy_batch *b, double h, int nleap) {
   };
   if (int rc = form()) return rc;
   WDY_HIP(hipStreamSynchronize(b->stream));
-  span_many_plan(d, m.info, b->reach, h, nleap, &b->shape);
-  if (b->shape < 0) return upload();
-  std::vector<uint2> list[2];
-  size_t words = 0;
-  b->launches = 0;
-  for (size_t k = 0; k < S; ++k) {
-    for (u32 j = 0; d[k].L && j < d[k].nwin; ++j)
-      list[d[k].flags & 1u ? 0 : 1].push_back(make_uint2((u32)k, j));
-    words += d[k].nwin > 1 ? 1 : 0;
-    b->launches = std::max(b->launches, d[k].L);
+  int shape = -1;
+  span_many_plan(d, m.info, b->reach, h, nleap, &shape);
+  if (shape < 0) return upload();
+  const int rc = [&]() -> int {
+    std::vector<uint2> list[2];
+    size_t words = 0;
+    b->launches = 0;
+    for (size_t k = 0; k < S; ++k) {
+      for (u32 j = 0; d[k].L && j < d[k].nwin; ++j)
+        list[d[k].flags & 1u ? 0 : 1].push_back(make_uint2((u32)k, j));
+      words += d[k].nwin > 1 ? 1 : 0;
+      b->launches = std::max(b->launches, d[k].L);
+    }
+    b->neq = (u32)list[0].size();
+    b->nun = (u32)list[1].size();
+    list[0].insert(list[0].end(), list[1].begin(), list[1].end());
+    if (b->d_list) WDY_HIP(hipFree(b->d_list));
+    b->d_list = nullptr;
+    WDY_HIP(hipMalloc(&b->d_list, list[0].size() * sizeof(uint2)));
+    WDY_HIP(hipMemcpyAsync(b->d_list, list[0].data(), list[0].size() * sizeof(uint2),
+                           hipMemcpyHostToDevice, b->stream));
+    if (m.vmax) WDY_HIP(hipFree(m.vmax));
+    m.vmax = nullptr;
+    WDY_HIP(hipMalloc(&m.vmax, (words ? words : 1) * SPAN_SLOTS * 3 * 8));
+    return upload();
+  }();
+  if (rc) {  // without windows, from where it is
+    for (BatchDesc &q : d) q.L = q.nwin = 0;
+    return rc;
   }
-  b->neq = (u32)list[0].size();
-  b->nun = (u32)list[1].size();
-  list[0].insert(list[0].end(), list[1].begin(), list[1].end());
-  if (b->d_list) WDY_HIP(hipFree(b->d_list));
-  b->d_list = nullptr;
-  WDY_HIP(hipMalloc(&b->d_list, list[0].size() * sizeof(uint2)));
-  WDY_HIP(hipMemcpyAsync(b->d_list, list[0].data(), list[0].size() * sizeof(uint2),
-                         hipMemcpyHostToDevice, b->stream));
-  if (m.vmax) WDY_HIP(hipFree(m.vmax));
-  m.vmax = nullptr;
-  WDY_HIP(hipMalloc(&m.vmax, (words ? words : 1) * SPAN_SLOTS * 3 * 8));
-  if (int rc = upload()) return rc;
+  b->shape = shape;
   // the speed words of the plan's first launch
   return form();
 }
