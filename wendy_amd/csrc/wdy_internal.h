@@ -367,7 +367,8 @@ int warm_ensure(wdy_sim *s);
 // h, false when the windows do not apply or the other paths are faster
 struct SpanPlan {
   int shape = 0;
-  u32 K = 1;  // steps per launch
+  u32 K = 1;           // steps per launch
+  double reach = 1.0;  // of the halos
 };
 bool span_plan(wdy_sim *s, double h, int nleap, SpanPlan *plan);
 // enqueues the set-up on the current (sorted) set; vmax: the largest |v|.

@@ -729,6 +729,10 @@ struct SpanCtx {
   u32 epoch = 0, iv = 0;  // launches and intervals so far
   int fails = 0;          // intervals redone in a row
   bool single = false;    // one window or none
+  SpanPlan last;          // the last search's result, for
+  double l_h = 0.0, l_a0 = 0.0;  // these
+  int l_nleap = 0;
+  bool l_single = false, l_ok = false;
   double fall = 0.8;      // how fast `reach` falls again
   bool off = false;
   bool pending = false;
@@ -766,8 +770,8 @@ struct SpanGeom {
   u32 T, H, nwin;
   double est;  // ranks the reach is expected to cross
 };
-static bool span_geom(const wdy_sim *s, int shape, double drift, double kicks,
-                      SpanGeom *g) {
+static bool span_geom(const wdy_sim *s, int shape, double reach, double drift,
+                      double kicks, SpanGeom *g) {
   const u32 n = (u32)s->n, cap = (u32)cap_of(shape, s->equal_mass);
   g->est = span_ranks(s, span_reach_x(s, drift, kicks));
   if (n <= cap) {  // one window, no halo
@@ -777,7 +781,7 @@ static bool span_geom(const wdy_sim *s, int shape, double drift, double kicks,
     return true;
   }
   if (s->span->single) return false;
-  const double H = std::ceil(SPAN_MARGIN * s->span->reach * g->est) + 2.0;
+  const double H = std::ceil(SPAN_MARGIN * reach * g->est) + 2.0;
   if (!(2.0 * H + cap / 16 <= cap)) return false;
   g->H = (u32)H;
   g->T = cap - 2 * g->H;
@@ -791,8 +795,29 @@ static double span_drift(double ah, int done, int K, int nleap) {
   return ah * (K + (done == 0 ? 0.5 : 0.0) - (done + K == nleap ? 0.5 : 0.0));
 }
 
+static bool span_search(const wdy_sim *s, double h, int nleap, SpanPlan *plan);
+
 bool span_plan(wdy_sim *s, double h, int nleap, SpanPlan *plan) {
   if (!s->span || s->span->off || !(h != 0.0) || !std::isfinite(h)) return false;
+  // The search takes 5-15 us of host time: its result is kept for the intervals
+  // that follow, while the halos they call for are those of the plan.
+  SpanCtx &c = *s->span;
+  double a0, a1;  // (an external force may have come or gone)
+  span_amax(s, &a0, &a1);
+  if (h != c.l_h || nleap != c.l_nleap || c.single != c.l_single || a0 != c.l_a0 ||
+      !(c.reach <= c.last.reach && c.reach >= 0.9 * c.last.reach)) {
+    c.l_h = h;
+    c.l_nleap = nleap;
+    c.l_single = c.single;
+    c.l_a0 = a0;
+    c.last.reach = 1.02 * c.reach;
+    c.l_ok = span_search(s, h, nleap, &c.last);
+  }
+  *plan = c.last;
+  return c.l_ok;
+}
+
+static bool span_search(const wdy_sim *s, double h, int nleap, SpanPlan *plan) {
   const u32 n = (u32)s->n;
   const int un = s->equal_mass ? 0 : 1;
   const double ah = std::fabs(h);
@@ -810,7 +835,7 @@ bool span_plan(wdy_sim *s, double h, int nleap, SpanPlan *plan) {
         const int count = q == 0 ? 1 : launches - 1;
         if (count == 0) break;
         SpanGeom g;
-        if (!span_geom(s, i, span_drift(ah, q * K, K, nleap), ah * K, &g)) {
+        if (!span_geom(s, i, plan->reach, span_drift(ah, q * K, K, nleap), ah * K, &g)) {
           cost = 1e300;
           break;
         }
@@ -968,7 +993,7 @@ int span_interval(wdy_sim *s, double h, int nleap, const SpanPlan &p, double *xo
     const int out = so[q & 1];
     const double ah = std::fabs(h);
     SpanGeom g;
-    if (!span_geom(s, p.shape, span_drift(ah, done, K, nleap), ah * K, &g))
+    if (!span_geom(s, p.shape, p.reach, span_drift(ah, done, K, nleap), ah * K, &g))
       return fail(WDY_ERUNTIME, "span_interval: no windows for shape %d", p.shape);
     if (done == 0) {
       c.p_nwin = g.nwin;
