@@ -335,16 +335,17 @@ __device__ __forceinline__ double pair_end(const PairEnd &e, const double *y,
   return (o + e.twopiG * mk * S) + mk * (vk * vk) / 2.0;
 }
 
-// S_k for QP points y per block over one stretch of
-// sheets: a thread's sheets are read once for all of its QP points, whose sums
-// it keeps in registers, so the sheets' traffic from L2 (16 B for QP pairs of
-// two f64 instructions) falls behind the arithmetic.  With one point per block
-// the loads were what bound it: 30000 x 30000 pairs 808 us, with QP = 16
-// 105 us (the two instructions alone take 46).  A thread adds up a stretch's
-// n / splits / 256 terms, the rest is a tree, in a fixed order.
+// S_k for QP points y per block over one stretch of sheets: a thread's sheets
+// are read once for all of its QP points, whose sums it keeps in registers, so
+// the sheets' traffic from L2 (16 B for QP pairs of two f64 instructions) falls
+// behind the arithmetic.  With one point per block the loads were what bound it:
+// 30000 x 30000 pairs 808 us, with QP = 16 88 us (the two instructions alone take
+// 46; without the bound of eight waves per SIMD, which only reorders them, 105).
+// A thread adds up a stretch's n / splits / 256 terms, the rest is a tree, in a
+// fixed order.
 // out: [splits][ny] sums, or, with one stretch, the results made of them.
 template <int QP>
-__global__ __launch_bounds__(BLOCK) void k_pair_sums(
+__global__ __launch_bounds__(BLOCK, 8) void k_pair_sums(
     u32 n, u32 ny, u32 per, const double *__restrict__ x,
     const double *__restrict__ m, const double *__restrict__ y, PairEnd end,
     double *__restrict__ out) {
