@@ -2,7 +2,7 @@
 // leapfrog steps without going back to memory.  Both forms are exact for any
 // input (positions, then sheet index).
 //
-// * WaveSort: one wave holds up to 64 * PER sheets in registers, PER
+// * WaveSheets: one wave holds up to 64 * PER sheets in registers, PER
 //   consecutive ranks per lane, and re-sorts them after each drift by odd-even
 //   transposition, ending as soon as the order is right: no LDS, no barrier,
 //   ~10 instructions per sheet and rank of displacement.  For steps that move

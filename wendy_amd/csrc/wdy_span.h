@@ -48,7 +48,7 @@ struct SpanArgs {
   u32 fail_value;        // core, or a sheet is no longer finite
 };
 
-// Window shapes: one wave (WaveSort), or a workgroup (BinRank).
+// Window shapes: one wave (WaveSheets), or a workgroup (BinRank).
 struct SpanShape {
   int threads, cap, cap_un;  // sheets, with equal and with unequal masses
   bool bin;
