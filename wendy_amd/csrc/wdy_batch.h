@@ -17,7 +17,7 @@ struct BatchDesc {
   // L launches an interval (0: not in windows)
   u32 T, H, nwin, K, L;
   u32 vslot;      // its word sets, with several windows
-  u32 pad_;
+  u32 id0;        // its first sheet index
   double h;       // leapfrog step
   double mq, totmass, omega2, fscale, finv;
 };

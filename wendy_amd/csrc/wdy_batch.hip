@@ -102,12 +102,18 @@ __device__ u64 block_leap(Lds<BSH, false> &s, const BatchDesc &d, u32 c,
   const u32 t = threadIdx.x;
   const bool eq = d.flags & 1u, harm = d.flags & 2u;
   const u32 r0 = t * BPER;  // ranks r0 .. r0 + BPER - 1 in order
-  u64 local = 0, total = 0;
+  u64 local = 0, total = 0, mf[BPER];
   if (!eq) {
     u64 part = 0;
 #pragma unroll
-    for (int i = 0; i < BPER; ++i)
-      if (r0 + i < c) part += mass_fix(s.m[s.ord[r0 + i]], d.fscale);
+    for (int i = 0; i < BPER; ++i) {
+      mf[i] = 0;
+      if (r0 + i < c) {
+        const u32 e = s.ord[r0 + i];
+        mf[i] = mass_fix(s.m[e], d.fscale, (u32)s.id[e] - d.id0);
+      }
+      part += mf[i];
+    }
     local = block_excl_u64<BNWAVE>(part, s_red, &total);
   }
   u64 pre = run + local;
@@ -123,7 +129,7 @@ __device__ u64 block_leap(Lds<BSH, false> &s, const BatchDesc &d, u32 c,
       } else {
         const double me = s.m[e];
         F = (d.totmass - 2.0 * ((double)pre * d.finv)) - me;
-        pre += mass_fix(me, d.fscale);
+        pre += mf[i];
       }
       if (harm) F = F - d.omega2 * x;
       const double a = 0.0 + F;
@@ -258,8 +264,9 @@ __device__ void window_form(Lds<BSH, false> &s, const BatchDesc &d, const BatchA
   const bool eq = d.flags & 1u;
   u64 *key = A.key[a] + d.off;
   double *vel = A.vel[a] + d.off;
+  i32 *idx = A.idx[a] + d.off;
   double *mass = eq ? nullptr : A.mass[a] + d.off;
-  if (!range_sort(s, n, key, vel, A.idx[a] + d.off, mass, s_red, s_mm, s_flag) && t == 0)
+  if (!range_sort(s, n, key, vel, idx, mass, s_red, s_mm, s_flag) && t == 0)
     atomicOr(err + d.eslot, 1u);
   if (!eq) {
     u64 *cf = M.cf[a] + d.off;
@@ -269,7 +276,7 @@ __device__ void window_form(Lds<BSH, false> &s, const BatchDesc &d, const BatchA
 #pragma unroll
       for (int i = 0; i < BPER; ++i) {
         const u32 r = lo + t * BPER + i;
-        m[i] = r < n ? mass_fix(mass[r], d.fscale) : 0ull;
+        m[i] = r < n ? mass_fix(mass[r], d.fscale, (u32)idx[r] - d.id0) : 0ull;
         part += m[i];
       }
       u64 c = run + block_excl_u64<BNWAVE>(part, s_red, &total);
@@ -505,7 +512,7 @@ void batch_desc_fill(BatchDesc &d, const double *m, u32 n, double totmass,
   d.cur = 0;
   d.nleap = 0;
   d.eslot = 0;
-  d.T = d.H = d.nwin = d.K = d.L = d.vslot = d.pad_ = 0;
+  d.T = d.H = d.nwin = d.K = d.L = d.vslot = d.id0 = 0;
   d.h = 0.0;
   d.mq = m[0];
   d.totmass = totmass;
@@ -741,6 +748,7 @@ int wdy_batch_create(int64_t nsims, const int64_t *offsets, const double *x,
       batch_desc_fill(d, m + offsets[k], (u32)(offsets[k + 1] - offsets[k]),
                       totmass[k], omega2[k]);
       d.off = (u64)offsets[k];
+      d.id0 = (u32)offsets[k];
       any_unequal = any_unequal || !(d.flags & 1u);
     }
     std::stable_sort(descs.begin(), descs.end(),

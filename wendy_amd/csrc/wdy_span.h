@@ -18,6 +18,7 @@ constexpr u32 SPAN_STAT_INIT = 0x7f000000u;  // no window has reported
 // are stored in sorted order (position, then sheet index).
 struct SpanArgs {
   u32 n, T, H, nwin, K;
+  u32 id0;  // the simulation's first sheet index
   const u64 *kin;
   const double *vin;
   const i32 *iin;

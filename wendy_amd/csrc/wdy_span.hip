@@ -153,7 +153,7 @@ __device__ __forceinline__ void span_wave(const SpanArgs &A, const u32 j) {
       s.id[q] = A.iin[i];
       if (!EQ) {
         s.m[q] = A.min[i];
-        s.mf[q] = mass_fix(s.m[q], A.fscale);
+        s.mf[q] = mass_fix(s.m[q], A.fscale, (u32)s.id[q] - A.id0);
       }
     }
     if (EQ) g[q] = (A.totmass - 2.0 * ((double)i * A.mq)) - A.mq;
@@ -235,7 +235,7 @@ __device__ __forceinline__ void span_block(const SpanArgs &A, const u32 j) {
       id[i] = A.iin[R.a + e];
       if (!EQ) {
         m[i] = A.min[R.a + e];
-        mf[i] = mass_fix(m[i], A.fscale);
+        mf[i] = mass_fix(m[i], A.fscale, (u32)id[i] - A.id0);
         c[i] = A.cin[R.a + e];
       }
     }
@@ -360,6 +360,7 @@ __global__ __launch_bounds__(PER ? 64 : SH::WT) void k_span_many(
   A.H = d.H;
   A.nwin = d.nwin;
   A.K = (u32)K;
+  A.id0 = d.id0;
   A.kin = arr.key[in] + d.off;
   A.vin = arr.vel[in] + d.off;
   A.iin = arr.idx[in] + d.off;
@@ -658,12 +659,13 @@ __global__ __launch_bounds__(256) void k_span_widths(u32 n, u32 starts, u32 stri
 // Fixed-point mass below each sheet, in three passes over tiles of FIX_TILE.
 constexpr u32 FIX_TILE = 4096;
 __global__ __launch_bounds__(256) void k_fix_sums(u32 n, const double *__restrict__ mass,
+                                                  const i32 *__restrict__ idx,
                                                   double fscale, u64 *sums) {
   __shared__ u64 s_red[4];
   u64 v = 0;
   for (u32 q = 0; q < FIX_TILE / 256; ++q) {
     const u32 i = blockIdx.x * FIX_TILE + q * 256 + threadIdx.x;
-    if (i < n) v += mass_fix(mass[i], fscale);
+    if (i < n) v += mass_fix(mass[i], fscale, (u32)idx[i]);
   }
   u64 tot;
   (void)block_excl_u64<4>(v, s_red, &tot);
@@ -683,6 +685,7 @@ __global__ __launch_bounds__(256) void k_fix_top(u32 nt, u64 *sums) {
   }
 }
 __global__ __launch_bounds__(256) void k_fix_apply(u32 n, const double *__restrict__ mass,
+                                                   const i32 *__restrict__ idx,
                                                    double fscale, const u64 *sums,
                                                    u64 *__restrict__ out) {
   __shared__ u64 s_red[4];
@@ -690,7 +693,7 @@ __global__ __launch_bounds__(256) void k_fix_apply(u32 n, const double *__restri
   u64 m[FIX_TILE / 256], v = 0;
 #pragma unroll
   for (u32 q = 0; q < FIX_TILE / 256; ++q) {
-    m[q] = base + q < n ? mass_fix(mass[base + q], fscale) : 0ull;
+    m[q] = base + q < n ? mass_fix(mass[base + q], fscale, (u32)idx[base + q]) : 0ull;
     v += m[q];
   }
   u64 run = sums[blockIdx.x] + block_excl_u64<4>(v, s_red, nullptr);
@@ -924,10 +927,11 @@ int span_prefix(wdy_sim *s) {
   SpanCtx &c = *s->span;
   const u32 n = (u32)s->n, nt = (n + FIX_TILE - 1) / FIX_TILE;
   u64 *sums = (u64 *)s->tile_sums;  // N / 4096 + 2 words
-  k_fix_sums<<<nt, 256, 0, s->stream>>>(n, s->mass[s->cur], c.fscale, sums);
+  k_fix_sums<<<nt, 256, 0, s->stream>>>(n, s->mass[s->cur], s->idx[s->cur], c.fscale,
+                                        sums);
   k_fix_top<<<1, 256, 0, s->stream>>>(nt, sums);
-  k_fix_apply<<<nt, 256, 0, s->stream>>>(n, s->mass[s->cur], c.fscale, sums,
-                                         c.cf[s->cur]);
+  k_fix_apply<<<nt, 256, 0, s->stream>>>(n, s->mass[s->cur], s->idx[s->cur], c.fscale,
+                                         sums, c.cf[s->cur]);
   WDY_CHECK_LAUNCH();
   return WDY_OK;
 }
@@ -972,6 +976,7 @@ int span_interval(wdy_sim *s, double h, int nleap, const SpanPlan &p, double *xo
   const int so[2] = {(start + 1) % 3, (start + 2) % 3};
   SpanArgs a;
   a.n = (u32)s->n;
+  a.id0 = 0;
   a.h = h;
   a.mq = s->m_equal;
   a.totmass = s->totmass;
