@@ -1,0 +1,49 @@
+"""The host code's launch rules (wendy_amd/csrc/wdy_rules.h) over everything the
+entry points accept, compiled by themselves: no GPU."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+from conftest import ROOT
+
+PAIRS = r'''
+#include "wdy_rules.h"
+#include <cstdio>
+using namespace wdy;
+int main() {
+  const uint32_t ns[] = {0, 1, 2, 255, 256, 1023, 1024, 1025, 2047, 4096, 30000,
+                         131072, 1000003, (1u << 30) - 1};
+  const uint32_t nys[] = {1, 3, 4, 5, 4095, 4096, 4097, 30000, 1u << 20, (1u << 31) - 1};
+  for (uint32_t n : ns)
+    for (uint32_t ny : nys) {
+      const PairPlan p = pair_plan(n, ny, 256);
+      const uint64_t all = (uint64_t)p.splits * p.per;
+      // every sheet in one stretch, none of them empty (unless there are none)
+      if (p.per < 1 || p.splits < 1 || p.splits > 128 || all < n ||
+          (n > 0 && all - p.per >= n) || (n == 0 && p.splits != 1)) {
+        std::printf("n=%u ny=%u: %u stretches of %u\n", n, ny, p.splits, p.per);
+        return 1;
+      }
+    }
+  return 0;
+}
+'''
+
+
+def run(tmp_path, source):
+    cxx = os.environ.get('CXX') or shutil.which('g++')
+    assert cxx, 'no C++ compiler'
+    src = tmp_path / 't.cpp'
+    src.write_text(source)
+    exe = str(tmp_path / 't')
+    subprocess.run([cxx, '-std=c++17', '-O1', '-Wall', '-Werror', '-I',
+                    os.path.join(ROOT, 'wendy_amd', 'csrc'), str(src), '-o', exe], check=True)
+    got = subprocess.run([exe], capture_output=True, text=True)
+    assert got.returncode == 0, (got.returncode, got.stdout)
+
+
+@pytest.mark.parametrize('source', [PAIRS], ids=['pairs'])
+def test_rules(tmp_path, source):
+    run(tmp_path, source)

@@ -1,0 +1,29 @@
+// Rules of the host code that decide how kernels are launched, in plain C++:
+// they are tested without a GPU.
+#pragma once
+
+#include <algorithm>
+#include <cstdint>
+
+namespace wdy {
+
+// How the pair sums of ny points over n sheets are launched, `block` threads to
+// a block: enough blocks to fill the GPU, stretches no shorter than 4 sheets per
+// thread and at most 128 of them (one thread adds up their sums).  Few points
+// (under 4096) take 4 to a block: their sheets come from L2 anyway, and 16
+// would leave too few blocks.  No sheets are one empty stretch.
+struct PairPlan {
+  uint32_t qp, splits, per;  // points per block, stretches, sheets in each
+};
+inline PairPlan pair_plan(uint32_t n, uint32_t ny, uint32_t block) {
+  PairPlan p;
+  p.qp = ny >= 4096 ? 16 : 4;
+  const uint32_t bx = (ny + p.qp - 1) / p.qp;
+  const uint32_t most = std::min<uint32_t>(128, std::max<uint32_t>(1, n / (4 * block)));
+  p.splits = std::min(most, std::max<uint32_t>(1, (1024 + bx - 1) / bx));
+  p.per = std::max<uint32_t>(1, (n + p.splits - 1) / p.splits);
+  p.splits = std::max<uint32_t>(1, (n + p.per - 1) / p.per);
+  return p;
+}
+
+}  // namespace wdy

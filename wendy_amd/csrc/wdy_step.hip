@@ -17,6 +17,7 @@
 #include <cmath>
 
 #include "wdy_internal.h"
+#include "wdy_rules.h"
 
 namespace wdy {
 namespace {
@@ -693,25 +694,6 @@ int launch_momentum_arrays(int64_t n64, const double *v, const double *m,
 
 namespace {
 
-// How the pair sums of ny points over n sheets are launched: enough blocks to
-// fill the GPU, stretches no shorter than 4 sheets per thread and at most 128 of
-// them (one thread adds up their sums).  Few points
-// (under 4096) take 4 to a block: their sheets come from L2 anyway, and 16
-// would leave too few blocks.
-struct PairPlan {
-  u32 qp, splits, per;
-};
-PairPlan pair_plan(u32 n, u32 ny) {
-  PairPlan p;
-  p.qp = ny >= 4096 ? 16 : 4;
-  const u32 bx = (ny + p.qp - 1) / p.qp;
-  const u32 most = std::min<u32>(128, std::max<u32>(1, n / (4 * BLOCK)));
-  p.splits = std::min(most, std::max<u32>(1, (1024 + bx - 1) / bx));
-  p.per = (n + p.splits - 1) / p.splits;
-  p.splits = (n + p.per - 1) / p.per;
-  return p;
-}
-
 int launch_pairs(const PairPlan &p, u32 n, u32 ny, const double *x, const double *m,
                  const double *y, const PairEnd &end, double *sums, double *out) {
   const dim3 grid((ny + p.qp - 1) / p.qp, p.splits);
@@ -734,7 +716,7 @@ int launch_potential_arrays(int64_t ny, const double *y, int64_t n64,
                             const double *x, const double *m, double twopiG,
                             double omega2, double *out) {
   const u32 n = (u32)n64;
-  const PairPlan p = pair_plan(n, (u32)ny);
+  const PairPlan p = pair_plan(n, (u32)ny, BLOCK);
   DevBufs b;
   double *dx;
   WDY_HIP(b.alloc(&dx, 2 * (size_t)n + (2 + p.splits) * (size_t)ny));
@@ -753,7 +735,7 @@ int launch_energy_individual_arrays(int64_t n64, const double *x,
                                     const double *v, const double *m,
                                     double twopiG, double omega2, double *out) {
   const u32 n = (u32)n64;
-  const PairPlan p = pair_plan(n, n);
+  const PairPlan p = pair_plan(n, n, BLOCK);
   DevBufs b;
   double *dx;
   WDY_HIP(b.alloc(&dx, (4 + p.splits) * (size_t)n));
