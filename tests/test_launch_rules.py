@@ -31,6 +31,25 @@ int main() {
 }
 '''
 
+# Launch q meets words that earlier launches left (0, or 1 + one of them) and,
+# once a window of it has failed, 1 + q: never both answers.
+LEAVES = r'''
+#include "wdy_rules.h"
+#include <cstdio>
+using namespace wdy;
+int main() {
+  for (uint32_t q = 0; q < 70; ++q)
+    for (uint32_t before = 0; before <= q; ++before) {
+      const bool leaves = span_leaves(before, q);
+      if (leaves != (before != 0) || (!leaves && span_leaves(q + 1, q))) {
+        std::printf("launch %u, word %u\n", q, before);
+        return 1;
+      }
+    }
+  return 0;
+}
+'''
+
 
 def run(tmp_path, source):
     cxx = os.environ.get('CXX') or shutil.which('g++')
@@ -44,6 +63,6 @@ def run(tmp_path, source):
     assert got.returncode == 0, (got.returncode, got.stdout)
 
 
-@pytest.mark.parametrize('source', [PAIRS], ids=['pairs'])
+@pytest.mark.parametrize('source', [PAIRS, LEAVES], ids=['pairs', 'leaves'])
 def test_rules(tmp_path, source):
     run(tmp_path, source)

@@ -26,4 +26,12 @@ inline PairPlan pair_plan(uint32_t n, uint32_t ny, uint32_t block) {
   return p;
 }
 
+// Whether a window of launch q of an interval leaves its simulation alone,
+// `word` being the simulation's: 0, or 1 + the launch in which a window could not
+// vouch for its core.  Only an earlier launch's failure counts: every wave of
+// every window of this launch then decides alike, also those that read the word
+// after another window of the launch has set it.  (What this launch writes is
+// not read: the interval is redone from what it was given.)
+constexpr bool span_leaves(uint32_t word, uint32_t q) { return word != 0 && word != q + 1; }
+
 }  // namespace wdy

@@ -22,6 +22,7 @@
 #include <type_traits>
 
 #include "wdy_rank.h"
+#include "wdy_rules.h"
 #include "wdy_span.h"
 
 namespace wdy {
@@ -350,7 +351,7 @@ __global__ __launch_bounds__(PER ? 64 : SH::WT) void k_span_many(
   const uint2 e = list[blockIdx.x];
   const BatchDesc d = descs[e.x];
   const int done = (int)(q * d.K);
-  if (M.fail[d.eslot] != 0 || done >= d.nleap) return;
+  if (span_leaves(M.fail[d.eslot], q) || done >= d.nleap) return;
   const int K = min((int)d.K, d.nleap - done);
   const u32 ep = iv * d.L + q;  // launches since the plan
   const int in = d.cur ^ (int)(ep & 1u), out = in ^ 1;
