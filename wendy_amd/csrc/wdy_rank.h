@@ -1,6 +1,8 @@
 // Sorting of nearly sorted sheets on chip, for kernels that run several
-// leapfrog steps without going back to memory.  Both forms are exact for any
-// input (positions, then sheet index).
+// leapfrog steps without going back to memory.  Both forms are exact (positions,
+// then sheet index) for finite positions, BinRank for a window that was in order
+// when it was loaded.  Otherwise a place may be taken twice and another by no
+// sheet, always inside the window: callers find out and do it again another way.
 //
 // * WaveSheets: one wave holds up to 64 * PER sheets in registers, PER
 //   consecutive ranks per lane, and re-sorts them after each drift by odd-even

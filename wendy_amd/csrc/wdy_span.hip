@@ -75,6 +75,7 @@ __device__ __forceinline__ Reach span_reach(const SpanArgs &A, const u32 j) {
     R.slack = fminf(R.slack, (float)(d / R.D));
   }
   if (j == 0 && threadIdx.x < SPAN_SLOTS) {
+    if (A.fail_clr && threadIdx.x == 0) *A.fail_clr = 0;
     if (A.vmax_clr) A.vmax_clr[threadIdx.x] = 0;
     if (A.stat_clr) A.stat_clr[threadIdx.x] = SPAN_STAT_INIT;
   }
@@ -117,6 +118,7 @@ __device__ __forceinline__ void span_report(const SpanArgs &A, u32 j, u32 sb, u6
   const u32 q = j & (SPAN_SLOTS - 1);
   if (sb == 0) {
     *A.fail = A.fail_value;
+    if (A.fail_host) *A.fail_host = A.fail_value;
     return;
   }
   // (a stale word only costs an atomic that changes nothing; the host's copies
@@ -211,8 +213,9 @@ __device__ __forceinline__ void span_wave(const SpanArgs &A, const u32 j) {
 }
 
 // ---- windows of one workgroup ----------------------------------------------------
+// word: *A.fail, or 0
 template <class SH, bool EQ, bool EXT>
-__device__ __forceinline__ void span_block(const SpanArgs &A, const u32 j) {
+__device__ __forceinline__ void span_block(const SpanArgs &A, const u32 j, u32 word) {
   constexpr int WT = SH::WT, PER = SH::PER, NWAVE = SH::NWAVE;
   extern __shared__ u64 lds_dyn[];
   __shared__ u64 s_vm[NWAVE];
@@ -242,6 +245,7 @@ __device__ __forceinline__ void span_block(const SpanArgs &A, const u32 j) {
     }
   }
   const u64 cbase = EQ ? 0ull : A.cin[R.a];
+  if (span_leaves(word, A.fail_value - 1u)) return;
   BinRank<SH, !EQ> rk(lds_dyn, R.w, A.kin + R.a, R.a > 0 ? (A.H + 1) / 2 : 0,
                        R.b < A.n ? (A.H + 1) / 2 : 0, R.D);
   bool slow = true;  // every speed within the bound
@@ -302,12 +306,15 @@ __device__ __forceinline__ void span_block(const SpanArgs &A, const u32 j) {
 
 template <int PER, bool EQ, bool EXT>
 __global__ __launch_bounds__(64) void k_span_wave(SpanArgs A) {
+  if (span_leaves(*A.fail, A.fail_value - 1u)) return;
   span_wave<PER, EQ, EXT>(A, blockIdx.x);
 }
 
 template <class SH, bool EQ, bool EXT>
 __global__ __launch_bounds__(SH::WT) void k_span_block(SpanArgs A) {
-  span_block<SH, EQ, EXT>(A, blockIdx.x);
+  // read now, looked at once the window's sheets are under way too: 480 us an
+  // interval of 2^20 lognormal sheets, looked at first 491
+  span_block<SH, EQ, EXT>(A, blockIdx.x, *(const volatile u32 *)A.fail);
 }
 
 template <int PER, bool EQ>
@@ -395,10 +402,12 @@ __global__ __launch_bounds__(PER ? 64 : SH::WT) void k_span_many(
   A.stat_host = nullptr;
   A.fail = M.fail + d.eslot;
   A.fail_value = q + 1u;
+  A.fail_clr = nullptr;
+  A.fail_host = nullptr;
   if constexpr (PER > 0)
     span_wave<PER, EQ, false>(A, e.y);
   else
-    span_block<SH, EQ, false>(A, e.y);
+    span_block<SH, EQ, false>(A, e.y, 0u);
 }
 
 template <int PER, class SH, bool EQ>
@@ -602,13 +611,14 @@ void span_many_plan(std::vector<BatchDesc> &d, const double *info,
 namespace {
 
 // vmax: three sets of words, all zero but the first of set `at`; stat: both
-// sets of stat words; width (may be null): the words of k_span_widths
+// sets of stat words, then both intervals' fail words; width (may be null): the words of k_span_widths
 __global__ void k_span_init(u64 *vmax, u32 *stat, u32 at, u64 v, u64 *width) {
   const u32 t = threadIdx.x;
   if (width && t < 16) width[t] = ~0ull;
   for (u32 q = t; q < 3 * SPAN_SLOTS; q += blockDim.x)
     vmax[q] = q == at * SPAN_SLOTS ? v : 0ull;
   for (u32 q = t; q < 2 * SPAN_SLOTS; q += blockDim.x) stat[q] = SPAN_STAT_INIT;
+  if (t < 2) stat[2 * SPAN_SLOTS + t] = 0;
 }
 
 // the largest |v|, into the words (zero before) of one set
@@ -724,8 +734,8 @@ __global__ __launch_bounds__(256) void k_span_gather(
 
 struct SpanCtx {
   u64 *cf[3] = {nullptr, nullptr, nullptr};  // unequal masses: mass below
-  u64 *vmax = nullptr;    // [3][SPAN_SLOTS], then stat [2][SPAN_SLOTS]
-  u32 *stat = nullptr;
+  u64 *vmax = nullptr;    // [3][SPAN_SLOTS]
+  u32 *stat = nullptr;    // [2][SPAN_SLOTS], then the fail words of two intervals
   u64 *h_buf = nullptr;   // pinned: [16] words of the widths, then
   u32 *h_stat = nullptr;  // [SPAN_SLOTS], then the fail word
   double fscale = 1.0, finv = 1.0;
@@ -873,7 +883,7 @@ void span_take(wdy_sim *s, Carve &k) {
   SpanCtx &c = *s->span;
   const size_t N = (size_t)s->n;
   k.take(c.vmax, 3 * SPAN_SLOTS + 16);
-  k.take(c.stat, 2 * SPAN_SLOTS);
+  k.take(c.stat, 2 * SPAN_SLOTS + 2);
   if (!s->equal_mass)
     for (int b = 0; b < 3; ++b) k.take(c.cf[b], N);
 }
@@ -990,10 +1000,12 @@ int span_interval(wdy_sim *s, double h, int nleap, const SpanPlan &p, double *xo
   for (u32 q = 0; q < SPAN_SLOTS; ++q) c.h_stat[q] = SPAN_STAT_INIT;
   c.h_stat[SPAN_SLOTS] = 0;
   a.stat_host = c.h_stat;
-  a.fail = c.h_stat + SPAN_SLOTS;
-  a.fail_value = 1;
-  a.stat = c.stat + SPAN_SLOTS * (c.iv & 1u);
-  a.stat_clr = c.stat + SPAN_SLOTS * ((c.iv + 1u) & 1u);
+  a.fail_host = c.h_stat + SPAN_SLOTS;
+  const u32 set = c.iv++ & 1u;
+  a.stat = c.stat + SPAN_SLOTS * set;
+  a.stat_clr = c.stat + SPAN_SLOTS * (set ^ 1u);
+  a.fail = c.stat + 2 * SPAN_SLOTS + set;
+  a.fail_clr = c.stat + 2 * SPAN_SLOTS + (set ^ 1u);
   double t = s->t0;
   int in = start, q = 0;
   for (int done = 0; done < nleap; ++q) {
@@ -1011,6 +1023,7 @@ int span_interval(wdy_sim *s, double h, int nleap, const SpanPlan &p, double *xo
     a.H = g.H;
     a.nwin = g.nwin;
     a.K = (u32)K;
+    a.fail_value = (u32)q + 1u;
     a.kin = s->key[in];
     a.vin = s->vel[in];
     a.iin = s->idx[in];
@@ -1038,7 +1051,6 @@ int span_interval(wdy_sim *s, double h, int nleap, const SpanPlan &p, double *xo
     done += K;
     in = out;
   }
-  ++c.iv;
   c.pending = true;
   c.p_start = start;
   c.p_h = h;
