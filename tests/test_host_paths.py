@@ -1,0 +1,99 @@
+"""What the library's host code does when device memory runs out or a kernel
+reports back, without a GPU: in a process of its own, on a stand-in for the HIP
+runtime (fake_hip.cpp) that writes launches down and fails allocations on demand.
+"""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+from conftest import ROOT
+
+HEAD = r'''
+import ctypes, sys
+fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+fake.fake_log.restype = ctypes.c_char_p
+fake.fake_deny.argtypes = [ctypes.c_size_t]
+fake.fake_spacing.argtypes = [ctypes.c_double]
+NONE = ctypes.c_size_t(-1).value
+sys.path.insert(0, sys.argv[2])
+import numpy
+import wendy_amd
+
+
+def launched():
+    names = fake.fake_log().decode().split('\n')
+    fake.fake_clear()
+    return names
+
+
+def sim(n, mass='unequal', **kw):
+    rs = numpy.random.default_rng(n)
+    m = rs.uniform(0.5, 2., n) / n if mass == 'unequal' else numpy.full(n, 1. / n)
+    return wendy_amd.Sim(rs.standard_normal(n), rs.standard_normal(n), m, numpy.sum(m),
+                         -1., **kw)
+
+
+def count(names, what):
+    return sum(what in k for k in names)
+
+'''
+
+
+@pytest.fixture(scope='module')
+def fake(tmp_path_factory):
+    cxx = os.environ.get('CXX') or shutil.which('g++')
+    assert cxx, 'no C++ compiler'
+    so = str(tmp_path_factory.mktemp('fake') / 'libfake_hip.so')
+    subprocess.run([cxx, '-std=c++17', '-O1', '-fPIC', '-shared',
+                    os.path.join(ROOT, 'tests', 'fake_hip.cpp'), '-o', so], check=True)
+    return so
+
+
+def run(fake, body):
+    got = subprocess.run([sys.executable, '-c', HEAD + body, fake, ROOT],
+                         capture_output=True, text=True, timeout=300)
+    assert got.returncode == 0, (got.returncode, got.stdout, got.stderr)
+
+
+def test_windows_declined_without_memory_for_the_warm_path(fake):
+    """Its arrays are allocated when they are first needed: radix steps then,
+    and no launch of the warm kernel without them."""
+    run(fake, r'''
+s = sim(20000)            # the stand-in reports no room for windows
+launched()
+config = s.warm_config()  # a question allocates nothing
+fake.fake_deny(1)
+assert s.warm_config() == config and config[0] >= 0
+for _ in range(2):
+    s.advance(0.01, 3)
+    k = launched()
+    assert count(k, 'k_scatter') > 0 and count(k, 'k_warm_step') == 0, k
+fake.fake_deny(NONE)
+s.advance(0.01, 3)        # and back to it
+assert count(launched(), 'k_warm_step') > 0
+s.close()
+''')
+
+
+@pytest.mark.parametrize('mass', ['equal', 'unequal'])
+def test_warm_path_that_cannot_grow(fake, mass):
+    run(fake, r'''
+s = sim(20000, '%s', path='large')
+fake.fake_deny(1)         # this step size calls for more buckets either side
+for _ in range(2):
+    launched()
+    s.advance(10., 3)
+    k = launched()
+    assert count(k, 'k_scatter') > 0 and count(k, 'k_warm_step') == 0, k
+try:
+    s.tune(0, 8, 0)
+    raise AssertionError('tuned without memory')
+except MemoryError:
+    pass
+s.advance(0.01, 3)
+assert count(launched(), 'k_warm_step') == 0
+s.close()
+''' % mass)

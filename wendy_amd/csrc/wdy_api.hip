@@ -394,13 +394,13 @@ static int advance_host_force(wdy_sim *s, double h, int nleap,
 static int cold_interval(wdy_sim *s, double h, int nleap, double *acc_last,
                          double *cum_last) {
   // size the warm-start layout for this h before the splitters of the
-  // next partition are written (a resize reallocates their buffers)
-  if (int rc = warm_ensure(s)) return rc;
-  if (s->warm) {
-    if (int rc = warm_fit(s, h)) return rc;
-  }
+  // next partition are written (a resize reallocates their buffers); without
+  // memory for it the steps stay on the radix path
+  int rc = warm_ensure(s);
+  if (!rc && s->warm) rc = warm_fit(s, h);
+  if (rc && rc != WDY_ENOMEM) return rc;
   s->span_sorted = false;
-  int rc = launch_drift(s, h / 2.);
+  rc = launch_drift(s, h / 2.);
   if (rc) return rc;
   u32 T = 0, nb = 0;
   u64 *spl = s->warm ? warm_cold_splitters(s, &T, &nb) : nullptr;
@@ -863,8 +863,9 @@ int wdy_tune(wdy_sim *sim, int shape, int bucket_target, int window) {
   WDY_HIP(hipSetDevice(sim->device));
   WDY_HIP(hipStreamSynchronize(sim->stream));
   warm_mark_tuned(sim);
+  if (int rc = warm_configure(sim, shape, (u32)bucket_target, (u32)window)) return rc;
   span_off(sim);  // the tuned kernel runs from now on
-  return warm_configure(sim, shape, (u32)bucket_target, (u32)window);
+  return WDY_OK;
 }
 
 int wdy_set_ext_force(wdy_sim *sim, int kind, const double *params, double t0) {
@@ -940,10 +941,9 @@ int wdy_warm_failures(wdy_sim *sim, int64_t *capacity, int64_t *overflow,
 
 int wdy_warm_config(wdy_sim *sim, int *shape, int *bucket_target, int *window) {
   if (int rc = check_settled(sim, "wdy_warm_config")) return rc;
-  if (int rc = warm_ensure(sim)) return rc;
   int sh = -1;
   u32 T = 0, W = 0;
-  if (!warm_config(sim, &sh, &T, &W)) sh = -1;
+  if (!warm_config(sim, &sh, &T, &W)) sh = -1, T = W = 0;
   if (shape) *shape = sh;
   if (bucket_target) *bucket_target = (int)T;
   if (window) *window = (int)W;

@@ -357,7 +357,8 @@ int warm_interval(wdy_sim *s, double h, int nleap);
 // and (h, nleap) must be redone on the radix path
 int warm_settle(wdy_sim *s, bool *failed, double *h, int *nleap);
 int warm_current_shape(wdy_sim *s);
-// the warm path's tile shape, bucket target and window; false without one
+// the warm path's tile shape, bucket target and window, those it would start from
+// if it has not been set up; false when the sim has none
 bool warm_config(wdy_sim *s, int *shape, u32 *T, u32 *W);
 // wait (without checking) for the warm interval in flight, if any
 void warm_wait(wdy_sim *s);

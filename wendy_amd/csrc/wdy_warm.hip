@@ -1307,9 +1307,8 @@ void warm_free(wdy_sim *s) {
   s->warm = nullptr;
 }
 
-// (Re)sizes the metadata for tile shape `shape` (-1: keep), bucket target T
-// (0: 3/4 of the shape's capacity) and window W.
-int warm_configure(wdy_sim *s, int shape, u32 T, u32 W) {
+// warm_configure's work; after a failure the context is not whole.
+static int configure(wdy_sim *s, int shape, u32 T, u32 W) {
   if (!s->warm) {
     s->warm = new (std::nothrow) WarmCtx();
     if (!s->warm) return fail(WDY_ENOMEM, "warm context allocation failed");
@@ -1364,6 +1363,18 @@ int warm_configure(wdy_sim *s, int shape, u32 T, u32 W) {
   }
   w.ready = false;
   return WDY_OK;
+}
+
+// (Re)sizes the metadata for tile shape `shape` (-1: keep), bucket target T
+// (0: 3/4 of the shape's capacity) and window W.  When that fails the simulation
+// has no warm path (until warm_ensure), rather than one without its arrays.
+int warm_configure(wdy_sim *s, int shape, u32 T, u32 W) {
+  const int rc = configure(s, shape, T, W);
+  if (rc) {
+    (void)hipGetLastError();  // else the next launch's check finds it
+    warm_free(s);
+  }
+  return rc;
 }
 
 int warm_ensure(wdy_sim *s) {
@@ -1515,7 +1526,12 @@ int warm_current_shape(wdy_sim *s) {
 }
 
 bool warm_config(wdy_sim *s, int *shape, u32 *T, u32 *W) {
-  if (!s->warm) return false;
+  if (!s->warm) {  // what warm_ensure would start from
+    *shape = s->warm_shape0;
+    *T = warm_default_target((u32)warm_shape(s->warm_shape0).cap);
+    *W = (u32)WARM_WINDOW_DEFAULT;
+    return s->warm_ok;
+  }
   *shape = s->warm->shape;
   *T = s->warm->T;
   *W = s->warm->W;
@@ -1685,7 +1701,8 @@ int warm_settle(wdy_sim *s, bool *failed, double *h, int *nleap) {
     warm_free(s);
     return WDY_OK;
   }
-  return warm_configure(s, shape, T, W);
+  const int rc = warm_configure(s, shape, T, W);
+  return rc == WDY_ENOMEM ? WDY_OK : rc;  // without memory: the radix path
 }
 
 
