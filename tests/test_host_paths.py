@@ -97,3 +97,26 @@ s.advance(0.01, 3)
 assert count(launched(), 'k_warm_step') == 0
 s.close()
 ''' % mass)
+
+
+@pytest.mark.parametrize('granted', [0, 1, 2, 3])
+def test_batch_without_memory_for_windows(fake, granted):
+    """The interval runs in the workgroup-per-simulation kernel, wherever among
+    the windows' allocations the memory runs out, and a later plan may have it."""
+    run(fake, r'''
+b = [numpy.random.default_rng(k) for k in range(40)]
+x = [r.standard_normal(700) for r in b]
+b = wendy_amd.Batch(x, x, [r.uniform(0.5, 2., 700) / 700. for r in b])
+b.advance(1e-3, 10)
+fake.fake_deny([1, 4 * 40 + 1, 40 * 100 + 1, 40 * 700 * 8 + 1][%d])
+for _ in range(2):
+    launched()
+    b.advance(1e-3, 10)
+    k = launched()
+    assert count(k, 'k_batch_advance') == 1
+    assert (count(k, 'k_span_many') > 0) == (%d == 3), k
+fake.fake_deny(NONE)
+b.advance(2e-3, 10)
+assert count(launched(), 'k_span_many') > 0
+b.close()
+''' % (granted, granted))

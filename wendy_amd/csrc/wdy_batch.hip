@@ -621,7 +621,69 @@ static void batch_free(wdy_batch *b) {
   delete b;
 }
 
-// New step parameters and, once the simulations are in order, windows.
+static int batch_upload(wdy_batch *b) {
+  WDY_HIP(hipMemcpyAsync(b->d_desc, b->h_desc.data(), b->h_desc.size() * sizeof(BatchDesc),
+                         hipMemcpyHostToDevice, b->stream));
+  WDY_HIP(hipStreamSynchronize(b->stream));
+  return WDY_OK;
+}
+
+// Every simulation's current set into the windows' form.
+static int batch_form(wdy_batch *b) {
+  const size_t lds = Lds<BSH, false>::BYTES;
+  WDY_HIP(hipFuncSetAttribute((const void *)k_batch_form,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  k_batch_form<<<(unsigned)b->h_desc.size(), BWT, lds, b->stream>>>(b->d_desc, b->arr,
+                                                                    b->many, b->err);
+  WDY_CHECK_LAUNCH();
+  return WDY_OK;
+}
+
+// Windows for the step parameters that batch_plan has set.
+static int batch_windows(wdy_batch *b) {
+  std::vector<BatchDesc> &d = b->h_desc;
+  SpanMany &m = b->many;
+  const size_t S = d.size();
+  if (!m.fail) WDY_HIP(hipMalloc(&m.fail, S * 4));
+  if (!m.info)
+    WDY_HIP(hipHostMalloc((void **)&m.info, S * (SPAN_INFO * 8 + 4), hipHostMallocDefault));
+  m.intact = (u32 *)(m.info + S * SPAN_INFO);
+  for (u64 *&p : m.cf)
+    if (b->arr.mass[0] && !p) WDY_HIP(hipMalloc(&p, b->ntot * 8));
+  if (int rc = batch_form(b)) return rc;
+  WDY_HIP(hipStreamSynchronize(b->stream));
+  int shape = -1;
+  span_many_plan(d, m.info, b->reach, b->h, b->nleap, &shape);
+  if (shape < 0) return batch_upload(b);
+  std::vector<uint2> list[2];
+  size_t words = 0;
+  b->launches = 0;
+  for (size_t k = 0; k < S; ++k) {
+    for (u32 j = 0; d[k].L && j < d[k].nwin; ++j)
+      list[d[k].flags & 1u ? 0 : 1].push_back(make_uint2((u32)k, j));
+    words += d[k].nwin > 1 ? 1 : 0;
+    b->launches = std::max(b->launches, d[k].L);
+  }
+  b->neq = (u32)list[0].size();
+  b->nun = (u32)list[1].size();
+  list[0].insert(list[0].end(), list[1].begin(), list[1].end());
+  if (b->d_list) WDY_HIP(hipFree(b->d_list));
+  b->d_list = nullptr;
+  WDY_HIP(hipMalloc(&b->d_list, list[0].size() * sizeof(uint2)));
+  WDY_HIP(hipMemcpyAsync(b->d_list, list[0].data(), list[0].size() * sizeof(uint2),
+                         hipMemcpyHostToDevice, b->stream));
+  if (m.vmax) WDY_HIP(hipFree(m.vmax));
+  m.vmax = nullptr;
+  WDY_HIP(hipMalloc(&m.vmax, (words ? words : 1) * SPAN_SLOTS * 3 * 8));
+  if (int rc = batch_upload(b)) return rc;
+  // the speed words of the plan's first launch
+  if (int rc = batch_form(b)) return rc;
+  b->shape = shape;
+  return WDY_OK;
+}
+
+// New step parameters and, once the simulations are in order, windows; without
+// memory for those the workgroup-per-simulation kernel goes on.
 static int batch_plan(wdy_batch *b, double h, int nleap) {
   std::vector<BatchDesc> &d = b->h_desc;
   WDY_HIP(hipStreamSynchronize(b->stream));
@@ -639,66 +701,15 @@ static int batch_plan(wdy_batch *b, double h, int nleap) {
   b->h = h;
   b->nleap = nleap;
   b->shape = -1;
-  const size_t bytes = d.size() * sizeof(BatchDesc);
-  auto upload = [&]() -> int {
-    WDY_HIP(hipMemcpyAsync(b->d_desc, d.data(), bytes, hipMemcpyHostToDevice, b->stream));
-    WDY_HIP(hipStreamSynchronize(b->stream));
-    return WDY_OK;
-  };
-  if (int rc = upload()) return rc;
+  if (int rc = batch_upload(b)) return rc;
   b->planned = b->started;
   if (!b->planned) return WDY_OK;
-  SpanMany &m = b->many;
-  const size_t S = d.size();
-  if (!m.fail) WDY_HIP(hipMalloc(&m.fail, S * 4));
-  if (!m.info)
-    WDY_HIP(hipHostMalloc((void **)&m.info, S * (SPAN_INFO * 8 + 4), hipHostMallocDefault));
-  m.intact = (u32 *)(m.info + S * SPAN_INFO);
-  for (u64 *&p : m.cf)
-    if (b->arr.mass[0] && !p) WDY_HIP(hipMalloc(&p, b->ntot * 8));
-  const size_t lds = Lds<BSH, false>::BYTES;
-  WDY_HIP(hipFuncSetAttribute((const void *)k_batch_form,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  auto form = [&]() -> int {
-    k_batch_form<<<(unsigned)S, BWT, lds, b->stream>>>(b->d_desc, b->arr, m, b->err);
-    WDY_CHECK_LAUNCH();
-    return WDY_OK;
-  };
-  if (int rc = form()) return rc;
-  WDY_HIP(hipStreamSynchronize(b->stream));
-  int shape = -1;
-  span_many_plan(d, m.info, b->reach, h, nleap, &shape);
-  if (shape < 0) return upload();
-  const int rc = [&]() -> int {
-    std::vector<uint2> list[2];
-    size_t words = 0;
-    b->launches = 0;
-    for (size_t k = 0; k < S; ++k) {
-      for (u32 j = 0; d[k].L && j < d[k].nwin; ++j)
-        list[d[k].flags & 1u ? 0 : 1].push_back(make_uint2((u32)k, j));
-      words += d[k].nwin > 1 ? 1 : 0;
-      b->launches = std::max(b->launches, d[k].L);
-    }
-    b->neq = (u32)list[0].size();
-    b->nun = (u32)list[1].size();
-    list[0].insert(list[0].end(), list[1].begin(), list[1].end());
-    if (b->d_list) WDY_HIP(hipFree(b->d_list));
-    b->d_list = nullptr;
-    WDY_HIP(hipMalloc(&b->d_list, list[0].size() * sizeof(uint2)));
-    WDY_HIP(hipMemcpyAsync(b->d_list, list[0].data(), list[0].size() * sizeof(uint2),
-                           hipMemcpyHostToDevice, b->stream));
-    if (m.vmax) WDY_HIP(hipFree(m.vmax));
-    m.vmax = nullptr;
-    WDY_HIP(hipMalloc(&m.vmax, (words ? words : 1) * SPAN_SLOTS * 3 * 8));
-    return upload();
-  }();
-  if (rc) {  // without windows, from where it is
-    for (BatchDesc &q : d) q.L = q.nwin = 0;
-    return rc;
-  }
-  b->shape = shape;
-  // the speed words of the plan's first launch
-  return form();
+  const int rc = batch_windows(b);
+  if (!rc) return WDY_OK;
+  (void)hipGetLastError();  // else the next launch's check finds it
+  for (BatchDesc &q : d) q.L = q.nwin = 0;  // from where it is
+  const int ru = batch_upload(b);
+  return rc == WDY_ENOMEM ? ru : rc;
 }
 
 extern "C" {
