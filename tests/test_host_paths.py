@@ -120,3 +120,25 @@ b.advance(2e-3, 10)
 assert count(launched(), 'k_span_many') > 0
 b.close()
 ''' % (granted, granted))
+
+
+@pytest.mark.parametrize('n', [300, 1000, 20000])
+def test_outputs_without_memory_for_staging(fake, n):
+    """They are de-sorted by a launch of their own."""
+    run(fake, r'''
+fake.fake_spacing(1e-4)   # room for windows
+s = sim(%d)
+x, v = numpy.empty(s.n), numpy.empty(s.n)
+s.advance(1e-6, 2)
+fake.fake_deny(1)
+for _ in range(3):
+    launched()
+    s.read_and_advance(x, v, 1e-6, 2)
+    assert count(launched(), 'k_desort') == 1
+fake.fake_deny(NONE)
+s.read_and_advance(x, v, 1e-6, 2)
+launched()
+s.read_and_advance(x, v, 1e-6, 2)
+assert count(launched(), 'k_desort') == 0
+s.close()
+''' % n)

@@ -651,12 +651,17 @@ int wdy_read_and_advance(wdy_sim *sim, double *x_out, double *v_out, double h,
   // outputs by itself, so the copy starts at once (before, a de-sorting launch
   // and an event stood in front of it: 10^4 sheets at 10 steps an output took
   // 60 us against 27, 30000 at one step 63 against 26).
-  const bool stages = sim->small ? (u64)sim->n <= SMALL_WAVE_MAX : sim->span != nullptr;
+  bool stages = sim->small ? (u64)sim->n <= SMALL_WAVE_MAX : sim->span != nullptr;
   if (!sim->copy_stream && N > (size_t)1 << 14)
     WDY_HIP(hipStreamCreate(&sim->copy_stream));
   if (stages && !sim->out_v2) {
-    WDY_HIP(hipMalloc(&sim->out_x2, 2 * N * 8));
-    sim->out_v2 = sim->out_x2 + N;
+    if (hipMalloc(&sim->out_x2, 2 * N * 8) == hipSuccess) {
+      sim->out_v2 = sim->out_x2 + N;
+    } else {  // de-sorted by a launch of their own then
+      (void)hipGetLastError();
+      sim->out_x2 = nullptr;
+      stages = false;
+    }
   }
   if (sim->small && sim->staged < 0) {
     // velocities live in the state buffer: read, then advance
