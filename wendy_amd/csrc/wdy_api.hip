@@ -288,9 +288,12 @@ static int create_impl(int64_t n, const double *x_slot, const i32 *id_slot,
                                               : warm_initial_shape(n, eq);
     if (s->warm_ok) s->disp_rate = displacement_rate(n, x_slot, v_id, id_slot);
     if (span) {
-      double vmax = 0.0;
-      for (int64_t i = 0; i < n; ++i) vmax = std::max(vmax, std::fabs(v_id[i]));
-      if ((r = span_create(s, vmax))) return r;
+      double xmax = 0.0, vmax = 0.0;
+      for (int64_t i = 0; i < n; ++i) {
+        xmax = std::max(xmax, std::fabs(x_slot[i]));
+        vmax = std::max(vmax, std::fabs(v_id[i]));
+      }
+      if ((r = span_create(s, xmax, vmax))) return r;
     } else if ((r = warm_ensure(s))) {
       return r;
     }

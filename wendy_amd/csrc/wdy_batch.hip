@@ -318,6 +318,7 @@ __device__ void window_form(Lds<BSH, false> &s, const BatchDesc &d, const BatchA
     for (u32 k = 0; k < SPAN_NW; ++k)
       info[k] = top[k] ? __longlong_as_double((long long)~top[k]) : 1e308;
     info[SPAN_NW] = __longlong_as_double((long long)top[SPAN_NW]);
+    info[SPAN_NW + 1] = fmax(fabs(decode_pos(key[0])), fabs(decode_pos(key[n - 1])));
   }
   if (d.nwin > 1)
     for (u32 i = t; i < 3 * SPAN_SLOTS; i += BWT)

@@ -372,13 +372,13 @@ struct SpanPlan {
   double reach = 1.0;  // of the halos
 };
 bool span_plan(wdy_sim *s, double h, int nleap, SpanPlan *plan);
-// enqueues the set-up on the current (sorted) set; vmax: the largest |v|.
+// enqueues the set-up on the current (sorted) set; xmax, vmax: the largest |x|, |v|.
 // span_created: once that work has finished
 // (its device arrays are part of the simulation's allocation: span_context,
 // then span_take, before it)
 bool span_context(wdy_sim *s);
 void span_take(wdy_sim *s, Carve &c);
-int span_create(wdy_sim *s, double vmax);
+int span_create(wdy_sim *s, double xmax, double vmax);
 void span_created(wdy_sim *s);
 void span_free(wdy_sim *s);
 void span_off(wdy_sim *s);

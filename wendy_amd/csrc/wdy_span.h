@@ -70,7 +70,7 @@ struct SpanMany {
   u64 *vmax;    // [vslot][3][SPAN_SLOTS]: the word sets of SpanArgs
   u32 *fail;    // [simulation] 0, or 1 + the launch of the interval that failed
   u32 *intact;  // [simulation] pinned: 0 once a window failed (multi-window ones)
-  double *info; // [simulation][SPAN_INFO] pinned: SPAN_NW widths, max |v|
+  double *info; // [simulation][SPAN_INFO] pinned: SPAN_NW widths, max |v|, max |x|
 };
 constexpr u32 SPAN_NW = 10;
 constexpr u32 SPAN_INFO = 12;

@@ -554,15 +554,19 @@ void span_many_plan(std::vector<BatchDesc> &d, const double *info,
   for (const BatchDesc &q : d) all += other(q.n) / 512.0;
   double best = std::max(other(maxn), all);
   int bs = -1, bk = 0;
+  auto amax = [&](size_t i) {  // |acceleration| of any sheet
+    return std::fabs(d[i].totmass) +
+           (d[i].flags & 2u ? d[i].omega2 * info[i * SPAN_INFO + SPAN_NW + 1] : 0.0);
+  };
   auto halo = [&](size_t i, int K) {
     const double *w = info + i * SPAN_INFO;
-    const double dx = 1.04 * (w[SPAN_NW] + ah * K * std::fabs(d[i].totmass)) * ah * (K + 0.5);
+    const double dx = 1.04 * (w[SPAN_NW] + ah * K * amax(i)) * ah * (K + 0.5);
     return std::ceil(SPAN_MANY_MARGIN * reach[i] * ranks_of(w, dx)) + 2.0;
   };
   double disp = 0.0;  // ranks of displacement per step
   for (size_t i = 0; i < d.size(); ++i) {
     const double *w = info + i * SPAN_INFO;
-    disp = std::max(disp, ranks_of(w, ah * (w[SPAN_NW] + ah * std::fabs(d[i].totmass))));
+    disp = std::max(disp, ranks_of(w, ah * (w[SPAN_NW] + ah * amax(i))));
   }
   if (h != 0.0)
     for (int L = 1; L <= nleap; L = L < 8 ? L + 1 : L + L / 4) {
@@ -741,16 +745,18 @@ struct SpanCtx {
   double fscale = 1.0, finv = 1.0;
   double width[16] = {};  // smallest width of 2^(k + 2) ranks at the start
   double vmax_h = 0.0;    // largest |v| at the start
+  double xmax_h = 0.0;    // largest |x| at the start
   double reach = 1.0;     // ranks of a launch's reach over those the two give
   u32 epoch = 0, iv = 0;  // launches and intervals so far
   int fails = 0;          // intervals redone in a row
   bool single = false;    // one window or none
+  bool given_up = false;  // not for steps of this size
   SpanPlan last;          // the last search's result, for
-  double l_h = 0.0, l_a0 = 0.0;  // these
+  double l_h = 0.0, l_a0 = 0.0, l_a1 = 0.0;  // these
   int l_nleap = 0;
   bool l_single = false, l_ok = false;
   double fall = 0.8;      // how fast `reach` falls again
-  bool off = false;
+  bool off = false;       // for good
   bool pending = false;
   int p_start = 0, p_nleap = 0;
   double p_h = 0.0, p_t0 = 0.0;
@@ -774,7 +780,7 @@ static void span_amax(const wdy_sim *s, double *a0, double *a1) {
 static double span_reach_x(const wdy_sim *s, double drift, double kicks) {
   double a0, a1;
   span_amax(s, &a0, &a1);
-  return 1.04 * (s->span->vmax_h + kicks * a0) * drift;
+  return 1.04 * (s->span->vmax_h + kicks * (a0 + a1 * s->span->xmax_h)) * drift;
 }
 static double span_ranks(const wdy_sim *s, double dx) {
   return ranks_of(s->span->width, dx);
@@ -815,17 +821,26 @@ static bool span_search(const wdy_sim *s, double h, int nleap, SpanPlan *plan);
 
 bool span_plan(wdy_sim *s, double h, int nleap, SpanPlan *plan) {
   if (!s->span || s->span->off || !(h != 0.0) || !std::isfinite(h)) return false;
+  SpanCtx &c = *s->span;
+  // Steps of another size try again what was given up for these, and give it up
+  // at the first failure.
+  if (h != c.l_h || nleap != c.l_nleap) {
+    if (c.given_up || c.single) c.fails = s->small_class ? 1 : 2;
+    c.given_up = c.single = false;
+  }
+  if (c.given_up) return false;
   // The search takes 5-15 us of host time: its result is kept for the intervals
   // that follow, while the halos they call for are those of the plan.
-  SpanCtx &c = *s->span;
   double a0, a1;  // (an external force may have come or gone)
   span_amax(s, &a0, &a1);
   if (h != c.l_h || nleap != c.l_nleap || c.single != c.l_single || a0 != c.l_a0 ||
+      a1 != c.l_a1 ||
       !(c.reach <= c.last.reach && c.reach >= 0.9 * c.last.reach)) {
     c.l_h = h;
     c.l_nleap = nleap;
     c.l_single = c.single;
     c.l_a0 = a0;
+    c.l_a1 = a1;
     c.last.reach = 1.02 * c.reach;
     c.l_ok = span_search(s, h, nleap, &c.last);
   }
@@ -888,8 +903,9 @@ void span_take(wdy_sim *s, Carve &k) {
     for (int b = 0; b < 3; ++b) k.take(c.cf[b], N);
 }
 
-int span_create(wdy_sim *s, double vmax) {
+int span_create(wdy_sim *s, double xmax, double vmax) {
   SpanCtx *c = s->span;
+  c->xmax_h = xmax;
   c->vmax_h = vmax;
   int e = 0;  // the fixed-point scale of the other paths: 2^k * totmass <= 2^62
   (void)frexp(s->totmass > 0.0 ? s->totmass : 1.0, &e);
@@ -1101,7 +1117,7 @@ int span_settle(wdy_sim *s, bool *failed, double *h, int *nleap, double **xo,
   ++c.fails;
   if (c.p_nwin == 1) c.off = true;  // not finite
   else if (s->small_class) c.single = c.fails >= 2;
-  else c.off = c.fails >= 3;
+  else c.given_up = c.fails >= 3;
   return span_vmax(s);
 }
 
