@@ -142,3 +142,33 @@ s.read_and_advance(x, v, 1e-6, 2)
 assert count(launched(), 'k_desort') == 0
 s.close()
 ''' % n)
+
+
+@pytest.mark.parametrize('bad', ['numpy.inf', 'numpy.nan'])
+@pytest.mark.parametrize('n', [2000, 9000])
+def test_one_simulation_not_finite(fake, n, bad):
+    """The others of its batch stay in windows."""
+    run(fake, r'''
+@ctypes.CFUNCTYPE(None, ctypes.c_char_p, ctypes.POINTER(ctypes.c_void_p))
+def report(name, args):
+    # what k_batch_form(descs, arrays, many, err) says of every simulation: ten
+    # widths of 4, 8, ... ranks, the largest |v| and |x|; `many` ends with their
+    # address
+    if b'k_batch_form' in name:
+        many = ctypes.cast(args[2], ctypes.POINTER(ctypes.c_void_p))
+        info = numpy.ctypeslib.as_array(
+            ctypes.cast(many[5], ctypes.POINTER(ctypes.c_double)), shape=(40, 12))
+        info[:, :10] = 1e-3 * 2. ** numpy.arange(2, 12)
+        info[:, 10:] = 1.
+        info[39, 10] = %s  # the smallest
+
+
+fake.fake_hook(report)
+r = [numpy.random.default_rng(k) for k in range(40)]
+x = [q.standard_normal(%d if k < 39 else 100) for k, q in enumerate(r)]
+b = wendy_amd.Batch(x, x, [numpy.full(len(q), 1. / len(q)) for q in x])
+for _ in range(2):
+    b.advance(1e-3, 10)
+assert count(launched(), 'k_span_many') > 0
+b.close()
+''' % (bad, n))

@@ -558,6 +558,9 @@ void span_many_plan(std::vector<BatchDesc> &d, const double *info,
     return std::fabs(d[i].totmass) +
            (d[i].flags & 2u ? d[i].omega2 * info[i * SPAN_INFO + SPAN_NW + 1] : 0.0);
   };
+  auto finite = [&](size_t i) {  // one that is not would take the others along
+    return std::isfinite(info[i * SPAN_INFO + SPAN_NW]) && std::isfinite(amax(i));
+  };
   auto halo = [&](size_t i, int K) {
     const double *w = info + i * SPAN_INFO;
     const double dx = 1.04 * (w[SPAN_NW] + ah * K * amax(i)) * ah * (K + 0.5);
@@ -566,7 +569,7 @@ void span_many_plan(std::vector<BatchDesc> &d, const double *info,
   double disp = 0.0;  // ranks of displacement per step
   for (size_t i = 0; i < d.size(); ++i) {
     const double *w = info + i * SPAN_INFO;
-    disp = std::max(disp, ranks_of(w, ah * (w[SPAN_NW] + ah * amax(i))));
+    if (finite(i)) disp = std::max(disp, ranks_of(w, ah * (w[SPAN_NW] + ah * amax(i))));
   }
   if (h != 0.0)
     for (int L = 1; L <= nleap; L = L < 8 ? L + 1 : L + L / 4) {
@@ -579,9 +582,10 @@ void span_many_plan(std::vector<BatchDesc> &d, const double *info,
         for (size_t i = 0; i < d.size(); ++i) {
           const double cap = cap_of(s, d[i].flags & 1u);
           const double H = d[i].n <= cap ? 0.0 : halo(i, K);
-          if (2.0 * H + cap / 16 <= cap) W += std::ceil(d[i].n / (cap - 2.0 * H));
+          if (finite(i) && 2.0 * H + cap / 16 <= cap) W += std::ceil(d[i].n / (cap - 2.0 * H));
           else rest = std::max(rest, other(d[i].n));
         }
+        if (W == 0.0) continue;
         double step = k.lat[un] + k.latd[un] * std::sqrt(disp);
         if (W > 256.0)
           step = std::max(step * k.two, (kShapes[s].bin ? 1.0 : 1.0 + std::sqrt(disp)) * k.sat[un] * std::ceil(W * k.per) / (256.0 * k.per));
@@ -601,7 +605,7 @@ void span_many_plan(std::vector<BatchDesc> &d, const double *info,
     q.L = q.K = q.T = q.H = q.nwin = q.vslot = 0;
     if (bs < 0) continue;
     const double cap = cap_of(bs, q.flags & 1u), H = q.n <= cap ? 0.0 : halo(i, bk);
-    if (!(2.0 * H + cap / 16 <= cap)) continue;
+    if (!finite(i) || !(2.0 * H + cap / 16 <= cap)) continue;
     q.H = (u32)H;
     q.T = q.n <= cap ? q.n : (u32)cap - 2 * q.H;
     q.nwin = (q.n + q.T - 1) / q.T;
