@@ -76,7 +76,9 @@ def test_outputs_of_an_interval_whose_first_launch_failed(gpu_lib, n, kind):
                 assert numpy.array_equal(g, w, equal_nan=True)
             b.advance(h, nleap)
             b.read(*want)
-        if kind == 'overflow' or n > 6144:
+        # (the field at the sheet that overflows leaves no room for several
+        # windows, and without several a collapse does no harm)
+        if (kind == 'overflow') == (n <= 6144):
             assert a.path_stats()[2] >= 1
     finally:
         a.close()

@@ -856,7 +856,9 @@ static bool span_search(const wdy_sim *s, double h, int nleap, SpanPlan *plan) {
   const u32 n = (u32)s->n;
   const int un = s->equal_mass ? 0 : 1;
   const double ah = std::fabs(h);
-  const double d = span_ranks(s, span_reach_x(s, ah, ah));  // one step
+  // ranks in one step (a number also where the field at the outermost sheet
+  // overflows: one window has no halos to fail)
+  const double d = std::min(span_ranks(s, span_reach_x(s, ah, ah)), 1e12);
   double best = 1e300;
   for (int L = 1; L <= nleap; L = L < 8 ? L + 1 : L + L / 4) {
     const int K = (nleap + L - 1) / L;
