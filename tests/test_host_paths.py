@@ -116,7 +116,8 @@ for _ in range(2):
     assert count(k, 'k_batch_advance') == 1
     assert (count(k, 'k_span_many') > 0) == (%d == 3), k
 fake.fake_deny(NONE)
-b.advance(2e-3, 10)
+for _ in range(2):
+    b.advance(2e-3, 10)
 assert count(launched(), 'k_span_many') > 0
 b.close()
 ''' % (granted, granted))
@@ -172,3 +173,20 @@ for _ in range(2):
 assert count(launched(), 'k_span_many') > 0
 b.close()
 ''' % (bad, n))
+
+
+def test_batch_of_changing_steps(fake):
+    """A plan sorts every simulation: only for steps that have come twice."""
+    run(fake, r'''
+x = [numpy.random.default_rng(k).standard_normal(700) for k in range(40)]
+b = wendy_amd.Batch(x, x, [numpy.full(700, 1. / 700.)] * 40)
+for k in range(6):
+    b.advance((1e-3, 2e-3)[k % 2], 10)
+for k in range(6):
+    b.advance(1e-3, 10 + k)
+assert count(launched(), 'k_batch_form') == 0
+b.advance(1e-3, 15)
+k = launched()
+assert count(k, 'k_batch_form') > 0 and count(k, 'k_span_many') > 0
+b.close()
+''')
