@@ -204,9 +204,16 @@ static int create_impl(int64_t n, const double *x_slot, const i32 *id_slot,
     const u64 lim = eq ? SMALL_MAX_EQUAL : SMALL_MAX_UNEQUAL;
     const u64 slim = smax < lim ? smax : lim;
     bool nonneg = true;  // the fixed-point mass prefixes need it
-    for (int64_t i = 0; nonneg && i < n; ++i) nonneg = m_id[i] >= 0.0;
-    // several steps per launch, for a simulation whose path is not asked for
-    const bool span = nonneg && (u64)n > SMALL_WAVE_MAX && (u64)n <= SPAN_MAX &&
+    double msum = 0.0;
+    for (int64_t i = 0; nonneg && i < n; ++i) {
+      nonneg = m_id[i] >= 0.0;
+      msum += m_id[i];
+    }
+    // several steps per launch, for a simulation whose path is not asked for.  (The
+    // windows take their unit of mass and their bound of the field from totmass,
+    // which a caller may have set to something else than the masses' sum; the
+    // one-workgroup path does not care.)
+    const bool span = nonneg && std::fabs(msum - totmass) <= 1e-6 * msum && (u64)n > SMALL_WAVE_MAX && (u64)n <= SPAN_MAX &&
                       !(flags & (WDY_FORCE_SMALL | WDY_FORCE_LARGE | WDY_NO_WARM |
                                  WDY_SHARED_GPU));
     s->small_class = (flags & WDY_FORCE_SMALL) ||
