@@ -13,6 +13,7 @@ size_t g_deny = SIZE_MAX;  // allocations of this many bytes or more fail
 int g_last = 0;
 std::string g_log;
 std::map<const void *, std::string> g_names;
+std::map<char *, size_t> g_host;
 struct Dim3 {
   uint32_t x, y, z;
 };
@@ -87,12 +88,39 @@ int hipLaunchKernel(const void *f, Dim3 grid, Dim3 block, void **args, size_t, v
 }
 
 int hipMalloc(void **p, size_t n) { return alloc(p, n); }
-int hipHostMalloc(void **p, size_t n, unsigned) { return alloc(p, n); }
 int hipFree(void *p) {
   free(p);
   return 0;
 }
-int hipHostFree(void *p) { return hipFree(p); }
+// page-locked host memory: allocations, and what a test registers
+void fake_register(void *p, size_t n) { g_host[(char *)p] = n; }
+int hipHostMalloc(void **p, size_t n, unsigned) {
+  const int rc = alloc(p, n);
+  if (!rc) fake_register(*p, n);
+  return rc;
+}
+int hipHostFree(void *p) {
+  g_host.erase((char *)p);
+  return hipFree(p);
+}
+int hipMemGetAddressRange(void **base, size_t *size, void *p) {
+  auto it = g_host.upper_bound((char *)p);
+  if (it == g_host.begin() || (--it, (char *)p >= it->first + it->second)) return fail(INVALID);
+  *base = it->first;
+  *size = it->second;
+  return 0;
+}
+struct Attributes {
+  int type, device;
+  void *device_pointer, *host_pointer;
+};
+int hipPointerGetAttributes(Attributes *a, void *p) {
+  void *base;
+  size_t size;
+  if (hipMemGetAddressRange(&base, &size, p)) return INVALID;
+  *a = {1 /* hipMemoryTypeHost */, 0, p, p};
+  return 0;
+}
 int hipMemcpy(void *d, const void *s, size_t n, int) {
   if (n) memmove(d, s, n);
   return 0;
@@ -126,7 +154,6 @@ int hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, const void *, int, size
 }
 int hipFuncSetAttribute(const void *, int, int) { return 0; }
 int hipGetSymbolAddress(void **, const void *) { return fail(INVALID); }
-int hipPointerGetAttributes(void *, const void *) { return fail(INVALID); }
 int hipGetLastError() {
   const int e = g_last;
   g_last = 0;

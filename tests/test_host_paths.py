@@ -17,6 +17,7 @@ fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
 fake.fake_log.restype = ctypes.c_char_p
 fake.fake_deny.argtypes = [ctypes.c_size_t]
 fake.fake_spacing.argtypes = [ctypes.c_double]
+fake.fake_register.argtypes = [ctypes.c_void_p, ctypes.c_size_t]
 NONE = ctypes.c_size_t(-1).value
 sys.path.insert(0, sys.argv[2])
 import numpy
@@ -189,4 +190,31 @@ b.advance(1e-3, 15)
 k = launched()
 assert count(k, 'k_batch_form') > 0 and count(k, 'k_span_many') > 0
 b.close()
+''')
+
+
+def test_outputs_written_by_a_kernel(fake):
+    """Only into memory that is page-locked from end to end."""
+    run(fake, r'''
+fake.fake_spacing(1e-4)
+s = sim(1000)
+s.advance(1e-6, 2)
+
+
+def copied(x, v):
+    launched()
+    s.read_and_advance(x, v, 1e-6, 2)
+    return count(launched(), 'k_copy_out') > 0
+
+
+pinned = wendy_amd._lib.pinned_empty
+assert copied(pinned(1000), pinned(1000))
+big = pinned(3000)
+assert copied(big[:1000], big[2000:])
+plain = numpy.empty(1000)
+assert not copied(plain, pinned(1000)) and not copied(pinned(1000), plain)
+fake.fake_register(plain.ctypes.data, 800)           # its ends, by themselves
+fake.fake_register(plain.ctypes.data + 7200, 800)
+assert not copied(plain, pinned(1000)) and not copied(pinned(1000), plain)
+s.close()
 ''')

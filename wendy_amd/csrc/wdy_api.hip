@@ -636,18 +636,20 @@ static bool copy_kernel(size_t n, int nleap) {
   return n <= (size_t)1 << 14 || (n <= (size_t)1 << 16 && nleap <= 2);
 }
 
-// Whether a kernel may write these bytes of host memory at their own address.
-static bool device_visible(const void *p, size_t bytes) {
-  const char *const q = (const char *)p;
-  for (const char *b : {q, q + bytes - 1}) {
-    hipPointerAttribute_t at;
-    if (hipPointerGetAttributes(&at, b) != hipSuccess) {
-      (void)hipGetLastError();
-      return false;
-    }
-    if (at.type != hipMemoryTypeHost || at.devicePointer != (const void *)b) return false;
+// Whether a kernel may write these bytes of host memory at their own address: they
+// lie in one page-locked allocation or registration (the pages between two of
+// them need not be).
+static bool device_visible(void *p, size_t bytes) {
+  hipPointerAttribute_t at;
+  void *base = nullptr;
+  size_t size = 0;
+  if (hipPointerGetAttributes(&at, p) != hipSuccess ||
+      hipMemGetAddressRange(&base, &size, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
   }
-  return true;
+  return at.type == hipMemoryTypeHost && at.devicePointer == p &&
+         (size_t)((char *)p - (char *)base) + bytes <= size;
 }
 
 int wdy_read_and_advance(wdy_sim *sim, double *x_out, double *v_out, double h,
