@@ -50,6 +50,30 @@ int main() {
 }
 '''
 
+SPLITS = r'''
+#include "wdy_rules.h"
+#include <cstdio>
+using namespace wdy;
+int main() {
+  const int ns[] = {1, 2, 7, 8, 9, 100, 1001, 1 << 30, 1879048193, 2147483647};
+  for (int nleap : ns) {
+    int tried = 0, most = 0;
+    bool ok = true;
+    each_split(nleap, [&](int K, int launches) {
+      ok = ok && K >= 1 && launches >= 1 && (int64_t)K * launches >= nleap &&
+           (int64_t)K * (launches - 1) < nleap;
+      tried += 1;
+      most = launches > most ? launches : most;
+    });
+    if (!ok || tried > 200 || most < (nleap < 9 ? nleap : nleap / 2)) {
+      std::printf("nleap=%d: %d tried, at most %d launches\n", nleap, tried, most);
+      return 1;
+    }
+  }
+  return 0;
+}
+'''
+
 
 def run(tmp_path, source):
     cxx = os.environ.get('CXX') or shutil.which('g++')
@@ -63,6 +87,7 @@ def run(tmp_path, source):
     assert got.returncode == 0, (got.returncode, got.stdout)
 
 
-@pytest.mark.parametrize('source', [PAIRS, LEAVES], ids=['pairs', 'leaves'])
+@pytest.mark.parametrize('source', [PAIRS, LEAVES, SPLITS],
+                         ids=['pairs', 'leaves', 'splits'])
 def test_rules(tmp_path, source):
     run(tmp_path, source)

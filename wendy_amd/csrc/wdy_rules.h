@@ -34,4 +34,15 @@ inline PairPlan pair_plan(uint32_t n, uint32_t ny, uint32_t block) {
 // not read: the interval is redone from what it was given.)
 constexpr bool span_leaves(uint32_t word, uint32_t q) { return word != 0 && word != q + 1; }
 
+// The ways of cutting an interval of nleap steps into launches that a plan tries:
+// fn(K, launches) with K steps a launch, for every number of launches up to 8,
+// then for numbers a quarter apart.  (In 64 bits: nleap may be any positive int.)
+template <class F>
+inline void each_split(int nleap, F fn) {
+  for (int64_t L = 1; L <= nleap; L = L < 8 ? L + 1 : L + L / 4) {
+    const int64_t K = (nleap + L - 1) / L;
+    fn((int)K, (int)((nleap + K - 1) / K));
+  }
+}
+
 }  // namespace wdy

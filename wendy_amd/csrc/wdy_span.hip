@@ -572,9 +572,7 @@ void span_many_plan(std::vector<BatchDesc> &d, const double *info,
     if (finite(i)) disp = std::max(disp, ranks_of(w, ah * (w[SPAN_NW] + ah * amax(i))));
   }
   if (h != 0.0)
-    for (int L = 1; L <= nleap; L = L < 8 ? L + 1 : L + L / 4) {
-      const int K = (nleap + L - 1) / L;
-      const int launches = (nleap + K - 1) / K;
+    each_split(nleap, [&](int K, int launches) {
       for (int s : {0, 1, 3, 5, 7, 8, 9}) {
         if ((kShapes[s].bin && K > SPAN_KBIN) || (s == 9 && un)) continue;
         const SpanCost &k = kCost[s];
@@ -597,7 +595,7 @@ void span_many_plan(std::vector<BatchDesc> &d, const double *info,
           bk = K;
         }
       }
-    }
+    });
   *shape = bs;
   u32 vslot = 0;
   for (size_t i = 0; i < d.size(); ++i) {
@@ -610,7 +608,7 @@ void span_many_plan(std::vector<BatchDesc> &d, const double *info,
     q.T = q.n <= cap ? q.n : (u32)cap - 2 * q.H;
     q.nwin = (q.n + q.T - 1) / q.T;
     q.K = (u32)bk;
-    q.L = (u32)((nleap + bk - 1) / bk);
+    q.L = (u32)(((int64_t)nleap + bk - 1) / bk);
     if (q.nwin > 1) q.vslot = vslot++;
   }
 }
@@ -817,8 +815,8 @@ static bool span_geom(const wdy_sim *s, int shape, double reach, double drift,
 
 // Time units a launch of K steps from step `done` of the interval drifts: the
 // interval opens and closes with half a drift.
-static double span_drift(double ah, int done, int K, int nleap) {
-  return ah * (K + (done == 0 ? 0.5 : 0.0) - (done + K == nleap ? 0.5 : 0.0));
+static double span_drift(double ah, int64_t done, int64_t K, int nleap) {
+  return ah * ((double)K + (done == 0 ? 0.5 : 0.0) - (done + K == nleap ? 0.5 : 0.0));
 }
 
 static bool span_search(const wdy_sim *s, double h, int nleap, SpanPlan *plan);
@@ -860,9 +858,7 @@ static bool span_search(const wdy_sim *s, double h, int nleap, SpanPlan *plan) {
   // overflows: one window has no halos to fail)
   const double d = std::min(span_ranks(s, span_reach_x(s, ah, ah)), 1e12);
   double best = 1e300;
-  for (int L = 1; L <= nleap; L = L < 8 ? L + 1 : L + L / 4) {
-    const int K = (nleap + L - 1) / L;
-    const int launches = (nleap + K - 1) / K;
+  each_split(nleap, [&](int K, int launches) {
     for (int i = 0; i < SPAN_NSHAPES; ++i) {
       const SpanCost &k = kCost[i];
       if (kShapes[i].bin && K > SPAN_KBIN) continue;
@@ -872,7 +868,7 @@ static bool span_search(const wdy_sim *s, double h, int nleap, SpanPlan *plan) {
         const int count = q == 0 ? 1 : launches - 1;
         if (count == 0) break;
         SpanGeom g;
-        if (!span_geom(s, i, plan->reach, span_drift(ah, q * K, K, nleap), ah * K, &g)) {
+        if (!span_geom(s, i, plan->reach, span_drift(ah, (int64_t)q * K, K, nleap), ah * K, &g)) {
           cost = 1e300;
           break;
         }
@@ -887,7 +883,7 @@ static bool span_search(const wdy_sim *s, double h, int nleap, SpanPlan *plan) {
         plan->K = (u32)K;
       }
     }
-  }
+  });
   if (s->small_class) return best < 1e300;
   // the one-step kernel over the whole GPU, measured on the sech^2 disk (us
   // per step, equal / unequal masses; the windows have to win clearly): 14 / 15 at 2^16, 21 / 24 at 2^18, 43 /
