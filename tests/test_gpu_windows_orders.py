@@ -1,0 +1,98 @@
+"""Windows over what their other tests leave out: steps back in time, massless
+tracers among unequal masses, unequal masses in an external force, and the large
+windows themselves (that they ran, and ran alike to another path).
+
+Unequal masses are held to the bar of the approximate path, 1e-10; the windows
+and a batch use the same exact mass prefix: bitwise.
+"""
+import numpy
+import pytest
+
+import wendy_amd
+from conftest import bits_equal, rel_inf
+from oracle import nbody_oracle as O
+from wendy_amd import forces
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-10
+
+
+def disk(n, mass):
+    x, v, m = O.sech2_disk(n, seed=n, mass='equal' if mass != 'lognormal' else ('lognormal', 0.5))
+    if mass == 'equal':
+        m = numpy.full(n, 2. ** -numpy.ceil(numpy.log2(n)))
+    elif mass == 'tracers':
+        m = numpy.zeros(n)
+        m[:(n + 1) // 2] = 1. / ((n + 1) // 2)
+    return x, v, m
+
+
+def outputs(x, v, m, h, nleap, nout, omega=None, force=None, path=None):
+    sim = wendy_amd.Sim(x, v, m, numpy.sum(m), -1. if omega is None else omega ** 2., path=path)
+    sim.set_ext_force(force, 0.)
+    out = []
+    for _ in range(nout):
+        gx, gv = numpy.empty(len(x)), numpy.empty(len(x))
+        sim.advance(h, nleap)
+        sim.read(gx, gv)
+        out.append((gx, gv))
+    st = sim.path_stats()
+    sim.close()
+    return out, st
+
+
+@pytest.mark.parametrize('mass', ['equal', 'lognormal', 'tracers'])
+@pytest.mark.parametrize('force', [None, forces.Harmonic(0.3), forces.Pulse(0.4, 0.01, 0.02)],
+                         ids=['none', 'harmonic', 'pulse'])
+@pytest.mark.parametrize('h', [1e-3, -1e-3])
+@pytest.mark.parametrize('n', [600, 1537, 5000, 30001])
+def test_against_the_oracle(gpu_lib, n, h, force, mass):
+    x, v, m = disk(n, mass)
+    st = O.ApproxState(x, v, m, h * 10, 10, omega=0.1, ext_force=force)
+    got, stats = outputs(x, v, m, h, 10, 3, omega=0.1, force=force)
+    assert stats[1:] == (0, 0)  # in windows, nothing redone
+    for gx, gv in got:
+        wx, wv = st.onestep()[:2]
+        # (the device's exp differs from the host's in the last place)
+        if mass == 'equal' and not isinstance(force, forces.Pulse):
+            assert bits_equal(gx, wx) and bits_equal(gv, wv)
+        else:
+            assert rel_inf(gx, wx) <= TOL and rel_inf(gv, wv) <= TOL
+
+
+@pytest.mark.parametrize('mass', ['lognormal', 'tracers'])
+@pytest.mark.parametrize('h', [1e-3, -1e-3])
+def test_batch_as_alone(gpu_lib, h, mass):
+    """Sizes that start at odd places of the batch's arrays."""
+    states = [disk(n, mass) for n in (20001, 513, 3000, 1537)]
+    b = wendy_amd.Batch(*[list(a) for a in zip(*states)], omegas=[0.1] * 4)
+    alone = [outputs(x, v, m, h, 10, 3, omega=0.1)[0] for x, v, m in states]
+    for k in range(3):
+        b.advance(h, 10)
+        gx, gv, _ = b.read()
+        for j, out in enumerate(alone):
+            assert bits_equal(gx[j], out[k][0]) and bits_equal(gv[j], out[k][1]), (k, j)
+    b.close()
+
+
+@pytest.mark.parametrize('mass', ['equal', 'lognormal', 'tracers'])
+@pytest.mark.parametrize('n', [150001, 700001, 1 << 20])
+def test_large_windows(gpu_lib, n, mass):
+    """Every step size here is taken in windows."""
+    x, v, m = disk(n, mass)
+    for h, nleap in ((2.5e-4, 20), (5e-4, 7)):
+        got, st = outputs(x, v, m, h, nleap, 2)
+        assert st == (2 * nleap, 0, 0)
+        if mass == 'equal':
+            want = outputs(x, v, m, h, nleap, 2, path='large')[0]
+        else:
+            b = wendy_amd.Batch([x], [v], [m])
+            want = []
+            for _ in range(2):
+                b.advance(h, nleap)
+                gx, gv, _ = b.read()
+                want.append((gx[0], gv[0]))
+            b.close()
+        for g, w in zip(got, want):
+            assert bits_equal(g[0], w[0]) and bits_equal(g[1], w[1]), (h, rel_inf(g[0], w[0]))
