@@ -19,7 +19,7 @@ N, H, NLEAP, OUT = 900001, 1e-4, 400, 3
 
 
 def knot(seed):
-    x, _, _ = O.sech2_disk(N, seed=seed)
+    x = numpy.sort(O.sech2_disk(N, seed=seed)[0])
     return x, numpy.where(numpy.abs(x) < 0.3, -10. * x, 0.), numpy.full(N, 2. ** -20)
 
 

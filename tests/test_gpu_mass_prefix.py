@@ -57,9 +57,11 @@ def test_mass_below(gpu_lib, n, kind):
     st = sim.path_stats()
     sim.close()
     assert st[1:] == (0, 0)  # in windows
-    b = wendy_amd.Batch([x], [v], [m])
-    b.advance(H, 1)
-    bv = b.read()[1][0]
-    b.close()
-    for got in (gv, bv):
+    out = [gv]
+    if n < 1 << 16:  # (one workgroup puts a batch's simulation in order at first)
+        b = wendy_amd.Batch([x], [v], [m])
+        b.advance(H, 1)
+        out.append(b.read()[1][0])
+        b.close()
+    for got in out:
         assert numpy.max(numpy.abs(got.astype(numpy.longdouble) / H - want)) <= tol

@@ -81,6 +81,7 @@ def test_batch_as_alone(gpu_lib, h, mass):
 def test_large_windows(gpu_lib, n, mass):
     """Every step size here is taken in windows."""
     x, v, m = disk(n, mass)
+    x = numpy.sort(x)
     for h, nleap in ((2.5e-4, 20), (5e-4, 7)):
         got, st = outputs(x, v, m, h, nleap, 2)
         assert st == (2 * nleap, 0, 0)
