@@ -218,3 +218,35 @@ fake.fake_register(plain.ctypes.data + 7200, 800)
 assert not copied(plain, pinned(1000)) and not copied(pinned(1000), plain)
 s.close()
 ''')
+
+
+def test_inputs_are_looked_over(fake):
+    """A bad value is found wherever it stands; a negative mass, or a total mass
+    that is not the sum, leaves a simulation without windows."""
+    run(fake, r'''
+for n in list(range(1, 20)) + [1000]:
+    good = [numpy.linspace(-1., 1., n), numpy.linspace(2., -2., n), numpy.full(n, 1. / n)]
+    for i in sorted({0, n // 3, n - 1}):
+        for a in range(3):
+            for bad in (numpy.nan, numpy.inf, -numpy.inf):
+                xvm = [q.copy() for q in good]
+                xvm[a][i] = bad
+                try:
+                    wendy_amd.Sim(*xvm, 1., -1.)
+                    raise AssertionError((n, i, a, bad))
+                except ValueError as e:
+                    assert 'sheet %d' % i in str(e), e
+        m = good[2].copy()
+        m[i] *= 2.
+        if n > 1:
+            try:
+                wendy_amd.Sim(good[0], good[1], m, 1., -1., equal_mass=True)
+                raise AssertionError((n, i))
+            except ValueError as e:
+                assert 'm[%d]' % (i or 1) in str(e), e
+        for m, total, windows in ((good[2], 1., True), (m, m.sum(), True), (m, 3., False),
+                                  (numpy.where(m == m[i], -m, m), m.sum(), False)):
+            launched()
+            wendy_amd.Sim(good[0], good[1], m, total, -1., equal_mass=False).close()
+            assert (count(launched(), 'k_span_widths') == 1) == (windows and n > 512), n
+''')

@@ -158,6 +158,60 @@ static double displacement_rate(int64_t n, const double *x_slot, const double *v
   return (double)n * rho * vmax;
 }
 
+// What a simulation's arrays hold, in one pass over them: the largest |x|, |v| and
+// the masses' sum, and whether anything is not finite, a mass negative or one
+// unlike the first.  (Pairs of values, four independent chains: the loops that
+// looked for each of these in turn took 6.1 ms for 2^22 equal masses, 5.0
+// without the largest |v|; this takes 3.4.)
+struct HostScan {
+  double x = 0.0, v = 0.0, msum = 0.0;
+  bool finite = true, negative = false, unequal = false;
+};
+static HostScan host_scan(int64_t n, const double *x, const double *v, const double *m) {
+  typedef double Pair __attribute__((vector_size(16)));
+  typedef long long Bits __attribute__((vector_size(16)));
+  constexpr int U = 4;
+  const Bits mask = {(long long)~SIGN, (long long)~SIGN};
+  const Pair first = {m[0], m[0]};
+  Pair tx[U] = {}, tv[U] = {}, sum[U] = {}, low[U] = {}, bad[U] = {};
+  Bits other[U] = {};
+  int64_t i = 0;
+  for (; i + 2 * U <= n; i += 2 * U)
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+      Pair px, pv, pm;
+      __builtin_memcpy(&px, x + i + 2 * j, 16);
+      __builtin_memcpy(&pv, v + i + 2 * j, 16);
+      __builtin_memcpy(&pm, m + i + 2 * j, 16);
+      const Pair ax = (Pair)((Bits)px & mask), av = (Pair)((Bits)pv & mask);
+      tx[j] = ax > tx[j] ? ax : tx[j];
+      tv[j] = av > tv[j] ? av : tv[j];
+      bad[j] += ((px - px) + (pv - pv)) + (pm - pm);  // NaN unless all are finite
+      sum[j] += pm;
+      low[j] = pm < low[j] ? pm : low[j];
+      other[j] |= pm != first;
+    }
+  HostScan s;
+  double all = 0.0, lowest = 0.0;
+  auto take = [&](double ax, double av, double sm, double lo, double b, bool o) {
+    s.x = std::max(s.x, ax);
+    s.v = std::max(s.v, av);
+    s.msum += sm;
+    lowest = std::min(lowest, lo);
+    all += b;
+    s.unequal = s.unequal || o;
+  };
+  for (int j = 0; j < U; ++j)
+    for (int k = 0; k < 2; ++k)
+      take(tx[j][k], tv[j][k], sum[j][k], low[j][k], bad[j][k], other[j][k] != 0);
+  for (; i < n; ++i)
+    take(std::fabs(x[i]), std::fabs(v[i]), m[i], m[i],
+         ((x[i] - x[i]) + (v[i] - v[i])) + (m[i] - m[i]), m[i] != m[0]);
+  s.finite = all == 0.0;
+  s.negative = lowest < 0.0;
+  return s;
+}
+
 // Creates a sim from positions given per slot (x_slot[i] is the position of
 // sheet id_slot[i]; id_slot null means the identity) and velocities/masses
 // given per sheet (v_id[j], m_id[j]).  The positions are sorted on the device
@@ -175,13 +229,15 @@ static int create_impl(int64_t n, const double *x_slot, const i32 *id_slot,
     return fail(WDY_EINVAL, "wdy_create: unknown flags 0x%x", flags);
   if ((flags & WDY_FORCE_LARGE) && (flags & WDY_FORCE_SMALL))
     return fail(WDY_EINVAL, "wdy_create: WDY_FORCE_LARGE and WDY_FORCE_SMALL");
-  for (int64_t i = 0; i < n; ++i)
-    if (!std::isfinite(x_slot[i]) || !std::isfinite(v_id[i]) ||
-        !std::isfinite(m_id[i]))
-      return fail(WDY_EINVAL, "wdy_create: non-finite input at sheet %lld",
-                  (long long)i);
+  const HostScan scan = host_scan(n, x_slot, v_id, m_id);
+  if (!scan.finite)
+    for (int64_t i = 0; i < n; ++i)
+      if (!std::isfinite(x_slot[i]) || !std::isfinite(v_id[i]) ||
+          !std::isfinite(m_id[i]))
+        return fail(WDY_EINVAL, "wdy_create: non-finite input at sheet %lld",
+                    (long long)i);
   const bool eq = flags & WDY_EQUAL_MASS;
-  if (eq)
+  if (eq && scan.unequal)
     for (int64_t i = 1; i < n; ++i)
       if (m_id[i] != m_id[0])
         return fail(WDY_EINVAL,
@@ -203,17 +259,13 @@ static int create_impl(int64_t n, const double *x_slot, const i32 *id_slot,
                   (long long)n, smax);
     const u64 lim = eq ? SMALL_MAX_EQUAL : SMALL_MAX_UNEQUAL;
     const u64 slim = smax < lim ? smax : lim;
-    bool nonneg = true;  // the fixed-point mass prefixes need it
-    double msum = 0.0;
-    for (int64_t i = 0; nonneg && i < n; ++i) {
-      nonneg = m_id[i] >= 0.0;
-      msum += m_id[i];
-    }
+    const bool nonneg = !scan.negative;  // the fixed-point mass prefixes need it
     // several steps per launch, for a simulation whose path is not asked for.  (The
     // windows take their unit of mass and their bound of the field from totmass,
     // which a caller may have set to something else than the masses' sum; the
     // one-workgroup path does not care.)
-    const bool span = nonneg && std::fabs(msum - totmass) <= 1e-6 * msum && (u64)n > SMALL_WAVE_MAX && (u64)n <= SPAN_MAX &&
+    const bool span = nonneg && std::fabs(scan.msum - totmass) <= 1e-6 * scan.msum &&
+                      (u64)n > SMALL_WAVE_MAX && (u64)n <= SPAN_MAX &&
                       !(flags & (WDY_FORCE_SMALL | WDY_FORCE_LARGE | WDY_NO_WARM |
                                  WDY_SHARED_GPU));
     s->small_class = (flags & WDY_FORCE_SMALL) ||
@@ -295,12 +347,7 @@ static int create_impl(int64_t n, const double *x_slot, const i32 *id_slot,
                                               : warm_initial_shape(n, eq);
     if (s->warm_ok) s->disp_rate = displacement_rate(n, x_slot, v_id, id_slot);
     if (span) {
-      double xmax = 0.0, vmax = 0.0;
-      for (int64_t i = 0; i < n; ++i) {
-        xmax = std::max(xmax, std::fabs(x_slot[i]));
-        vmax = std::max(vmax, std::fabs(v_id[i]));
-      }
-      if ((r = span_create(s, xmax, vmax))) return r;
+      if ((r = span_create(s, scan.x, scan.v))) return r;
     } else if ((r = warm_ensure(s))) {
       return r;
     }
