@@ -216,10 +216,12 @@ struct BinRank {
   u32 s;
   u32 g[PER];  // the sheets' segments
 
-  // kin: the keys of the window's w sheets, in order.  The segments go by rank
-  // as if there were eL ranks more in a length d below the first sheet and eR
-  // in d above the last (each 0 or the same): where the sheets go that leave the window.
-  __device__ BinRank(u64 *base, u32 w, const u64 *kin, u32 eL, u32 eR, double d) {
+  // kin: the keys of the window's w sheets, in order; d, d1: how far a sheet may
+  // move in the launch and in one of its steps.  The segments go by rank as if there were eL ranks more in a
+  // length d below the first sheet and eR in d above the last (each 0 or the
+  // same): where the sheets go that leave the window.
+  __device__ BinRank(u64 *base, u32 w, const u64 *kin, u32 eL, u32 eR, double d,
+                     double d1) {
     seg = (BinSeg *)base;
     xs = (double *)(seg + BIN_SEGS + 1);
     ms = (u64 *)(xs + CAP + PAD);
@@ -256,10 +258,15 @@ struct BinRank {
       const double first = at(0), last = at(tot), all = last - first;
       const bool full = !((double)q.cnt * all <= 6.0 * (double)NB * range);
       const u32 any = __ballot(full) != 0 ? 1u : 0u;
+      // sheets that a step moves further than they are apart (all of them may
+      // start at one place, and so in one bin: 6144 of them took 45 ms an interval
+      // of 20 steps, now 0.4): over where they can go
+      const bool apart = e > 0 || !(all < 2.0 * d1);
       if (t == 0) {
-        q.lo = first;
-        q.scale = all > 1.0e-300 && all < 1.0e300 ? (double)NB / all : 0.0;
-        q.base = any;
+        const double to = apart ? all : all + 2.0 * d;
+        q.lo = apart ? first : first - d;
+        q.scale = to > 1.0e-300 && to < 1.0e300 ? (double)NB / to : 0.0;
+        q.base = apart ? any : 0u;
         seg[BIN_SEGS] = q;
       }
     }

@@ -247,7 +247,7 @@ __device__ __forceinline__ void span_block(const SpanArgs &A, const u32 j, u32 w
   const u64 cbase = EQ ? 0ull : A.cin[R.a];
   if (span_leaves(word, A.fail_value - 1u)) return;
   BinRank<SH, !EQ> rk(lds_dyn, R.w, A.kin + R.a, R.a > 0 ? (A.H + 1) / 2 : 0,
-                       R.b < A.n ? (A.H + 1) / 2 : 0, R.D);
+                       R.b < A.n ? (A.H + 1) / 2 : 0, R.D, R.D / (double)A.K);
   bool slow = true;  // every speed within the bound
   auto steps = [&](auto segs) {
     constexpr bool SEGS = decltype(segs)::value;
