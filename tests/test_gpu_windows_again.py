@@ -45,6 +45,18 @@ def test_strong_fields_from_rest(gpu_lib, by):
         assert bits_equal(bx[0], wx) and bits_equal(bv[0], wv)
 
 
+@pytest.mark.parametrize('n,h', [(10000, 0.1), (32768, 0.03)])
+def test_steps_too_large_for_windows(gpu_lib, n, h):
+    """About a thousand ranks a step: one step per launch is faster."""
+    x, v, m = disk(n)
+    sim = wendy_amd.Sim(x, v, m, numpy.sum(m), -1.)
+    for _ in range(2):
+        sim.advance(h, 20)
+    stats = sim.path_stats()
+    sim.close()
+    assert stats[:2] == (20, 20)  # a radix interval, then the warm-start kernel
+
+
 def test_steps_of_another_size_try_again(gpu_lib):
     """A knot of sheets falls through one point within an interval, where no
     halos hold; later, shorter steps are taken in windows again."""

@@ -875,6 +875,11 @@ static bool span_search(const wdy_sim *s, double h, int nleap, SpanPlan *plan) {
         double step = k.lat[un] + k.latd[un] * std::sqrt(d);
         if (g.nwin > 256)
           step = std::max(step * k.two, k.sat[un] * std::ceil(g.nwin * k.per) / (256.0 * k.per));
+        // (sheets that cross a good part of their window every step also change
+        // its segments: us per 20 steps, windows / one step per launch: 8000 sheets
+        // at h = 0.1 254 / 240, 10^4 261 / 242, 32768 at 0.03 297 / 253; at half of
+        // that the windows win, 20000 at 0.03 235 / 249)
+        if (!un && g.nwin > 1 && d > 800.0) step *= 1.4;
         cost += count * (k.base[un] + k.basew[un] * g.nwin + K * step) + (q == 0 ? step : 0.0);
       }
       if (cost < best) {
