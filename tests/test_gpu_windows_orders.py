@@ -117,3 +117,36 @@ def test_sheets_from_one_place(gpu_lib, width, n, mass):
             assert bits_equal(gx, wx) and bits_equal(gv, wv)
         else:
             assert rel_inf(gx, wx) <= TOL and rel_inf(gv, wv) <= TOL
+
+
+@pytest.mark.parametrize('n', [513, 6145, 30000])
+def test_outputs_in_any_order_of_calls(gpu_lib, n):
+    """Reads after every interval, after some, twice, beside an energy, and
+    changing over to pipelined reads and back; a collapse that is redone."""
+    x, v, m = disk(n, 'equal')
+    if n == 30000:
+        v = numpy.where(numpy.abs(x) < 0.05, -10. * x, 0.)
+    st = O.ApproxState(x, v, m, 0.05, 10, omega=0.1)
+    sim = wendy_amd.Sim(x, v, m, numpy.sum(m), 0.1 ** 2.)
+    gx, gv = numpy.empty(n), numpy.empty(n)
+    px, pv = wendy_amd._lib.pinned_empty(n), wendy_amd._lib.pinned_empty(n)
+
+    def equal(a, b):
+        assert bits_equal(a, wx) and bits_equal(b, wv)
+    sim.advance(0.005, 10)
+    wx, wv = [a.copy() for a in st.onestep()[:2]]
+    for call in 'raraaraeraarrpparappaar':
+        if call == 'a':
+            sim.advance(0.005, 10)
+            wx, wv = [a.copy() for a in st.onestep()[:2]]
+        elif call == 'r':
+            gx[:] = gv[:] = numpy.nan
+            sim.read(gx, gv)
+            equal(gx, gv)
+        elif call == 'e':
+            sim.energy()
+        else:
+            sim.read_and_advance(px, pv, 0.005, 10)
+            equal(px, pv)
+            wx, wv = [a.copy() for a in st.onestep()[:2]]
+    sim.close()

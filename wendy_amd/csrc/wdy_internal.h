@@ -237,6 +237,7 @@ struct wdy_sim {
   double *out_x2 = nullptr, *out_v2 = nullptr;
   int stage_next = 0;  // the pair the next interval would write
   int staged = -1;     // the pair that holds the current state's outputs
+  bool was_read = false;  // the current state's outputs have been read (wdy_read)
   wdy::RadixWork radix;
   wdy::WarmCtx *warm = nullptr;  // null: no warm path, or not set up yet
   wdy::u32 *warm_words = nullptr;  // [16] its error words and tickets
