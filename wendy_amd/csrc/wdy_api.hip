@@ -562,7 +562,7 @@ static int advance_impl(wdy_sim *s, double h, int nleap, double *acc_last,
   } else if (s->small) {
     int rc = launch_small_advance(s, h, nleap, acc_last, cum_last, xo, vo);
     if (rc) return rc;
-    if (outputs && (u64)s->n <= SMALL_WAVE_MAX) s->staged = s->stage_next;
+    if (outputs && small_wave(s)) s->staged = s->stage_next;
     if (s->ext.kind)  // the kernel's clock, replayed (wendy/wendy.c:401-408)
       for (int ii = 0; ii < nleap; ++ii) s->t0 = s->t0 + h;
   } else if (!acc_last && !cum_last && span_plan(s, h, nleap, &plan)) {
@@ -731,7 +731,7 @@ int wdy_read_and_advance(wdy_sim *sim, double *x_out, double *v_out, double h,
   // outputs by itself, so the copy starts at once (before, a de-sorting launch
   // and an event stood in front of it: 10^4 sheets at 10 steps an output took
   // 60 us against 27, 30000 at one step 63 against 26).
-  bool stages = sim->small ? (u64)sim->n <= SMALL_WAVE_MAX : sim->span != nullptr;
+  bool stages = sim->small ? small_wave(sim) : sim->span != nullptr;
   if (!sim->copy_stream && N > (size_t)1 << 14)
     WDY_HIP(hipStreamCreate(&sim->copy_stream));
   if (stages && !sim->out_v2) {

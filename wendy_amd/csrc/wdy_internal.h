@@ -335,7 +335,16 @@ constexpr u64 SMALL_WAVE_MAX = 512;
 // Largest n the multi-step windows are set up for (beyond, a window of 4096
 // sheets is mostly halo at the step sizes in use).
 constexpr u64 SPAN_MAX = 1u << 22;
-// xo, vo (or null): also the de-sorted outputs, for n <= SMALL_WAVE_MAX
+// Whether a small simulation runs in one wave.  The force of an isothermal slab,
+// a tanh per sheet and step, is what its steps wait for then: equal masses, us per
+// interval of 100 steps and its outputs, one wave / one workgroup: 256 sheets 219 /
+// 275, 300 sheets 410 / 288, 512 sheets 425 / 334.  (Unequal masses, whose prefix
+// the workgroup sums one by one, take longer there in any case.)
+inline bool small_wave(const wdy_sim *s) {
+  return s->n <= (int64_t)SMALL_WAVE_MAX &&
+         !(s->equal_mass && s->ext.kind == WDY_EXT_ISOTHERMAL && s->n > 256);
+}
+// xo, vo (or null): also the de-sorted outputs, if small_wave
 int launch_small_advance(wdy_sim *s, double h, int nleap, double *acc_out,
                          double *cum_out, double *xo = nullptr, double *vo = nullptr);
 int launch_energy(wdy_sim *s, double twopiG, double omega2, double *e_out);

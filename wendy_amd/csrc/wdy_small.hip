@@ -355,7 +355,7 @@ u32 small_max_n(int device) {
 int launch_small_advance(wdy_sim *s, double h, int nleap, double *acc_out,
                          double *cum_out, double *xo, double *vo) {
   const u32 n = (u32)s->n;
-  if (n <= SMALL_WAVE_MAX) {
+  if (small_wave(s)) {
     if (s->timing) timer_begin(s->timer, s->stream, KC_LEAP);
     const int rc =
         s->ext.kind ? launch_wave_per<true>(s, h, nleap, acc_out, cum_out, xo, vo)
