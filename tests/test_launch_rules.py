@@ -50,6 +50,24 @@ int main() {
 }
 '''
 
+RING = r'''
+#include "wdy_rules.h"
+#include <cstdio>
+using namespace wdy;
+int main() {
+  for (uint32_t first : {0u, 1u, 1000u, LAUNCH_RING - 3, LAUNCH_RING - 1}) {
+    uint32_t q = first;
+    for (int k = 0; k < 10; ++k, q = next_launch(q))
+      if (q >= LAUNCH_RING || q + 1 == 0 || launch_of(q, first, 7) != (k < 7 ? k : -1)) {
+        std::printf("launch %u from %u: place %lld\n", q, first,
+                    (long long)launch_of(q, first, 7));
+        return 1;
+      }
+  }
+  return 0;
+}
+'''
+
 SPLITS = r'''
 #include "wdy_rules.h"
 #include <cstdio>
@@ -87,7 +105,7 @@ def run(tmp_path, source):
     assert got.returncode == 0, (got.returncode, got.stdout)
 
 
-@pytest.mark.parametrize('source', [PAIRS, LEAVES, SPLITS],
-                         ids=['pairs', 'leaves', 'splits'])
+@pytest.mark.parametrize('source', [PAIRS, LEAVES, RING, SPLITS],
+                         ids=['pairs', 'leaves', 'ring', 'splits'])
 def test_rules(tmp_path, source):
     run(tmp_path, source)

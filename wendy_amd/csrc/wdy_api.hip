@@ -511,24 +511,30 @@ static int settle(wdy_sim *s) {
     }
   }
   if (s->span) {
-    bool failed = false;
-    double h = 0.0;
-    int nleap = 0;
-    double *xo = nullptr, *vo = nullptr;
-    if (int rc = span_settle(s, &failed, &h, &nleap, &xo, &vo)) return rc;
-    while (failed) {  // again with wider halos, or on the other paths
-      s->redos += 1;
-      SpanPlan p;
-      if (span_plan(s, h, nleap, &p)) {
-        if (int rc = span_interval(s, h, nleap, p, xo, vo)) return rc;
-        WDY_HIP(hipEventRecord(s->ev1, s->stream));
-        if (int rc = span_settle(s, &failed, &h, &nleap, &xo, &vo)) return rc;
-      } else {
-        failed = false;
-        s->staged = -1;
-        if (int rc = cold_interval(s, h, nleap, nullptr, nullptr)) return rc;
-        WDY_HIP(hipEventRecord(s->ev1, s->stream));
-        if (int rc = radix_check_enqueue(s)) return rc;
+    SpanRedo redo[SPAN_QUEUE], now;
+    int count = 0;
+    if (int rc = span_settle(s, redo, &count)) return rc;
+    for (int i = 0; i < count; ++i) {  // again with wider halos, or on the other paths
+      bool failed = i == 0;            // (the others have not run)
+      for (int left = 1; left > 0;) {
+        if (failed) s->redos += 1;
+        const SpanRedo &r = redo[i];
+        SpanPlan p;
+        if (span_plan(s, r.h, r.nleap, &p)) {
+          const bool resorts = !s->span_sorted;
+          if (int rc = span_interval(s, r.h, r.nleap, p, r.xo, r.vo)) return rc;
+          WDY_HIP(hipEventRecord(s->ev1, s->stream));
+          if (resorts)
+            if (int rc = radix_check_enqueue(s)) return rc;
+          if (int rc = span_settle(s, &now, &left)) return rc;
+          failed = true;
+        } else {
+          left = 0;
+          s->staged = -1;
+          if (int rc = cold_interval(s, r.h, r.nleap, nullptr, nullptr)) return rc;
+          WDY_HIP(hipEventRecord(s->ev1, s->stream));
+          if (int rc = radix_check_enqueue(s)) return rc;
+        }
       }
     }
   }
@@ -548,14 +554,20 @@ static int settle(wdy_sim *s) {
 static int advance_impl(wdy_sim *s, double h, int nleap, double *acc_last,
                         double *cum_last, bool outputs = false) {
   WDY_HIP(hipSetDevice(s->device));
-  if (int rc = settle(s)) return rc;
+  SpanPlan plan;
+  // intervals one after the other without outputs in between are enqueued behind
+  // each other in windows, and checked together
+  const bool chained = span_chains(s) && !acc_last && !cum_last && !outputs &&
+                       !s->host_force && !s->rerr_pending && !s->broken &&
+                       span_plan(s, h, nleap, &plan);
+  if (!chained)
+    if (int rc = settle(s)) return rc;
   s->staged = -1;
   s->was_read = false;
   double *const xo = !outputs ? nullptr : s->stage_next ? s->out_x2 : s->out_x;
   double *const vo = !outputs ? nullptr : s->stage_next ? s->out_v2 : s->out_v;
   warm_gang_release(s);  // ev0/ev1 bracket this interval
   WDY_HIP(hipEventRecord(s->ev0, s->stream));
-  SpanPlan plan;
   if (s->host_force) {
     if (int rc = advance_host_force(s, h, nleap, acc_last, cum_last)) return rc;
     if (int rc = radix_check_enqueue(s)) return rc;

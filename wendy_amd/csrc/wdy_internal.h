@@ -396,7 +396,14 @@ int span_prefix(wdy_sim *s);
 // xo, vo: the de-sorted outputs, or null
 int span_interval(wdy_sim *s, double h, int nleap, const SpanPlan &p, double *xo,
                   double *vo);
-int span_settle(wdy_sim *s, bool *failed, double *h, int *nleap, double **xo, double **vo);
+constexpr int SPAN_QUEUE = 32;  // intervals in flight, at most
+struct SpanRedo {
+  double h = 0.0;
+  int nleap = 0;
+  double *xo = nullptr, *vo = nullptr;
+};
+bool span_chains(wdy_sim *s);
+int span_settle(wdy_sim *s, SpanRedo *redo, int *count);
 // the events bracketing the last interval when it ran in a gang
 bool warm_gang_events(wdy_sim *s, hipEvent_t *start, hipEvent_t *done);
 // the next interval runs outside a gang: drop the settled gang record

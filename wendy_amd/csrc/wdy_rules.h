@@ -26,13 +26,23 @@ inline PairPlan pair_plan(uint32_t n, uint32_t ny, uint32_t block) {
   return p;
 }
 
-// Whether a window of launch q of an interval leaves its simulation alone,
-// `word` being the simulation's: 0, or 1 + the launch in which a window could not
-// vouch for its core.  Only an earlier launch's failure counts: every wave of
-// every window of this launch then decides alike, also those that read the word
-// after another window of the launch has set it.  (What this launch writes is
-// not read: the interval is redone from what it was given.)
+// Whether a window of launch q leaves its simulation alone, `word` being the
+// simulation's: 0, or 1 + the launch in which a window could not vouch for its
+// core.  Only an earlier launch's failure counts: every wave of every window of
+// this launch then decides alike, also those that read the word after another
+// window of the launch has set it.  (What this launch writes is not read: the
+// interval is redone from what it was given.)
 constexpr bool span_leaves(uint32_t word, uint32_t q) { return word != 0 && word != q + 1; }
+
+// The launches of a simulation are numbered in a ring, so that 1 + the number is
+// never 0.  launch_of: the place of launch `q` in `count` launches from `first`
+// on, or -1.
+constexpr uint32_t LAUNCH_RING = 0xffffffffu;
+constexpr uint32_t next_launch(uint32_t q) { return q + 1 == LAUNCH_RING ? 0 : q + 1; }
+constexpr int64_t launch_of(uint32_t q, uint32_t first, uint32_t count) {
+  const uint64_t d = ((uint64_t)q + LAUNCH_RING - first) % LAUNCH_RING;
+  return d < count ? (int64_t)d : -1;
+}
 
 // The ways of cutting an interval of nleap steps into launches that a plan tries:
 // fn(K, launches) with K steps a launch, for every number of launches up to 8,

@@ -45,13 +45,12 @@ struct SpanArgs {
                          // reach, with several windows (or null)
   u32 *stat_clr;         // stat words of the next interval, to be reset (or null)
   u32 *stat_host;        // copies of stat in pinned host memory (or null)
-  // set to fail_value = 1 + the launch's number in the interval if a window could
-  // not vouch for its core, or a sheet is no longer finite: what the launch wrote
-  // may then be out of order or lack sheets, and the later launches of the
-  // interval, for which that is the input, leave (span_leaves)
+  // set to fail_value = 1 + the launch's number if a window could not vouch for its
+  // core, or a sheet is no longer finite: what the launch wrote may then be out
+  // of order or lack sheets, and the later launches, for which that is the input,
+  // leave (span_leaves)
   u32 *fail;
   u32 fail_value;
-  u32 *fail_clr;         // the next interval's word, to be cleared (or null)
   u32 *fail_host;        // set too, in pinned host memory (or null)
 };
 

@@ -75,7 +75,6 @@ __device__ __forceinline__ Reach span_reach(const SpanArgs &A, const u32 j) {
     R.slack = fminf(R.slack, (float)(d / R.D));
   }
   if (j == 0 && threadIdx.x < SPAN_SLOTS) {
-    if (A.fail_clr && threadIdx.x == 0) *A.fail_clr = 0;
     if (A.vmax_clr) A.vmax_clr[threadIdx.x] = 0;
     if (A.stat_clr) A.stat_clr[threadIdx.x] = SPAN_STAT_INIT;
   }
@@ -402,7 +401,6 @@ __global__ __launch_bounds__(PER ? 64 : SH::WT) void k_span_many(
   A.stat_host = nullptr;
   A.fail = M.fail + d.eslot;
   A.fail_value = q + 1u;
-  A.fail_clr = nullptr;
   A.fail_host = nullptr;
   if constexpr (PER > 0)
     span_wave<PER, EQ, false>(A, e.y);
@@ -617,14 +615,14 @@ void span_many_plan(std::vector<BatchDesc> &d, const double *info,
 namespace {
 
 // vmax: three sets of words, all zero but the first of set `at`; stat: both
-// sets of stat words, then both intervals' fail words; width (may be null): the words of k_span_widths
+// sets of stat words, then the fail word; width (may be null): the words of k_span_widths
 __global__ void k_span_init(u64 *vmax, u32 *stat, u32 at, u64 v, u64 *width) {
   const u32 t = threadIdx.x;
   if (width && t < 16) width[t] = ~0ull;
   for (u32 q = t; q < 3 * SPAN_SLOTS; q += blockDim.x)
     vmax[q] = q == at * SPAN_SLOTS ? v : 0ull;
   for (u32 q = t; q < 2 * SPAN_SLOTS; q += blockDim.x) stat[q] = SPAN_STAT_INIT;
-  if (t < 2) stat[2 * SPAN_SLOTS + t] = 0;
+  if (t == 0) stat[2 * SPAN_SLOTS] = 0;
 }
 
 // the largest |v|, into the words (zero before) of one set
@@ -738,10 +736,20 @@ __global__ __launch_bounds__(256) void k_span_gather(
 
 }  // namespace
 
+// An interval that has not been checked yet.
+struct SpanPending {
+  SpanRedo again;       // what would have to be redone
+  int start = 0;        // the set it started from
+  double t0 = 0.0;
+  u32 nwin = 0;
+  double ratio = 0.0;   // halo ranks taken over ranks expected
+  u32 first = 0, count = 0;  // its launches
+};
+
 struct SpanCtx {
   u64 *cf[3] = {nullptr, nullptr, nullptr};  // unequal masses: mass below
   u64 *vmax = nullptr;    // [3][SPAN_SLOTS]
-  u32 *stat = nullptr;    // [2][SPAN_SLOTS], then the fail words of two intervals
+  u32 *stat = nullptr;    // [2][SPAN_SLOTS], then the fail word
   u64 *h_buf = nullptr;   // pinned: [16] words of the widths, then
   u32 *h_stat = nullptr;  // [SPAN_SLOTS], then the fail word
   double fscale = 1.0, finv = 1.0;
@@ -749,7 +757,8 @@ struct SpanCtx {
   double vmax_h = 0.0;    // largest |v| at the start
   double xmax_h = 0.0;    // largest |x| at the start
   double reach = 1.0;     // ranks of a launch's reach over those the two give
-  u32 epoch = 0, iv = 0;  // launches and intervals so far
+  u32 epoch = 0, iv = 0;  // launches (word sets) and intervals so far
+  u32 launch = 0;         // the next launch's number
   int fails = 0;          // intervals redone in a row
   bool single = false;    // one window or none
   bool given_up = false;  // not for steps of this size
@@ -759,12 +768,8 @@ struct SpanCtx {
   bool l_single = false, l_ok = false;
   double fall = 0.8;      // how fast `reach` falls again
   bool off = false;       // for good
-  bool pending = false;
-  int p_start = 0, p_nleap = 0;
-  double p_h = 0.0, p_t0 = 0.0;
-  u32 p_nwin = 0;
-  double p_ratio = 0.0;  // halo ranks taken over ranks expected
-  double *p_xo = nullptr, *p_vo = nullptr;
+  SpanPending pend[SPAN_QUEUE];
+  int npend = 0;
 };
 
 // |acceleration| of a sheet at x <= a0 + a1 * |x|
@@ -905,7 +910,7 @@ void span_take(wdy_sim *s, Carve &k) {
   SpanCtx &c = *s->span;
   const size_t N = (size_t)s->n;
   k.take(c.vmax, 3 * SPAN_SLOTS + 16);
-  k.take(c.stat, 2 * SPAN_SLOTS + 2);
+  k.take(c.stat, 2 * SPAN_SLOTS + 1);
   if (!s->equal_mass)
     for (int b = 0; b < 3; ++b) k.take(c.cf[b], N);
 }
@@ -997,10 +1002,16 @@ static int span_resort(wdy_sim *s) {
   return span_vmax(s);
 }
 
+// Whether the next interval may be enqueued before those in flight are checked.
+// Each starts from the current set and writes only the two others, so an interval
+// that failed can go back to its start: the next would write there, but its
+// launches leave if one before them has failed.
+bool span_chains(wdy_sim *s) {
+  return s->span && s->span->npend > 0 && s->span->npend < SPAN_QUEUE;
+}
+
 // Enqueues one output interval, which span_settle checks once the caller has
-// recorded ev1 behind it.  It starts from the
-// current set and writes only the two others, so a failure found later can
-// go back to its start.
+// recorded ev1 behind it.
 int span_interval(wdy_sim *s, double h, int nleap, const SpanPlan &p, double *xo,
                   double *vo) {
   SpanCtx &c = *s->span;
@@ -1019,16 +1030,21 @@ int span_interval(wdy_sim *s, double h, int nleap, const SpanPlan &p, double *xo
   a.finv = c.finv;
   a.ext = s->ext;
   span_amax(s, &a.amax0, &a.amax1);
-  // (the interval before has been settled: nothing writes there now)
-  for (u32 q = 0; q < SPAN_SLOTS; ++q) c.h_stat[q] = SPAN_STAT_INIT;
-  c.h_stat[SPAN_SLOTS] = 0;
+  if (c.npend == 0) {  // (nothing writes there now)
+    for (u32 q = 0; q < SPAN_SLOTS; ++q) c.h_stat[q] = SPAN_STAT_INIT;
+    c.h_stat[SPAN_SLOTS] = 0;
+  }
+  SpanPending pend;
+  pend.again = {h, nleap, xo, vo};
+  pend.start = start;
+  pend.t0 = s->t0;
+  pend.first = c.launch;
   a.stat_host = c.h_stat;
   a.fail_host = c.h_stat + SPAN_SLOTS;
   const u32 set = c.iv++ & 1u;
   a.stat = c.stat + SPAN_SLOTS * set;
   a.stat_clr = c.stat + SPAN_SLOTS * (set ^ 1u);
-  a.fail = c.stat + 2 * SPAN_SLOTS + set;
-  a.fail_clr = c.stat + 2 * SPAN_SLOTS + (set ^ 1u);
+  a.fail = c.stat + 2 * SPAN_SLOTS;
   double t = s->t0;
   int in = start, q = 0;
   for (int done = 0; done < nleap; ++q) {
@@ -1039,14 +1055,16 @@ int span_interval(wdy_sim *s, double h, int nleap, const SpanPlan &p, double *xo
     if (!span_geom(s, p.shape, p.reach, span_drift(ah, done, K, nleap), ah * K, &g))
       return fail(WDY_ERUNTIME, "span_interval: no windows for shape %d", p.shape);
     if (done == 0) {
-      c.p_nwin = g.nwin;
-      c.p_ratio = g.H / std::max(g.est, 1e-300);
+      pend.nwin = g.nwin;
+      pend.ratio = g.H / std::max(g.est, 1e-300);
     }
     a.T = g.T;
     a.H = g.H;
     a.nwin = g.nwin;
     a.K = (u32)K;
-    a.fail_value = (u32)q + 1u;
+    a.fail_value = c.launch + 1u;
+    c.launch = next_launch(c.launch);
+    ++pend.count;
     a.kin = s->key[in];
     a.vin = s->vel[in];
     a.iin = s->idx[in];
@@ -1074,55 +1092,57 @@ int span_interval(wdy_sim *s, double h, int nleap, const SpanPlan &p, double *xo
     done += K;
     in = out;
   }
-  c.pending = true;
-  c.p_start = start;
-  c.p_h = h;
-  c.p_nleap = nleap;
-  c.p_t0 = s->t0;
-  c.p_xo = xo;
-  c.p_vo = vo;
+  c.pend[c.npend++] = pend;
   s->cur = in;
   if (s->ext.kind) s->t0 = t;
   return WDY_OK;
 }
 
-// Waits for and checks the interval in flight; *failed: the state is back at
-// its start and (h, nleap) must be redone, with the halo estimate widened.
-int span_settle(wdy_sim *s, bool *failed, double *h, int *nleap, double **xo,
-                double **vo) {
-  *failed = false;
+// Waits for and checks the intervals in flight.  redo[0 .. *count): the first that
+// failed and those after it, which did not run; the state is back at its start,
+// with the halo estimate widened, and the caller must redo them.
+int span_settle(wdy_sim *s, SpanRedo *redo, int *count) {
+  *count = 0;
   SpanCtx *cp = s->span;
-  if (!cp || !cp->pending) return WDY_OK;
+  if (!cp || cp->npend == 0) return WDY_OK;
   SpanCtx &c = *cp;
   WDY_HIP(hipEventSynchronize(s->ev1));
-  c.pending = false;
-  u32 st = SPAN_STAT_INIT;
-  for (u32 q = 0; q < SPAN_SLOTS; ++q) st = std::min(st, c.h_stat[q]);
-  if (c.h_stat[SPAN_SLOTS] == 0) {
+  const int n = c.npend;
+  c.npend = 0;
+  const u32 word = c.h_stat[SPAN_SLOTS];
+  int bad = n;
+  for (int i = 0; word && i < n && bad == n; ++i)
+    if (launch_of(word - 1u, c.pend[i].first, c.pend[i].count) >= 0) bad = i;
+  if (word && bad == n)
+    return fail(WDY_ERUNTIME, "a window of launch %u failed, which is not in flight", word - 1u);
+  for (int i = 0; i < bad; ++i)
+    if (!s->small_class) s->warm_steps += c.pend[i].again.nleap;
+  if (bad == n) {
     c.fails = 0;
-    if (!s->small_class) s->warm_steps += c.p_nleap;
-    if (c.p_nwin > 1 && st < SPAN_STAT_INIT) {
+    u32 st = SPAN_STAT_INIT;
+    for (u32 q = 0; q < SPAN_SLOTS; ++q) st = std::min(st, c.h_stat[q]);
+    double ratio = 0.0;
+    for (int i = 0; i < n; ++i)
+      if (c.pend[i].nwin > 1) ratio = std::max(ratio, c.pend[i].ratio);
+    if (ratio > 0.0 && st < SPAN_STAT_INIT) {
       float slack;
       __builtin_memcpy(&slack, &st, 4);
       // ranks the reach took over those expected.  It falls slowly, and not
       // below what the widths say: the cores' boundaries are a few of the
       // places where the next plan may put its own.
-      c.reach = std::max(std::max(c.p_ratio / slack, c.fall * c.reach), 1.0);
+      c.reach = std::max(std::max(ratio / slack, c.fall * c.reach), 1.0);
     }
     return WDY_OK;
   }
-  *failed = true;
-  *h = c.p_h;
-  *nleap = c.p_nleap;
-  *xo = c.p_xo;
-  *vo = c.p_vo;
-  s->cur = c.p_start;
-  s->t0 = c.p_t0;
+  const SpanPending &p = c.pend[bad];
+  for (int i = bad; i < n; ++i) redo[(*count)++] = c.pend[i].again;
+  s->cur = p.start;
+  s->t0 = p.t0;
   s->fail_overflow += 1;
   c.reach = std::min(2.0 * c.reach, 1e6);
   c.fall = 0.97;
   ++c.fails;
-  if (c.p_nwin == 1) c.off = true;  // not finite
+  if (p.nwin == 1) c.off = true;  // not finite
   else if (s->small_class) c.single = c.fails >= 2;
   else c.given_up = c.fails >= 3;
   return span_vmax(s);
