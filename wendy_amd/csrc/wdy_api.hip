@@ -647,10 +647,11 @@ int wdy_advance(wdy_sim *sim, double h, int nleap) {
   if (int rc = check_sim(sim, "wdy_advance")) return rc;
   if (nleap < 1) return fail(WDY_EINVAL, "wdy_advance: nleap=%d < 1", nleap);
   if (!std::isfinite(h)) return fail(WDY_EINVAL, "wdy_advance: h not finite");
-  // A program that reads after each interval (wdy_read) has the windows' last
-  // launch write the outputs: a launch less at the read.  (No copy is under way:
-  // the first pair.)
-  const bool outputs = sim->span && sim->was_read;
+  // A program that reads after each interval (wdy_read) has its last launch write
+  // the outputs, on the paths that can: a launch less at the read.  (No copy is
+  // under way: the first pair.)
+  const bool outputs =
+      sim->was_read && (sim->small ? small_wave(sim) : sim->span != nullptr);
   sim->stage_next = 0;
   return advance_impl(sim, h, nleap, nullptr, nullptr, outputs);
 }
