@@ -250,3 +250,29 @@ for n in list(range(1, 20)) + [1000]:
             wendy_amd.Sim(good[0], good[1], m, total, -1., equal_mass=False).close()
             assert (count(launched(), 'k_span_widths') == 1) == (windows and n > 512), n
 ''')
+
+
+def test_every_set_holds_indices(fake):
+    """Those of a simulation with windows and of a batch, before any launch reads
+    them."""
+    run(fake, r'''
+@ctypes.CFUNCTYPE(None, ctypes.c_char_p, ctypes.POINTER(ctypes.c_void_p))
+def look(name, args):
+    at = [int(ctypes.cast(args[k], ctypes.POINTER(ctypes.c_uint64))[0]) for k in sets.get(name, ())]
+    seen.extend(at)
+
+
+seen = []
+sets = {}
+sim(1000).close()
+assert count(launched(), 'k_iota') == 2  # the staged set, and the one not sorted into
+sim(1000, path='large').close()
+assert count(launched(), 'k_iota') == 1
+x = numpy.linspace(-1., 1., 700)
+wendy_amd.Batch([x], [x], [x * 0. + 1.]).close()
+init = [q for q in launched() if 'k_batch_init' in q][0].encode()
+sets[init] = (3, 4)               # (n, x, key, idx, idx2)
+fake.fake_hook(look)
+wendy_amd.Batch([x], [x], [x * 0. + 1.]).close()
+assert len(seen) == 2 and len(set(seen)) == 2 and 0 not in seen
+''')

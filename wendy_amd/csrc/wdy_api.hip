@@ -339,6 +339,12 @@ static int create_impl(int64_t n, const double *x_slot, const i32 *id_slot,
     }
     r = launch_build_state(s, s->out_x, s->idx[1], s->out_v, s->cum);
     if (r) return r;
+    if (span) {
+      // the set that nothing has written yet: whatever a launch may leave out of
+      // it (after a sort that gave up), what is read there is a sheet's index
+      k_iota<<<(unsigned)((N + 255) / 256), 256, 0, s->stream>>>((u32)n, s->idx[2]);
+      WDY_CHECK_LAUNCH();
+    }
     // warm-start step for the large path, unless disabled; it needs
     // non-negative masses (fixed-point prefix).  With windows it is set up
     // when it is first needed.

@@ -546,12 +546,14 @@ int batch_launch(hipStream_t st, const BatchDesc *d_descs, int count,
 namespace wdy {
 namespace {
 
+// (idx2: the set that is written first, so that it never holds anything else)
 __global__ void k_batch_init(u64 n, const double *__restrict__ x,
-                             u64 *__restrict__ key, i32 *__restrict__ idx) {
+                             u64 *__restrict__ key, i32 *__restrict__ idx,
+                             i32 *__restrict__ idx2) {
   const u64 i = (u64)blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
   key[i] = encode_pos(x[i]);
-  idx[i] = (i32)i;
+  idx[i] = idx2[i] = (i32)i;
 }
 
 // One workgroup per descriptor: de-sort its current set into x_out, v_out
@@ -788,7 +790,7 @@ int wdy_batch_create(int64_t nsims, const int64_t *offsets, const double *x,
       WDY_HIP(hipMemcpyAsync(b->arr.mass[0], m, N * 8, hipMemcpyHostToDevice,
                              b->stream));
     k_batch_init<<<(unsigned)((N + 255) / 256), 256, 0, b->stream>>>(
-        (u64)N, b->out_x, b->arr.key[0], b->arr.idx[0]);
+        (u64)N, b->out_x, b->arr.key[0], b->arr.idx[0], b->arr.idx[1]);
     WDY_CHECK_LAUNCH();
     WDY_HIP(hipStreamSynchronize(b->stream));
     return WDY_OK;
