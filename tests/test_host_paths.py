@@ -276,3 +276,16 @@ fake.fake_hook(look)
 wendy_amd.Batch([x], [x], [x * 0. + 1.]).close()
 assert len(seen) == 2 and len(set(seen)) == 2 and 0 not in seen
 ''')
+
+
+@pytest.mark.parametrize('n', [1 << 20, (1 << 20) + 1])
+def test_warm_path_of_large_simulations(fake, n):
+    """Set up with the simulation above 2^20 sheets, whatever windows it has."""
+    run(fake, r'''
+s = sim(%d, 'equal')      # no room for windows here
+launched()
+fake.fake_deny(1)
+s.advance(1e-9, 3)
+assert (count(launched(), 'k_warm_step') > 0) == (s.n > 1 << 20)
+s.close()
+''' % n)

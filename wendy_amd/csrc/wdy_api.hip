@@ -347,13 +347,19 @@ static int create_impl(int64_t n, const double *x_slot, const i32 *id_slot,
     }
     // warm-start step for the large path, unless disabled; it needs
     // non-negative masses (fixed-point prefix).  With windows it is set up
-    // when it is first needed.
+    // when it is first needed; at once for large simulations, which need it at
+    // more step sizes and whose steps are faster with arrays made by then (2^22
+    // sheets, 20 steps: 1.89 ms, 1.93 with arrays made later).
     s->warm_ok = !s->small_class && !(flags & WDY_NO_WARM) && nonneg;
     s->warm_shape0 = (flags & WDY_SHARED_GPU) ? WARM_SHAPE_DEFAULT
                                               : warm_initial_shape(n, eq);
     if (s->warm_ok) s->disp_rate = displacement_rate(n, x_slot, v_id, id_slot);
     if (span) {
       if ((r = span_create(s, scan.x, scan.v))) return r;
+      if (n > (int64_t)1 << 20) {
+        r = warm_ensure(s);
+        if (r && r != WDY_ENOMEM) return r;
+      }
     } else if ((r = warm_ensure(s))) {
       return r;
     }
