@@ -87,12 +87,14 @@ int wdy_create(int64_t n, const double *x, const double *v, const double *m,
  * drift), last drift halved -- the body of _wendy_nbody_approx_onestep
  * (wendy/wendy.c:394-411) with h = dt/nleap.  Asynchronous: it returns
  * once the interval is enqueued.  The device's verdict on a warm-start
- * interval (a bucket that outgrew its capacity, too many far movers) is
+ * interval (a bucket that outgrew its capacity, too many far movers) or on
+ * windows (a halo too narrow) is
  * checked by the next call on the handle that reads or extends the state
  * (wdy_advance, wdy_read, wdy_read_and_advance, wdy_energy, wdy_tune, the
- * ext-force setters and the statistics), which then redoes the interval from
- * its untouched start on the radix path before doing its own work; so a
- * result never depends on whether a redo happened. */
+ * ext-force setters and the statistics; up to 32 wdy_advance calls in windows
+ * are enqueued first), which then redoes the interval from
+ * its untouched start, on the radix path or with wider halos, before doing its
+ * own work; so a result never depends on whether a redo happened. */
 int wdy_advance(wdy_sim *sim, double h, int nleap);
 
 /* De-sort the state into original sheet order and copy it to the host:
@@ -299,8 +301,8 @@ int wdy_potential_arrays(int64_t ny, const double *y, int64_t n,
                          double omega2, double *out);
 
 /* ---- batched ensemble ------------------------------------------------------
- * Many independent simulations (uneven n) advanced together: one kernel
- * launch per output interval for all of them.  No reference counterpart
+ * Many independent simulations (uneven n) advanced together: a few kernel
+ * launches per output interval for all of them.  No reference counterpart
  * (the reference runs one simulation per generator); each simulation's
  * arithmetic is that of wdy_create/wdy_advance.
  *   offsets   nsims + 1 increasing values, offsets[0] = 0: simulation k owns

@@ -2,8 +2,10 @@
 
 No reference counterpart (the reference runs one simulation per ``nbody``
 generator); each simulation's arithmetic is that of ``wendy_amd.nbody`` with
-``approx=True``.  One kernel launch advances every simulation by one output
-interval (see wdy_batch_create in include/wendy_amd.h).
+``approx=True``.  The first output interval of any steps is one kernel launch
+for all of them, one workgroup per simulation; while the steps stay the same the
+following ones are a few launches of windows over all simulations (see
+wdy_batch_create in include/wendy_amd.h).
 """
 import ctypes
 import sys

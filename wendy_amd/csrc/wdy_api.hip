@@ -711,9 +711,11 @@ int wdy_read(wdy_sim *sim, double *x_out, double *v_out, double *seconds_out) {
 // Both output arrays to pinned host memory in one launch, where the copy is what
 // an output waits for: 2^14 sheets or fewer, and up to 2^16 with one or two
 // steps an output.  Beside a longer interval the two copy calls disturb it less
-// and are hidden behind it.  us per output of the generator, two copies / this
-// kernel: 10^4 sheets at 2 steps 31 / 24, at 10 steps 33 / 34; 30000 at 1 step
-// 36 / 32, at 20 steps 55 / 59; 65536 at 2 steps 47 / 44, at 20 steps 69 / 83.
+// and are hidden behind it.  us per output, two copies / this kernel, of one
+// generator alone (and of three in turn): 3000 sheets at 20 steps 60 / 47 (30 /
+// 19), 10^4 at 1 step 43 / 31 (31 / 21), at 20 steps 76 / 63 (31 / 22); 30000 at 1
+// step 36 / 33 (38 / 26), at 20 steps 68 / 74 (41 / 39); 65536 at 2 steps 47 / 47
+// (49 / 37), at 20 steps 90 / 105 (56 / 59).
 __global__ __launch_bounds__(256) void k_copy_out(u32 n, const double *__restrict__ xs,
                                                   const double *__restrict__ vs,
                                                   double *__restrict__ xd,
@@ -754,8 +756,8 @@ int wdy_read_and_advance(wdy_sim *sim, double *x_out, double *v_out, double h,
   const size_t N = (size_t)sim->n;
   // From the second interval on, the last launch of an interval has written the
   // outputs by itself, so the copy starts at once (before, a de-sorting launch
-  // and an event stood in front of it: 10^4 sheets at 10 steps an output took
-  // 60 us against 27, 30000 at one step 63 against 26).
+  // and an event stood in front of it: three generators in turn, 10^4 sheets at 10
+  // steps an output took 60 us against 27, 30000 at one step 63 against 26).
   bool stages = sim->small ? small_wave(sim) : sim->span != nullptr;
   if (!sim->copy_stream && N > (size_t)1 << 14)
     WDY_HIP(hipStreamCreate(&sim->copy_stream));

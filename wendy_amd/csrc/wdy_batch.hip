@@ -7,9 +7,9 @@
 // the longest workgroups start first).  Its time is that of the largest
 // simulation: 3.4 ms for 10 steps of 65536 sheets.
 //
-// From the second interval of the same steps on a batch runs in windows (wdy_span.h), one
-// workgroup or wave per (simulation, window) and several steps per launch,
-// planned on the host from the densities and speeds that k_batch_form reports.
+// From the second interval of the same steps on a batch runs in windows
+// (wdy_span.h), one workgroup or wave per (simulation, window) and several steps
+// per launch, planned on the host from the densities and speeds that k_batch_form reports.
 // Nothing waits for the host within a plan: a window that cannot vouch for its
 // core marks its simulation, whose later launches then leave it alone, and
 // k_batch_advance, which ends every interval, redoes the rest of the interval

@@ -332,8 +332,9 @@ constexpr u64 SMALL_MAX_UNEQUAL = 1536;
 // ones (whose prefix stays a sequential sum), at 1000 sheets the windows' single
 // workgroup 21 and 25.
 constexpr u64 SMALL_WAVE_MAX = 512;
-// Largest n the multi-step windows are set up for (beyond, a window of 4096
-// sheets is mostly halo at the step sizes in use).
+// Largest n the multi-step windows are set up for (beyond, the largest windows,
+// 7168 sheets of equal and 5120 of unequal masses, are mostly halo at the step
+// sizes in use; at 2^22 they win up to h = 1e-4: 1.17 ms per 20 steps against 1.89).
 constexpr u64 SPAN_MAX = 1u << 22;
 // Whether a small simulation runs in one wave.  The force of an isothermal slab,
 // a tanh per sheet and step, is what its steps wait for then: equal masses, us per

@@ -5,16 +5,16 @@
 // window runs K steps on its sheets by itself: the force on a sheet is its
 // rank, or the mass below it, and the ranks outside a window do not change
 // until a sheet has crossed its halo.  Windows prove on the device that none
-// could have (Reach below); the host sees the verdict when it settles the
-// interval and otherwise redoes it, from the set the interval started from,
-// with wider halos.
+// could have (Reach below); a window that cannot marks the simulation, whose
+// later launches leave, and the host, which sees the verdict when it settles,
+// redoes the interval from the set it started from, with wider halos.
 //
 // What bounds the one-step kernel at these sizes is not the GPU's rates but a
 // launch per step, ~12 us of dependent phases each.  Measured, us per interval
-// of 20 steps on the sech^2 disk, before (one launch per step) -> with windows,
-// equal / unequal masses: 2^14 239 -> 30 / 266 -> 40, 2^16 265 -> 51 / 306 ->
-// 66, 2^18 412 -> 100 / 479 -> 132, 2^20 851 -> 283 / 950 -> 500.  What bounds
-// a window is the latency of its step, ~1 us of LDS round trips and barriers
+// of 20 steps of h = 2.5e-4 on the sech^2 disk, one launch per step -> windows,
+// equal / unequal masses: 2^14 244 -> 30 / 270 -> 41, 2^16 267 -> 51 / 306 ->
+// 66, 2^18 415 -> 98 / 485 -> 131, 2^20 870 -> 312 / 954 -> 477, 2^21 1178 -> 807
+// / 1649 -> 1316.  What bounds a window is the latency of its step, ~1 us of LDS round trips and barriers
 // (0.2-0.5 us for one wave), and from ~256 windows on the CUs' issue rate.
 #include <algorithm>
 #include <cmath>
