@@ -264,7 +264,7 @@ static int create_impl(int64_t n, const double *x_slot, const i32 *id_slot,
     // windows take their unit of mass and their bound of the field from totmass,
     // which a caller may have set to something else than the masses' sum; the
     // one-workgroup path does not care.)
-    const bool span = nonneg && std::fabs(scan.msum - totmass) <= 1e-6 * scan.msum &&
+    const bool span = nonneg && std::fabs(scan.msum - totmass) <= 1e-3 * scan.msum &&
                       (u64)n > SMALL_WAVE_MAX && (u64)n <= SPAN_MAX &&
                       !(flags & (WDY_FORCE_SMALL | WDY_FORCE_LARGE | WDY_NO_WARM |
                                  WDY_SHARED_GPU));
