@@ -78,4 +78,6 @@ def test_steps_of_another_size_try_again(gpu_lib):
         warm, cold, redo = both(1e-4, 400)
     assert cold > 0 and redo >= 3
     assert both(5e-5, 20) == (warm + 20, cold, redo)
+    # (not the ones they were given up for: a radix interval again)
+    assert both(1e-4, 400)[1:] == (cold + 400, redo)
     sim.close()

@@ -761,7 +761,8 @@ struct SpanCtx {
   u32 launch = 0;         // the next launch's number
   int fails = 0;          // intervals redone in a row
   bool single = false;    // one window or none
-  bool given_up = false;  // not for steps of this size
+  // given up for steps of this size or longer, in intervals of this time or longer
+  double up_h = 1e308, up_t = 1e308;
   SpanPlan last;          // the last search's result, for
   double l_h = 0.0, l_a0 = 0.0, l_a1 = 0.0;  // these
   int l_nleap = 0;
@@ -829,13 +830,11 @@ static bool span_search(const wdy_sim *s, double h, int nleap, SpanPlan *plan);
 bool span_plan(wdy_sim *s, double h, int nleap, SpanPlan *plan) {
   if (!s->span || s->span->off || !(h != 0.0) || !std::isfinite(h)) return false;
   SpanCtx &c = *s->span;
-  // Steps of another size try again what was given up for these, and give it up
-  // at the first failure.
-  if (h != c.l_h || nleap != c.l_nleap) {
-    if (c.given_up || c.single) c.fails = s->small_class ? 1 : 2;
-    c.given_up = c.single = false;
-  }
-  if (c.given_up) return false;
+  // (shorter steps or intervals try again what was given up for these)
+  const bool given_up =
+      std::fabs(h) >= c.up_h && std::fabs(h) * (double)nleap >= c.up_t;
+  if (given_up && !s->small_class) return false;
+  c.single = given_up;
   // The search takes 5-15 us of host time: its result is kept for the intervals
   // that follow, while the halos they call for are those of the plan.
   double a0, a1;  // (an external force may have come or gone)
@@ -1143,8 +1142,10 @@ int span_settle(wdy_sim *s, SpanRedo *redo, int *count) {
   c.fall = 0.97;
   ++c.fails;
   if (p.nwin == 1) c.off = true;  // not finite
-  else if (s->small_class) c.single = c.fails >= 2;
-  else c.given_up = c.fails >= 3;
+  else if (c.fails >= (s->small_class ? 2 : 3)) {
+    c.up_h = std::min(c.up_h, std::fabs(p.again.h));
+    c.up_t = std::min(c.up_t, std::fabs(p.again.h) * (double)p.again.nleap);
+  }
   return span_vmax(s);
 }
 
