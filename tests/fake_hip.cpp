@@ -170,12 +170,22 @@ int hipStreamCreateWithFlags(void **s, unsigned) { return token(s); }
 int hipStreamDestroy(void *) { return 0; }
 int hipStreamSynchronize(void *) { return 0; }
 int hipStreamWaitEvent(void *, void *, unsigned) { return 0; }
-int hipEventCreate(void **e) { return token(e); }
-int hipEventCreateWithFlags(void **e, unsigned) { return token(e); }
-int hipEventDestroy(void *) { return 0; }
-int hipEventRecord(void *, void *) { return 0; }
+int hipEventCreate(void **e) {
+  *e = calloc(1, sizeof(int));  // whether it has been recorded
+  return 0;
+}
+int hipEventCreateWithFlags(void **e, unsigned) { return hipEventCreate(e); }
+int hipEventDestroy(void *e) {
+  free(e);
+  return 0;
+}
+int hipEventRecord(void *e, void *) {
+  *(int *)e = 1;
+  return 0;
+}
 int hipEventSynchronize(void *) { return 0; }
-int hipEventElapsedTime(float *ms, void *, void *) {
+int hipEventElapsedTime(float *ms, void *a, void *) {
+  if (!*(int *)a) return fail(INVALID);  // never recorded
   *ms = 1.f;
   return 0;
 }

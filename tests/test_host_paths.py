@@ -289,3 +289,27 @@ s.advance(1e-9, 3)
 assert (count(launched(), 'k_warm_step') > 0) == (s.n > 1 << 20)
 s.close()
 ''' % n)
+
+
+@pytest.mark.parametrize('n', [3, 1000, 20000])
+def test_read_before_the_first_interval(fake, n):
+    """There is no time of an interval to ask for yet, and no error of that left
+    for the next call."""
+    run(fake, r'''
+fake.fake_spacing(1e-4)
+s = sim(%d)
+x, v = numpy.empty(s.n), numpy.empty(s.n)
+assert s.read(x, v) == 0.
+s.advance(1e-6, 2)
+assert s.read(x, v) > 0.
+s.close()
+s = sim(%d)
+assert s.read_and_advance(x, v, 1e-6, 2) == 0.
+assert s.read(x, v) > 0.
+s.close()
+b = wendy_amd.Batch([x], [x], [numpy.full(s.n, 1.)])
+assert b.read()[2] == 0.
+b.advance(1e-6, 2)
+assert b.read()[2] > 0.
+b.close()
+''' % (n, n))

@@ -615,7 +615,10 @@ static float interval_ms(wdy_sim *s) {
   hipEvent_t a = s->ev0, b = s->ev1;
   (void)warm_gang_events(s, &a, &b);
   float ms = 0.f;
-  if (hipEventElapsedTime(&ms, a, b) != hipSuccess) ms = 0.f;
+  if (hipEventElapsedTime(&ms, a, b) != hipSuccess) {  // no interval has run yet
+    (void)hipGetLastError();  // else the next launch's check finds it
+    ms = 0.f;
+  }
   return ms;
 }
 

@@ -863,7 +863,10 @@ int wdy_batch_read(wdy_batch *b, double *x_out, double *v_out,
                 "its bound");
   if (seconds_out) {
     float ms = 0.f;
-    if (hipEventElapsedTime(&ms, b->ev0, b->ev1) != hipSuccess) ms = 0.f;
+    if (hipEventElapsedTime(&ms, b->ev0, b->ev1) != hipSuccess) {  // none has run yet
+      (void)hipGetLastError();  // else the next launch's check finds it
+      ms = 0.f;
+    }
     *seconds_out = ms * 1e-3;
   }
   return WDY_OK;
