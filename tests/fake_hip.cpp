@@ -5,11 +5,13 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <new>
 #include <string>
 
 namespace {
 constexpr int OOM = 2, INVALID = 1;
 size_t g_deny = SIZE_MAX;  // allocations of this many bytes or more fail
+size_t g_deny_new = SIZE_MAX;  // those of the C++ code itself
 int g_last = 0;
 std::string g_log;
 std::map<const void *, std::string> g_names;
@@ -38,9 +40,18 @@ int alloc(void **p, size_t n) {
 }
 }  // namespace
 
+void *operator new(size_t n) {
+  void *p = n >= g_deny_new ? nullptr : malloc(n);
+  if (!p) throw std::bad_alloc();
+  return p;
+}
+void operator delete(void *p) noexcept { free(p); }
+void operator delete(void *p, size_t) noexcept { free(p); }
+
 extern "C" {
 
 void fake_deny(size_t bytes) { g_deny = bytes; }
+void fake_deny_new(size_t bytes) { g_deny_new = bytes; }
 // the kernels launched so far, one a line
 const char *fake_log() { return g_log.c_str(); }
 void fake_clear() { g_log.clear(); }

@@ -16,6 +16,7 @@ import ctypes, sys
 fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
 fake.fake_log.restype = ctypes.c_char_p
 fake.fake_deny.argtypes = [ctypes.c_size_t]
+fake.fake_deny_new.argtypes = [ctypes.c_size_t]
 fake.fake_spacing.argtypes = [ctypes.c_double]
 fake.fake_register.argtypes = [ctypes.c_void_p, ctypes.c_size_t]
 NONE = ctypes.c_size_t(-1).value
@@ -313,3 +314,23 @@ b.advance(1e-6, 2)
 assert b.read()[2] > 0.
 b.close()
 ''' % (n, n))
+
+
+def test_batch_without_host_memory_for_windows(fake):
+    """Their list: no exception leaves the library, the interval runs without them."""
+    run(fake, r'''
+x = [numpy.random.default_rng(k).standard_normal(700) for k in range(1100)]
+b = wendy_amd.Batch(x, x, [numpy.full(700, 1. / 700.)] * 1100)
+b.advance(1e-3, 10)
+launched()
+fake.fake_deny_new(4096)
+for _ in range(2):
+    b.advance(1e-3, 10)
+fake.fake_deny_new(NONE)
+k = launched()
+assert count(k, 'k_batch_advance') == 2 and count(k, 'k_span_many') == 0, k
+for _ in range(2):
+    b.advance(2e-3, 10)
+assert count(launched(), 'k_span_many') > 0
+b.close()
+''')

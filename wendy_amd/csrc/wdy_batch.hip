@@ -707,7 +707,12 @@ static int batch_plan(wdy_batch *b, double h, int nleap, bool windows) {
   if (int rc = batch_upload(b)) return rc;
   b->planned = windows;
   if (!windows) return WDY_OK;
-  const int rc = batch_windows(b);
+  int rc;
+  try {
+    rc = batch_windows(b);
+  } catch (const std::bad_alloc &) {  // the list of them, on the host
+    rc = WDY_ENOMEM;
+  }
   if (!rc) return WDY_OK;
   (void)hipGetLastError();  // else the next launch's check finds it
   for (BatchDesc &q : d) q.L = q.nwin = 0;  // from where it is
