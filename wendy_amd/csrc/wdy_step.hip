@@ -340,7 +340,7 @@ __device__ __forceinline__ double pair_end(const PairEnd &e, const double *y,
 // are read once for all of its QP points, whose sums it keeps in registers, so
 // the sheets' traffic from L2 (16 B for QP pairs of two f64 instructions) falls
 // behind the arithmetic.  With one point per block the loads were what bound it:
-// 30000 x 30000 pairs 808 us, with QP = 16 88 us (the two instructions alone take
+// 30000 x 30000 pairs 808 us, with QP = 16 86 us (the two instructions alone take
 // 46; without the bound of eight waves per SIMD, which only reorders them, 105).
 // A thread adds up a stretch's n / splits / 256 terms, the rest is a tree, in a
 // fixed order.
